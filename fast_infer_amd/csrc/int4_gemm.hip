@@ -8,28 +8,18 @@
 // :309-326): one rounding of an exact product, which is what v_pk_mul_f16 computes.
 //
 // C[m, n] = fp16( sum_k X[m, k] * W[n, k] ), fp32 accumulation (matmul.py:14-132,
-// :135-186), by the rows M of X:
-//   M <= 16          gemv_kernel: one workgroup per 16 output columns, K split over its waves;
-//   17..64, packed   gemm_sk_kernel: loader and multiplier waves, K split over workgroups
-//                    whose partial sums are added inside the launch (sk_reduce_kernel when
-//                    the stream has no counters);
-//   17..128          gemm_kernel (packed weights from 65 rows), below;
-//   >= 129           the weight dequantized once into the workspace, then
-//                    wide_gemm_kernel, an fp16 GEMM.
-//
-// gemm_kernel: one workgroup = 4 waves = 64 output columns (16 per wave) x MT rows, over a
-// slice of the K groups.  Per 128-wide group, X[MT, 128] is staged in LDS (double
-// buffered, rows padded to 272 bytes so the 16 rows a wave reads are on distinct banks);
-// each lane loads 16 bytes of its weight row (32 int4 values), dequantizes them in
-// registers and feeds v_mfma_f32_16x16x32_f16 with W as the A operand and X^T as the B
-// operand.  In k-step s (0..3) of a group, lane group g = lane/16 supplies k = 32g + 8s
-// .. +7: the 16 bytes one lane loads are exactly its four k-steps.  Small grids split the
-// K groups over blockIdx.z; a second kernel adds the fp32 partials in a fixed order.
-#include <stdlib.h>
-
+// :135-186).  By the rows M of X and the measured costs in plan():
+//   up to 4 rows, and up to 16 where it is the fastest:
+//                     gemv_kernel: one workgroup per 16 output columns, K split over its waves;
+//   packed weights:   mid_gemm_kernel, which unpacks them in registers, and for many row tiles
+//                     one unpacking into the workspace followed by tile_gemm_kernel;
+//   fp16 weights:     tile_gemm_kernel.
+// The last two split K over workgroups where the tiles alone leave CUs idle, and add the splits
+// inside the launch (add_splits).  gemm_kernel serves rows of X too far apart for their 32-bit
+// offsets: one workgroup = 4 waves = 64 output columns (16 per wave) x MT rows, X[MT, 128] per
+// group staged through registers in LDS (double buffered, rows padded to 272 bytes so the 16
+// rows a wave reads are on distinct banks), K split over blockIdx.z.
 #include <algorithm>
-#include <atomic>
-#include <mutex>
 #include <type_traits>
 
 #include "common.h"
@@ -58,10 +48,16 @@ struct Params {
   int groups_per_split;
   const half_t* norm_w;  // RMSNorm weight [K] when the norm is fused into the X operand
   float eps;
-  // gemm_sk_kernel: column tiles, K splits and the per-tile arrival counters
+  // mid_gemm_kernel and tile_gemm_kernel: row tiles, all tiles, K splits, the per-tile arrival
+  // counters (one line set per XCD group, counter_stride apart); row tiles per XCD when they
+  // are banded (tile_gemm_kernel), else 0; 16-byte output stores
+  int tiles_m;
   int tiles;
   int ksplit;
   unsigned* counters;
+  int counter_stride;
+  int band;
+  int vec_out;
 };
 
 __device__ __forceinline__ uint32_t as_u32(half2_t h) { return __builtin_bit_cast(uint32_t, h); }
@@ -333,56 +329,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(Params p) {
   store_tile<kMSub>(p, acc, m0, blockIdx.x * kNTile);
 }
 
-// ---------------------------------------------------------------------------------------
-// Packed-weight GEMM for 17..64 rows with the K split added up in the same launch.
-//
-// A workgroup of eight multiplying waves and four loading waves computes a 64-column x MT-row
-// tile over a slice of G <= 8 K groups.  Multiplying wave w = 4h + q takes output columns
-// 32h .. 32h + 31 (column half h) and the q-th quarter of each phase's k-steps (32 k each),
-// so the two waves of a SIMD (w and w + 4) read the same X fragments for different weights,
-// and each weight is unpacked once.  Within a wave the next k-step's unpack is interleaved
-// with the current k-step's MFMAs.  X fragments are read from LDS once per 32 output columns.
-//
-// The loading waves copy the slice's X tiles (MT rows x 256 bytes per group, 16-byte chunks
-// XOR-permuted by row % 16) and W tiles (64 columns x 64 bytes per group, 16-byte chunks
-// XOR-permuted by (column / 2) % 4) global -> LDS with `buffer_load ... lds`, in two phases
-// (the first ceil(G / 2) groups, then the rest while the first phase is multiplied), so that
-// a full memory queue stalls only those waves.  The multiplying waves load only the scales
-// of their columns.  The four quarters' sums of each column half are then added through LDS
-// in quarter order.
-//
-// K split: the workgroups of one column tile have block ids congruent modulo 8, which the
-// dispatcher places on one XCD (checked once per device before this kernel is used), so a
-// tile's partial sums and its arrival counter are shared through that XCD's L2.  Each
-// workgroup stores its partial tile, waits until the stores are done, and increments the
-// tile's counter; the workgroup that arrives last loads the other partials (bypassing L1),
-// adds all of them in split order (the same sum whichever workgroup is last), writes the
-// fp16 tile and sets the counter back to zero for the next call.  No workgroup waits for
-// another.  Block id b: XCD group b % 8, split (b / 8) / T8, tile 8 * ((b / 8) % T8) + b % 8,
-// with T8 = ceil(tiles / 8).
-constexpr int kSkWaves = 8;                         // multiplying waves
-constexpr int kSkLoaders = 4;                       // loading waves
-constexpr int kSkMaxGroups = 8;                     // K groups per workgroup
-constexpr int kSkTilesPerXcd = 256;                 // counters per XCD group and stream
-constexpr int kSkMaxTiles = 8 * kSkTilesPerXcd;     // column tiles per call
-constexpr int kSkStreamSlots = kXcdMaxSlots;        // streams per device with their own counters
-
-template <int MT>
-struct SkTile {
-  static constexpr int kX = MT * 256;              // X tile of one group
-  static constexpr int kW = kNTile * 64;           // W tile of one group
-  static constexpr int kSlot = kX + kW;
-  static constexpr int kXCopies = MT / 4;          // 1 KiB copies (16 rows of one X panel)
-  static constexpr int kCopies = kXCopies + 4;     // + 4 of 16 W columns
-  static constexpr int kMSub = MT / 16;            // 16-row blocks
-  static constexpr int kBlocks = 4 * kMSub;        // 16 x 16 output blocks
-  static constexpr int kOwn = kBlocks / kSkWaves;  // blocks each wave finishes
-  static constexpr int kLds = kSkMaxGroups * kSlot;
-  static_assert(kLds <= 160 * 1024, "the slots fit one CU's LDS");
-  static_assert(kBlocks * 4 * 1024 + 16 <= kLds, "the reduction area fits the slots");
-  static_assert(kOwn >= 1 && kBlocks % kSkWaves == 0, "whole blocks per wave");
-};
-
 // fp16 store of C[m][nb .. nb + 3] (columns past N dropped)
 __device__ __forceinline__ void store_half4(const Params& p, floatx4 v, int m, int nb) {
   half_t* dst = p.out + (int64_t)m * p.out_stride + nb;
@@ -420,464 +366,493 @@ __device__ __forceinline__ half8 dequant8_ao(uint32_t d, half2_t s2, uint32_t ma
   return as_half8(r);
 }
 
-template <int MT>
-__global__ __launch_bounds__((kSkWaves + kSkLoaders) * 64, 1) void gemm_sk_kernel(Params p) {
-  using T = SkTile<MT>;
+// K split of a tile whose block b of wave w is acc[b] of every lane.  The workgroups of one tile
+// have block ids congruent modulo 8, which the dispatcher places on one XCD (checked once per
+// device before counters are handed out), so the tile's partial sums and its arrival counter
+// are shared through that XCD's L2.  Each workgroup stores its partials
+// ([tile][split][wave][block][lane]), waits until the stores are done and increments the tile's
+// counter; the one that arrives last loads the other partials (bypassing L1), adds all of them
+// in split order from 0 (the same sum whichever is last) and sets the counter back to zero for
+// the next call.  No workgroup waits for another.  True for the last one, whose acc holds the
+// sums.  `ti`: index of tile t among those of XCD group xg.
+template <int kB>
+__device__ __forceinline__ bool add_splits(const Params& p, floatx4 (&acc)[kB], int t, int s,
+                                           int xg, int ti, int wave, int lane) {
+  __shared__ unsigned arrived;
+  floatx4* part = (floatx4*)p.partial + (int64_t)t * p.ksplit * (4 * kB * 64);
+  floatx4* mine = part + ((int64_t)s * 4 + wave) * (kB * 64) + lane;
+#pragma unroll
+  for (int b = 0; b < kB; ++b) mine[b * 64] = acc[b];
+  if (!p.counters) return false;  // no counters: a second launch adds the splits
+  wait_vmcnt<0>();  // the stores are in L2 before the counter moves
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned* ctr = p.counters + xg * p.counter_stride + ti;
+    const unsigned old = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (old == (unsigned)p.ksplit - 1)  // every other split has arrived: clear for the next call
+      __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    arrived = old;
+  }
+  __syncthreads();
+  if (arrived != (unsigned)p.ksplit - 1) return false;
+  // the other splits' partials, loaded with sc0 (L1 bypassed), four blocks x four splits in
+  // flight; own sums in place of split s
+  const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+      part, (short)0, p.ksplit * 4 * kB * 1024, 0x00020000);
+  constexpr int kBatch = kB < 4 ? kB : 4;
+#pragma unroll
+  for (int b0 = 0; b0 < kB; b0 += kBatch) {
+    floatx4 sum[kBatch] = {};
+    for (int s0 = 0; s0 < p.ksplit; s0 += 4) {
+      floatx4 pv[kBatch][4] = {};
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (s0 + k < p.ksplit && s0 + k != s)
+            pv[b][k] = __builtin_bit_cast(
+                floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                             pr, ((((s0 + k) * 4 + wave) * kB + b0 + b) * 64 + lane) * 16, 0, 1));
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (s0 + k < p.ksplit) sum[b] += s0 + k == s ? acc[b0 + b] : pv[b][k];
+    }
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) acc[b0 + b] = sum[b];
+  }
+  return true;
+}
+
+// The same sum for element `idx` of the partials (one thread each): tile t, place `at` in it.
+template <int kB>
+__device__ __forceinline__ floatx4 split_sum(const Params& p, int64_t idx, int& t, int& at) {
+  at = (int)(idx % (4 * kB * 64));
+  t = (int)(idx / (4 * kB * 64));
+  const floatx4* part = (const floatx4*)p.partial + (int64_t)t * p.ksplit * (4 * kB * 64) + at;
+  floatx4 sum = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < p.ksplit; ++s) sum += part[(int64_t)s * (4 * kB * 64)];
+  return sum;
+}
+
+// ---------------------------------------------------------------------------------------
+// Packed weights, unpacked inside the GEMM: from a few rows up to where one unpacking of the
+// whole weight into memory costs less than unpacking it once per row tile (plan()).
+//
+// One workgroup of four waves per TM-row x 64 NB-column tile of C and K split; wave w owns all
+// TM rows of columns 16 NB w .. 16 NB w + 16 NB - 1, so every weight is read and unpacked by one
+// wave only, straight in registers, and an X fragment read from LDS feeds NB MFMAs.  Per
+// 128-wide K group the tile's X rows are copied global -> LDS (buffer_load ... lds) into one of
+// two stages while the other is multiplied; the next group's weights travel in registers at
+// the same time.  LDS and registers leave room for two workgroups per CU (four of the smaller
+// tiles), so one workgroup's wait at the group boundary is covered by another's MFMAs.
+//
+// X stage layout: two panels of 128 bytes per row (64 k each), 16-byte chunk c of row r at slot
+// c ^ ((r / 2) % 8), so that the 16 rows a quarter-wave reads fall on distinct banks.  Lane
+// group g supplies k = 32 g + 8 q .. +7 in k-step q: its 16 weight bytes of the group.
+//
+// Block ids congruent modulo 8 share an XCD: XCD e takes the e-th eighth of the column-major
+// tile list, so a weight column tile is read by one XCD, and a tile's K splits meet in its L2
+// (add_splits).
+//
+// What bounds it: at small M the weight stream and one memory latency per group; at large M
+// the unpack (18 VALU instructions per eight weights beside TM / 16 MFMAs), which overlaps the
+// MFMAs only in part.  3072 columns, K 8192, batches of layers with cold weights: 509 rows
+// 157 -> 44 us against one unpacking pass and 256 x 256 tiles (24 of them for 256 CUs), 128
+// rows 25.4 -> 17.8 us and 64 rows 18.8 -> 13.5 us against the kernels it replaces there.
+template <int TM, int NB>
+struct MidTile {
+  static constexpr int kN = 64 * NB;           // columns per workgroup
+  static constexpr int kMSub = TM / 16;
+  static constexpr int kBlocks = NB * kMSub;   // 16 x 16 output blocks per wave
+  static constexpr int kStage = TM * 256;      // LDS bytes of one group's X rows
+};
+
+template <int TM, int NB>
+__global__ __launch_bounds__(kThreads, 2) void mid_gemm_kernel(Params p) {
+  using T = MidTile<TM, NB>;
   constexpr int kMSub = T::kMSub;
-  __shared__ __attribute__((aligned(16))) char lds[T::kLds];
+  __shared__ __attribute__((aligned(16))) char lds[2 * T::kStage];
 
   const int t8 = (p.tiles + 7) >> 3;
   const int xg = blockIdx.x & 7, kk = blockIdx.x >> 3;
-  const int s = kk / t8;
-  const int t = 8 * (kk - s * t8) + xg;
-  if (t >= p.tiles) return;  // padding of the last XCD group (uniform, before any barrier)
+  const int s = __builtin_amdgcn_readfirstlane(kk / t8), ti = kk - s * t8;
+  const int t_first = (int)((int64_t)xg * p.tiles >> 3);
+  const int t = t_first + ti;
+  if (t >= (int)((int64_t)(xg + 1) * p.tiles >> 3)) return;  // uniform, before any barrier
+  const int tn = __builtin_amdgcn_readfirstlane(t / p.tiles_m), tm = t - tn * p.tiles_m;
+  const int m0 = tm * TM;
 
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool producer = w >= kSkWaves;
-  const int l = w - kSkWaves;  // loading wave index
-  const int h = (w >> 2) & 1;  // column half
-  const int q = w & 3;         // k-step of every group
-  const int row = lane & 15;
-  const int grp = lane >> 4;
-  const int n0 = t * kNTile;
-  const int groups = p.K / kGroup;
-  const int g_begin = s * p.groups_per_split;
-  const int G = min(p.groups_per_split, groups - g_begin);  // 1 .. 8 (host plan)
-  const int GA = (G + 1) >> 1;                               // groups of phase A
-  const int GB = G - GA;                                     // of phase B
-
-  floatx4 acc[2][kMSub];
-#pragma unroll
-  for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-    for (int i = 0; i < kMSub; ++i) acc[jj][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  if (producer) {
-    // X rows past M and weight rows past N read zeros through the buffer bounds
-    const rsrc_t xr = raw_rsrc(p.x, (int)((min(MT, p.M) - 1) * p.x_stride * 2 + p.K * 2));
-    const rsrc_t wr = raw_rsrc(p.w + (int64_t)n0 * p.w_stride,
-                              (int)((min(kNTile, p.N - n0) - 1) * p.w_stride + p.K / 2));
-    // X of a group is stored as four panels, panel c holding 16-byte chunks 4c .. 4c + 3 of
-    // every row (64 bytes per row); sub-chunk kk of row r of panel c sits at slot
-    // kk ^ ((r / 2) % 4) ^ c.  Loading wave l fills panel l: its copy i covers rows 16i ..
-    // 16i + 15 (row 16i + lane / 4, slot lane % 4).  Then W columns 16cw .. 16cw + 15 (column
-    // 16cw + lane / 4, slot lane % 4 <- 16-byte chunk slot ^ ((column / 2) % 4)); loading wave
-    // l issues W copy cw = l of every group.  Both layouts make the fragment reads of 16
-    // consecutive rows (columns) at one chunk conflict-free; per-lane offsets at group 0.
-    constexpr int kXPer = T::kXCopies / kSkLoaders;
-    static_assert(T::kXCopies % kSkLoaders == 0 && kSkLoaders == 4,
-                  "one X panel per loading wave, whole 16-row copies");
-    int xoff[kXPer];
-#pragma unroll
-    for (int i = 0; i < kXPer; ++i) {
-      const int r = 16 * i + (lane >> 2);
-      const int kk = (lane & 3) ^ ((lane >> 3) & 3) ^ l;
-      xoff[i] = r * (int)p.x_stride * 2 + ((4 * l + kk) << 4);
-    }
-    const int woff = (16 * l + (lane >> 2)) * (int)p.w_stride + (((lane & 3) ^ ((lane >> 3) & 3)) << 4);
-    auto issue = [&](int u0, int gp) {
-#pragma unroll 1
-      for (int u = u0; u < u0 + gp; ++u) {
-        const uint32_t base = lds_addr(lds + u * T::kSlot);
-        const int g = g_begin + u;
-#pragma unroll
-        for (int i = 0; i < kXPer; ++i)
-          lds_copy16(xr, base + l * (MT * 64) + i * 1024, xoff[i], g * 256);
-        lds_copy16(wr, base + T::kX + l * 1024, woff, g * (kGroup / 2));
-      }
-    };
-    // phase A, then phase B while the other waves multiply phase A
-    issue(0, GA);
-    wait_vmcnt<0>();
-    asm volatile("s_barrier" ::: "memory");
-    if (GB > 0) {
-      issue(GA, GB);
-      wait_vmcnt<0>();
-      asm volatile("s_barrier" ::: "memory");
-    }
-  } else {
-    // Wave (h, q) multiplies the q-th quarter of each phase's k-steps (a k-step is 32 k of one
-    // group: lane group grp supplies k = 32 grp + 8k .. +7, weight dword k of the lane's 16
-    // bytes and X chunk 4 grp + k) for its two column blocks j = 2h, 2h + 1.  In a phase of gp
-    // groups from u0 these are k-steps q gp .. q gp + gp - 1, in group u0 + (q gp) / 4 and
-    // possibly the next one (the same group for all four when gp = 4).  The scales of the
-    // lane's columns (16j + row; past N the last column, times zero weights) for those two
-    // groups: sv[jj][second].  These are the only memory loads of these waves, so the
-    // compiler's own wait before their first use waits for nothing else.
-    struct Scales {  // bits of sv[jj][0] in the low half, sv[jj][1] in the high half
-      uint32_t v0, v1;
-    };
-    auto load_scales = [&](int u0, int gp) {
-      const int uf = u0 + (q * gp) / 4;
-      const int us = min(uf + 1, G - 1);
-      uint32_t v[2];
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const uint16_t* sp = (const uint16_t*)p.scales +
-                             (int64_t)min(n0 + 16 * (2 * h + jj) + row, p.N - 1) * p.s_stride + g_begin;
-        v[jj] = (uint32_t)sp[uf] | ((uint32_t)sp[us] << 16);
-      }
-      return Scales{v[0], v[1]};
-    };
-    const Scales sca = load_scales(0, GA);
-    const Scales scb = GB > 0 ? load_scales(GA, GB) : sca;
-    const uint32_t mask = __builtin_amdgcn_readfirstlane(0x000F000Fu);
-    const uint32_t bits = 0x64006400u;
-
-    // One phase, software pipelined: k-step i + 2's fragments are read and k-step i + 1's
-    // weights unpacked while k-step i's MFMAs run.
-    auto run_phase = [&](int u0, int gp, const Scales sv) {
-      const int ks0 = q * gp;
-      const int uf = u0 + ks0 / 4;
-      u32x4 xv[3][kMSub];
-      uint32_t wd[3][2];
-      bool sec[3];
-      half8 wf[2][2];
-      auto read = [&](int b, int i) {  // k-step ks0 + i
-        const int ks = ks0 + i;
-        const int u = u0 + ks / 4, k = ks & 3;
-        const char* slot = lds + u * T::kSlot;
-#pragma unroll
-        for (int ii = 0; ii < kMSub; ++ii)
-          xv[b][ii] = *(const u32x4*)(slot + grp * (MT * 64) + (16 * ii + row) * 64 +
-                                      ((k ^ ((row >> 1) & 3) ^ grp) << 4));
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-          wd[b][jj] = *(const uint32_t*)(slot + T::kX + (16 * (2 * h + jj) + row) * 64 +
-                                         ((grp ^ ((row >> 1) & 3)) << 4) + 4 * k);
-        sec[b] = u != uf;
-      };
-      auto unpack = [&](int b, int i) {
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-          const uint32_t both = jj ? sv.v1 : sv.v0;
-          const half_t sc = __builtin_bit_cast(half_t, (uint16_t)(both >> (sec[b] ? 16 : 0)));
-          wf[i & 1][jj] = dequant8_ao(wd[b][jj], half2_t{sc, sc}, mask, bits);
-        }
-      };
-      read(0, 0);
-      read(1, min(1, gp - 1));
-      unpack(0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (i < gp) {  // uniform
-          if (i + 2 < gp) read((i + 2) % 3, i + 2);
-          // k-step i + 1's unpack (unused past the phase) between k-step i's MFMAs
-          if (i < 3) unpack((i + 1) % 3, i + 1);
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int ii = 0; ii < kMSub; ++ii) {
-              acc[jj][ii] = mfma16x16x32(wf[i & 1][jj], as_half8(xv[i % 3][ii]), acc[jj][ii]);
-              if (i < 3) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 36 / (2 * kMSub), 0);  // then VALU
-              }
-            }
-        }
-      }
-    };
-
-    asm volatile("s_barrier" ::: "memory");  // phase A has landed
-    run_phase(0, GA, sca);
-    if (GB > 0) {
-      asm volatile("s_barrier" ::: "memory");  // phase B has landed
-      run_phase(GA, GB, scb);
-    }
-  }
-
-  // The quarters' sums, added in quarter order through the (now idle) slots: block b = 4 i + j
-  // of quarter q at red[(b * 4 + q) * 64 + lane]; wave (h, q) finishes blocks 2 i + jj = q * kOwn
-  // .. + kOwn - 1 of its half.  The loading waves only take part in the barriers.
-  floatx4* red = (floatx4*)lds;
-  __syncthreads();  // every wave is done with the slots
-  if (!producer) {
-#pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-      for (int i = 0; i < kMSub; ++i)
-        red[((4 * i + 2 * h + jj) * 4 + q) * 64 + lane] = acc[jj][i];
-  }
-  __syncthreads();
-  floatx4 v[T::kOwn];
-  int ob[T::kOwn];  // block index (4 i + j) of each finished block
-#pragma unroll
-  for (int o = 0; o < T::kOwn; ++o) {
-    const int hb = q * T::kOwn + o;  // block within the half: 2 i + jj
-    const int b = 4 * (hb >> 1) + 2 * h + (hb & 1);
-    ob[o] = b;
-    v[o] = red[(b * 4) * 64 + lane];
-#pragma unroll
-    for (int qq = 1; qq < 4; ++qq) v[o] += red[(b * 4 + qq) * 64 + lane];
-  }
-
-  if (p.ksplit > 1) {
-    // partial tile of (t, s): block b at [b][lane], 1 KiB per block
-    floatx4* part = (floatx4*)p.partial + (int64_t)t * p.ksplit * T::kBlocks * 64;
-    if (!producer) {
-#pragma unroll
-      for (int o = 0; o < T::kOwn; ++o) part[((int64_t)s * T::kBlocks + ob[o]) * 64 + lane] = v[o];
-    }
-    if (!p.counters) return;  // no counters: sk_reduce_kernel adds the splits
-    wait_vmcnt<0>();  // the stores are in L2 before the counter moves
-    __syncthreads();
-    unsigned* flag = (unsigned*)(lds + T::kLds - 16);
-    if (threadIdx.x == 0) {
-      unsigned* ctr = p.counters + (t & 7) * kSkTilesPerXcd + (t >> 3);
-      const unsigned old = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (old == (unsigned)p.ksplit - 1)  // every other split has arrived: clear for the next call
-        __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      *flag = old;
-    }
-    __syncthreads();
-    if (*flag != (unsigned)p.ksplit - 1 || producer) return;
-    // the partials of every split, added in split order (own sums in place of split s),
-    // loaded with sc0 (L1 bypassed, served by the XCD's L2)
-    const __amdgpu_buffer_rsrc_t pr =
-        __builtin_amdgcn_make_buffer_rsrc(part, (short)0, p.ksplit * T::kBlocks * 1024, 0x00020000);
-    // every load of a batch of eight splits goes out before the first add
-    floatx4 sum[T::kOwn] = {};
-    for (int s0 = 0; s0 < p.ksplit; s0 += 8) {
-      floatx4 pv[T::kOwn][8] = {};
-#pragma unroll
-      for (int o = 0; o < T::kOwn; ++o)
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (s0 + k < p.ksplit && s0 + k != s)
-            pv[o][k] = __builtin_bit_cast(
-                floatx4, __builtin_amdgcn_raw_buffer_load_b128(
-                             pr, (((s0 + k) * T::kBlocks + ob[o]) * 64 + lane) * 16, 0, 1));
-#pragma unroll
-      for (int o = 0; o < T::kOwn; ++o)
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (s0 + k < p.ksplit) sum[o] += s0 + k == s ? v[o] : pv[o][k];
-    }
-#pragma unroll
-    for (int o = 0; o < T::kOwn; ++o) v[o] = sum[o];
-  }
-  if (producer) return;
-#pragma unroll
-  for (int o = 0; o < T::kOwn; ++o) {
-    const int m = 16 * (ob[o] >> 2) + row;
-    if (m < p.M) store_half4(p, v[o], m, n0 + 16 * (ob[o] & 3) + 4 * grp);
-  }
-}
-
-// gemm_sk_kernel's split sums in a second launch, for streams without arrival counters: the
-// same additions in the same order as the last workgroup of a tile (from 0.f, split 0 first),
-// so both paths give the same bits.  One thread per (tile, 16 x 16 block, lane).
-template <int MT>
-__global__ __launch_bounds__(256) void sk_reduce_kernel(Params p) {
-  using T = SkTile<MT>;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)p.tiles * T::kBlocks * 64) return;
-  const int lane = (int)(idx & 63);
-  const int b = (int)((idx >> 6) % T::kBlocks);
-  const int t = (int)(idx / (64 * T::kBlocks));
-  const floatx4* part = (const floatx4*)p.partial + (int64_t)t * p.ksplit * T::kBlocks * 64;
-  floatx4 sum = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.ksplit; ++s) sum += part[((int64_t)s * T::kBlocks + b) * 64 + lane];
-  const int m = 16 * (b >> 2) + (lane & 15);
-  if (m < p.M) store_half4(p, sum, m, t * kNTile + 16 * (b & 3) + 4 * (lane >> 4));
-}
-
-// Arrival counters of gemm_sk_kernel: one per column tile and stream slot, laid out
-// [XCD group][tile / 8] so that each XCD group's counters share no cache line with another's.
-__device__ __attribute__((aligned(256))) unsigned sk_counters[kSkStreamSlots * kSkMaxTiles];
-
-
-// Prefill-sized calls: the MFMA kernels above spend most of their time dequantizing (each
-// weight is dequantized once per row tile) at these sizes, so the weight is dequantized once
-// into the workspace and a plain fp16 GEMM runs on it: wide_gemm_kernel.
-//
-// C[M, N] = X[M, K] * W[N, K]^T, fp16 in and out, fp32 accumulation, K a multiple of 64.
-// One workgroup per 256 x 256 tile of C, four waves, one per SIMD.  Wave w owns 128 rows
-// (m, 128 * (w / 2)..) x 128 columns (n, 128 * (w % 2)..) of the tile: 8 x 8 MFMA tiles of
-// v_mfma_f32_16x16x32_f16, W as the A operand and X^T as the B operand, 256 fp32 sums held
-// in the accumulation registers (AGPRs), so each 16-byte fragment read from LDS feeds eight
-// MFMAs (a 64 x 128 wave tile feeds four to eight).  Per 64-wide K step the tile's X and W
-// rows (128 bytes each, 16-byte chunk c of row r at slot c ^ ((r / 2) % 8), so the 16 rows a
-// quarter-wave reads fall on distinct banks) are copied global->LDS with buffer_load ... lds
-// into one of two 64 KiB stages.  A step is two k-substeps of 64 MFMAs: the second
-// substep's 16 fragments are read between the first substep's MFMAs; after 48 of the second
-// substep's MFMAs the wave waits for its copies of the next step and passes a barrier (every
-// wave has then read this step's stage and landed the next), and the next step's first
-// fragments are read between the last 16 MFMAs.  The copies of step t + 1 go out between
-// the first substep's MFMAs of step t, into the stage every wave finished reading before
-// the previous step's barrier.
-constexpr int kGemmTile = 256;                     // rows and columns of C per workgroup
-constexpr int kGemmK = 64;                         // K per step
-constexpr int kGemmThreads = 256;
-constexpr int kGemmRowB = kGemmK * 2;              // bytes per LDS row
-constexpr int kGemmOperand = kGemmTile * kGemmRowB;  // 32 KiB: X or W rows of one step
-constexpr int kGemmStage = 2 * kGemmOperand;         // 64 KiB: X rows, then W rows
-
-struct GemmParams {
-  const half_t* x;
-  int64_t ldx;
-  const half_t* w;
-  int64_t ldw;
-  half_t* o;
-  int64_t ldo;
-  int M, N, K;
-  int tiles_m;
-  int band;     // tiles_m / 8 when tiles_m % 8 == 0 (row tiles banded by XCD), else 0
-  int vec_out;  // output rows 16-byte aligned and N % 8 == 0: 16-byte stores
-};
-
-__global__ __launch_bounds__(kGemmThreads, 1) void wide_gemm_kernel(GemmParams p) {
-  __shared__ __attribute__((aligned(16))) char lds[2 * kGemmStage];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wn = wave & 1, wm = wave >> 1;  // wave tile: columns 128 * wn.., rows 128 * wm..
-  // Tile order: with p.band, block id L runs on XCD L % 8 and XCD e takes row tiles
-  // e * band .. e * band + band - 1 against every column tile, so the X rows of its tiles
-  // stay in its own L2; otherwise row tiles vary fastest.
-  int tm, tn;
-  {
-    const int L = blockIdx.x;
-    if (p.band) {
-      const int t = L >> 3;
-      tm = (L & 7) * p.band + t % p.band;
-      tn = t / p.band;
-    } else {
-      tm = L % p.tiles_m;
-      tn = L / p.tiles_m;
+  const int row = lane & 15;
+  const int grp = lane >> 4;
+  const int nw = tn * T::kN + wave * 16 * NB;  // first column of this wave
+  const int groups = p.K / kGroup;
+  const int g_begin = s * p.groups_per_split;
+  const int g_end = min(g_begin + p.groups_per_split, groups);
+
+  // X rows past M read zeros through the buffer bounds
+  const int rows_x = min(TM, p.M - m0);
+  const rsrc_t xr = raw_rsrc(p.x + (int64_t)m0 * p.x_stride,
+                             (int)(((int64_t)(rows_x - 1) * p.x_stride + p.K) * 2));
+  // wave l fills its half (l / 2) of the rows of panel l % 2: copy i covers rows 8 i .. 8 i + 7
+  // of them, lane l row l / 8, slot l % 8 <- chunk (l % 8) ^ ((r / 2) % 8)
+  const int xr0 = (wave >> 1) * (TM / 2) + (lane >> 3);
+  const int xrow = xr0 * (int)p.x_stride * 2 + (wave & 1) * 128;
+  const int xoff0 = xrow + (((lane & 7) ^ ((xr0 >> 1) & 7)) << 4);
+  const int xoff1 = xrow + (((lane & 7) ^ (((xr0 >> 1) + 4) & 7)) << 4);
+  const int xstep = 8 * (int)p.x_stride * 2;
+  const uint32_t lds0 = lds_addr(lds) + (wave & 1) * (TM * 128) + (wave >> 1) * (TM * 64);
+  auto issue_x = [&](int buf, int g) {
+    const int soff = __builtin_amdgcn_readfirstlane(g * 256);
+#pragma unroll
+    for (int i = 0; i < kMSub; ++i)
+      lds_copy16(xr, lds0 + buf * T::kStage + i * 1024, ((i & 1) ? xoff1 : xoff0) + i * xstep, soff);
+  };
+
+  // this lane's weight rows (columns past N compute on the last row, never stored)
+  struct Weights {
+    u32x4 v[NB];
+    uint32_t s[NB];  // scale bits
+  };
+  const uint8_t* wp[NB];
+  const uint16_t* sp[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int64_t n = min(nw + 16 * j + row, p.N - 1);
+    wp[j] = p.w + n * p.w_stride + grp * 16;
+    sp[j] = (const uint16_t*)p.scales + n * p.s_stride;
+  }
+  auto load_w = [&](Weights& w, int g) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      w.v[j] = *(const u32x4*)(wp[j] + (int64_t)g * (kGroup / 2));
+      w.s[j] = sp[j][g];
+    }
+  };
+
+  floatx4 acc[T::kBlocks];  // block j * kMSub + i: columns 16 j.., rows 16 i.. of the wave's
+#pragma unroll
+  for (int b = 0; b < T::kBlocks; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  const uint32_t mask = __builtin_amdgcn_readfirstlane(0x000F000Fu);
+  const uint32_t bits = 0x64006400u;
+  // One group's MFMAs, software pipelined: the next k-step's X fragments are read and its
+  // weights unpacked between this one's MFMAs (sched_group_barrier).
+  auto compute = [&](int buf, const Weights& w) {
+    half8 wf[2][NB], xf[2][kMSub];
+    auto unpack = [&](int q) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+        wf[q & 1][j] = dequant8_ao(w.v[j][q], as_h2(w.s[j] * 0x10001u), mask, bits);
+    };
+    auto read = [&](int q) {
+      const int ch = 4 * grp + q;
+      const char* pa = lds + buf * T::kStage + (ch >> 3) * (TM * 128) + row * 128 +
+                       (((ch & 7) ^ ((row >> 1) & 7)) << 4);
+#pragma unroll
+      for (int i = 0; i < kMSub; ++i) xf[q & 1][i] = as_half8(*(const u32x4*)(pa + i * 2048));
+    };
+    read(0);
+    unpack(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q < 3) {
+        read(q + 1);
+        unpack(q + 1);
+      }
+#pragma unroll
+      for (int i = 0; i < kMSub; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[j * kMSub + i] = mfma16x16x32(wf[q & 1][j], xf[q & 1][i], acc[j * kMSub + i]);
+      if (q < 3) {
+#pragma unroll
+        for (int i = 0; i < kMSub; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one fragment read
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, (20 + kMSub - 1) / kMSub, 0);  // VALU
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // every wave has landed its part of this group's X and its weights, and is done reading
+  // the other stage
+  auto boundary = [&] {
+    wait_vmcnt<0>();
+    wait_lgkmcnt0();
+    asm volatile("s_barrier" ::: "memory");
+  };
+
+  Weights wa, wb;
+  load_w(wa, g_begin);
+  issue_x(0, g_begin);
+  for (int g = g_begin; g < g_end; g += 2) {
+    boundary();
+    if (g + 1 < g_end) {
+      load_w(wb, g + 1);
+      issue_x(1, g + 1);
+    }
+    compute(0, wa);
+    if (g + 1 >= g_end) break;
+    boundary();
+    if (g + 2 < g_end) {
+      load_w(wa, g + 2);
+      issue_x(0, g + 2);
+    }
+    compute(1, wb);
+  }
+
+  if (p.ksplit > 1 && !add_splits<T::kBlocks>(p, acc, t, s, xg, ti, wave, lane)) return;
+#pragma unroll
+  for (int i = 0; i < kMSub; ++i) {
+    const int m = m0 + 16 * i + row;
+    if (m < p.M) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) store_half4(p, acc[j * kMSub + i], m, nw + 16 * j + 4 * grp);
     }
   }
-  const int m0 = tm * kGemmTile, n0 = tn * kGemmTile;
-  const int rows_x = min(kGemmTile, p.M - m0), rows_w = min(kGemmTile, p.N - n0);
+}
+
+// mid_gemm_kernel's split sums in a second launch, for streams without arrival counters: the
+// same additions in the same order.  One thread per (tile, wave, block, lane).
+template <int TM, int NB>
+__global__ __launch_bounds__(256) void mid_reduce_kernel(Params p) {
+  using T = MidTile<TM, NB>;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (int64_t)p.tiles * 4 * T::kBlocks * 64) return;
+  int t, at;
+  const floatx4 sum = split_sum<T::kBlocks>(p, idx, t, at);
+  const int lane = at & 63, b = (at >> 6) % T::kBlocks, wave = at / (64 * T::kBlocks);
+  const int tn = t / p.tiles_m, tm = t - tn * p.tiles_m;
+  const int m = tm * TM + 16 * (b % T::kMSub) + (lane & 15);
+  if (m < p.M)
+    store_half4(p, sum, m, tn * T::kN + wave * 16 * NB + 16 * (b / T::kMSub) + 4 * (lane >> 4));
+}
+
+// ---------------------------------------------------------------------------------------
+// fp16 weights from 5 rows, and packed weights unpacked once into the workspace where the row
+// tiles are many (mid_gemm_kernel spends a third of its time unpacking there).
+//
+// C[M, N] = X[M, K] * W[N, K]^T, fp16 in and out, fp32 accumulation, K a multiple of 128.
+// One workgroup per 32 BM x 32 BN tile of C (and K split), four waves, one per SIMD.  Wave w
+// owns 16 BM rows (m, 16 BM * (w / 2)..) x 16 BN columns (n, 16 BN * (w % 2)..) of the tile: BM x
+// BN MFMA tiles of v_mfma_f32_16x16x32_f16, W as the A operand and X^T as the B operand.  Per
+// 64-wide K step the tile's X and W rows (128 bytes each, 16-byte chunk c of row r at slot
+// c ^ ((r / 2) % 8), so the 16 rows a quarter-wave reads fall on distinct banks) are copied
+// global -> LDS with buffer_load ... lds into one of S stages, S - 1 steps ahead.  A step is two
+// k-substeps: the second substep's fragments are read between the first substep's MFMAs; after
+// three quarters of the second substep's MFMAs the wave waits for its copies of the next step
+// and passes a barrier (every wave has then read this step's stage and landed the next), and
+// the next step's first fragments are read between the last quarter.  The copies go out between
+// the first substep's MFMAs, into the stage every wave finished reading before the previous
+// step's barrier.
+//
+// Tiles: 256 x 256 (256 fp32 sums per lane in the AGPRs, each fragment feeds eight MFMAs, one
+// workgroup per CU) reaches the highest rate, 1.35 PFLOP/s when its tiles fill whole rounds of
+// the CUs; the smaller ones, two workgroups per CU with two to five stages, fill the chip when
+// those tiles are too few (3072 columns, K 8192: 509 rows 160 -> 43 us with 128 x 128 tiles and
+// four K splits; 100 rows x 3072 columns, K 3072: 30 -> 11 us with 64 x 64 and four).
+constexpr int kGemmK = 64;              // K per step
+constexpr int kGemmRowB = kGemmK * 2;   // bytes per LDS row
+
+// Tile of the fp16 GEMM: four waves, two by two, each 16 BM rows x 16 BN columns; S LDS stages.
+template <int BM, int BN, int S>
+struct GemmTile {
+  static constexpr int kM = 32 * BM, kN = 32 * BN;      // rows and columns of C per workgroup
+  static constexpr int kXB = kM * kGemmRowB;            // X rows of one step
+  static constexpr int kStage = kXB + kN * kGemmRowB;   // X rows, then W rows
+  static constexpr int kBlocks = BM * BN;               // 16 x 16 output blocks per wave
+  static constexpr int kOps = BM + BN;                  // copies (and fragments) per wave
+  static constexpr bool kSplit = kBlocks < 64;          // K splits (256 x 256 tiles take none)
+  static constexpr int kPerCu = S * kStage <= 80 * 1024 ? 2 : 1;  // workgroups per CU
+  static_assert(4 * 16 * BM * 32 * BN <= S * kStage, "the staged output fits the stages");
+};
+
+template <int BM, int BN, int S>
+__global__ __launch_bounds__(kThreads, (GemmTile<BM, BN, S>::kPerCu)) void tile_gemm_kernel(Params p) {
+  using T = GemmTile<BM, BN, S>;
+  __shared__ __attribute__((aligned(16))) char lds[S * T::kStage];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wn = wave & 1, wm = wave >> 1;  // wave tile: columns 16 BN wn.., rows 16 BM wm..
+  // Tile order: block id L runs on XCD L % 8.  With p.band XCD e takes row tiles e * band ..
+  // e * band + band - 1 against every column tile (the X rows of its tiles stay in its own
+  // L2); otherwise the e-th eighth of the column-major tile list (its W rows do, and a tile's
+  // K splits meet there).
+  const int xg = blockIdx.x & 7, kk = blockIdx.x >> 3;
+  int tm, tn, s = 0, ti = 0, t = 0;
+  if (p.band) {
+    tm = xg * p.band + kk % p.band;
+    tn = kk / p.band;
+  } else {
+    const int t8 = (p.tiles + 7) >> 3;
+    s = __builtin_amdgcn_readfirstlane(kk / t8);
+    ti = kk - s * t8;
+    t = (int)((int64_t)xg * p.tiles >> 3) + ti;
+    if (t >= (int)((int64_t)(xg + 1) * p.tiles >> 3)) return;  // uniform, before any barrier
+    tn = t / p.tiles_m;
+    tm = t - tn * p.tiles_m;
+  }
+  tm = __builtin_amdgcn_readfirstlane(tm);
+  tn = __builtin_amdgcn_readfirstlane(tn);
+  const int m0 = tm * T::kM, n0 = tn * T::kN;
+  const int rows_x = min(T::kM, p.M - m0), rows_w = min(T::kN, p.N - n0);
   // descriptors over exactly the tile's rows: lanes of rows past M or N read zeros
-  const rsrc_t xr = raw_rsrc(p.x + (int64_t)m0 * p.ldx,
-                             (int)(((int64_t)(rows_x - 1) * p.ldx + p.K) * 2));
-  const rsrc_t wr = raw_rsrc(p.w + (int64_t)n0 * p.ldw,
-                             (int)(((int64_t)(rows_w - 1) * p.ldw + p.K) * 2));
-  // this wave copies rows 64w .. 64w + 63 of X and of W: eight instructions of 8 rows each
-  // per operand; lane l fills slot l % 8 of row r0 + l / 8 with chunk (l % 8) ^ ((r / 2) % 8)
-  int xoff[8], woff[8];
+  const rsrc_t xr = raw_rsrc(p.x + (int64_t)m0 * p.x_stride,
+                             (int)(((int64_t)(rows_x - 1) * p.x_stride + p.K) * 2));
+  const rsrc_t wr = raw_rsrc((const half_t*)p.w + (int64_t)n0 * p.w_stride,
+                             (int)(((int64_t)(rows_w - 1) * p.w_stride + p.K) * 2));
+  // this wave copies a quarter of the X rows and of the W rows, eight rows an instruction;
+  // lane l fills slot l % 8 of row r0 + l / 8 with chunk (l % 8) ^ ((r / 2) % 8)
+  int xoff[BM], woff[BN];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = 64 * wave + 8 * i + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
-    xoff[i] = r < rows_x ? (int)((int64_t)r * p.ldx * 2) + (c << 4) : 0x7ffffff0;
-    woff[i] = r < rows_w ? (int)((int64_t)r * p.ldw * 2) + (c << 4) : 0x7ffffff0;
+  for (int i = 0; i < BM; ++i) {
+    const int r = 8 * (BM * wave + i) + (lane >> 3);
+    xoff[i] = r < rows_x ? (int)((int64_t)r * p.x_stride * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4)
+                         : 0x7ffffff0;
+  }
+#pragma unroll
+  for (int i = 0; i < BN; ++i) {
+    const int r = 8 * (BN * wave + i) + (lane >> 3);
+    woff[i] = r < rows_w ? (int)((int64_t)r * p.w_stride * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4)
+                         : 0x7ffffff0;
   }
   const uint32_t lds0 = lds_addr(lds);
-  const int steps = p.K / kGemmK;
-  // copy q (0..15) of step kt: X rows for q < 8, W rows for q >= 8
-  auto copy = [&](int kt, int q) {
-    const uint32_t base = lds0 + (kt & 1) * kGemmStage;
-    if (q < 8)
-      lds_copy16(xr, base + (64 * wave + 8 * q) * kGemmRowB, xoff[q], kt * kGemmRowB);
+  const int k0 = 2 * s * p.groups_per_split;  // first step (two per 128-wide group)
+  const int steps = min(2 * p.groups_per_split, p.K / kGemmK - k0);
+  // copy q of step kt into stage st: X rows for q < BM, W rows for q >= BM
+  auto copy = [&](int kt, int st, int q) {
+    const uint32_t base = lds0 + st * T::kStage;
+    const int soff = __builtin_amdgcn_readfirstlane((k0 + kt) * kGemmRowB);
+    if (q < BM)
+      lds_copy16(xr, base + 8 * (BM * wave + q) * kGemmRowB, xoff[q < BM ? q : 0], soff);
     else
-      lds_copy16(wr, base + kGemmOperand + (64 * wave + 8 * (q - 8)) * kGemmRowB, woff[q - 8],
-                 kt * kGemmRowB);
+      lds_copy16(wr, base + T::kXB + 8 * (BN * wave + q - BM) * kGemmRowB,
+                 woff[q < BM ? 0 : q - BM], soff);
   };
 
-  floatx4 acc[8][8];
+  floatx4 acc[T::kBlocks];  // block i * BM + j: columns 16 i.., rows 16 j.. of the wave's tile
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int b = 0; b < T::kBlocks; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  // fragment q of k-substep s: W tile q (q < 8) or X tile q - 8, row 16 * tile + fr, chunk
-  // 4s + fg; rows 16i + fr share (row / 2) % 8 with row fr
+  // fragment q of k-substep h: W tile q (q < BN) or X tile q - BN, row 16 * tile + fr, chunk
+  // 4h + fg; rows 16i + fr share (row / 2) % 8 with row fr
   const int fr = lane & 15, fg = lane >> 4;
   const int sw = (fr >> 1) & 7;
-  const int xrow0 = (128 * wm + fr) * kGemmRowB;
-  const int wrow0 = kGemmOperand + (128 * wn + fr) * kGemmRowB;
-  auto frag = [&](const char* st, int s, int q) {
-    const int row0 = q < 8 ? wrow0 + q * 16 * kGemmRowB : xrow0 + (q - 8) * 16 * kGemmRowB;
-    return as_half8(*(const u32x4*)(st + row0 + (((4 * s + fg) ^ sw) << 4)));
+  const int xrow0 = (16 * BM * wm + fr) * kGemmRowB;
+  const int wrow0 = T::kXB + (16 * BN * wn + fr) * kGemmRowB;
+  auto frag = [&](const char* st, int h, int q) {
+    const int row0 = q < BN ? wrow0 + q * 16 * kGemmRowB : xrow0 + (q - BN) * 16 * kGemmRowB;
+    return as_half8(*(const u32x4*)(st + row0 + (((4 * h + fg) ^ sw) << 4)));
   };
-  half8 f0[16], f1[16];
+  half8 f0[T::kOps], f1[T::kOps];
   // the scheduler keeps each group of MFMAs with its reads and copies (sched_barrier)
   auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+  auto mfmas = [&](half8 (&f)[T::kOps], int e0, int e1) {
+#pragma unroll
+    for (int e = e0; e < e1; ++e) acc[e] = mfma16x16x32(f[e / BM], f[BN + e % BM], acc[e]);
+  };
 
 #pragma unroll
-  for (int q = 0; q < 16; ++q) copy(0, q);
-  wait_vmcnt<0>();
-  __builtin_amdgcn_s_barrier();
+  for (int d = 0; d < S - 1; ++d)
+    if (d < steps) {
+#pragma unroll
+      for (int q = 0; q < T::kOps; ++q) copy(d, d, q);
+    }
+  if (steps >= S - 1)
+    wait_vmcnt<(S - 2) * T::kOps>();
+  else
+    wait_vmcnt<0>();
+  asm volatile("s_barrier" ::: "memory");
   fence();
 #pragma unroll
-  for (int q = 0; q < 16; ++q) f0[q] = frag(lds, 0, q);
+  for (int q = 0; q < T::kOps; ++q) f0[q] = frag(lds, 0, q);
   fence();
-  auto step = [&](int kt, auto more_c) {
-    constexpr bool more = decltype(more_c)::value;  // a step follows
-    const char* st = lds + (kt & 1) * kGemmStage;
-    // substep 0 on f0; substep 1's fragments read and the next step's copies issued
+  int cur = 0, fill = S - 1;  // stages of this step and of the step the copies go to
+  // kMore: a step follows; kFill: step kt + S - 1 exists
+  auto step = [&](int kt, auto more_c, auto fill_c) {
+    constexpr bool kMore = decltype(more_c)::value, kFill = decltype(fill_c)::value;
+    const char* st = lds + cur * T::kStage;
+    // substep 0 on f0; substep 1's fragments read and step kt + S - 1's copies issued
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
+    for (int g = 0; g < T::kOps; ++g) {
       f1[g] = frag(st, 1, g);
-      if constexpr (more) copy(kt + 1, g);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int e = 4 * g + t, i = e >> 3, j = e & 7;
-        acc[i][j] = mfma16x16x32(f0[i], f0[8 + j], acc[i][j]);
-      }
+      if constexpr (kFill) copy(kt + S - 1, fill, g);
+      mfmas(f0, g * T::kBlocks / T::kOps, (g + 1) * T::kBlocks / T::kOps);
       fence();
     }
-    // substep 1 on f1: 48 MFMAs, the wait and barrier, then 16 MFMAs with the next step's
-    // substep-0 fragments read between them
+    // substep 1 on f1: three quarters of its MFMAs, the wait and barrier, then the last
+    // quarter with the next step's substep-0 fragments read between them
+    constexpr int kQ = T::kBlocks * 3 / 4;
 #pragma unroll
-    for (int g = 0; g < 12; ++g) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int e = 4 * g + t, i = e >> 3, j = e & 7;
-        acc[i][j] = mfma16x16x32(f1[i], f1[8 + j], acc[i][j]);
-      }
+    for (int e = 0; e < kQ; e += 4) {
+      mfmas(f1, e, e + 4 < kQ ? e + 4 : kQ);
       fence();
     }
-    if constexpr (more) {
-      wait_vmcnt<0>();
-      __builtin_amdgcn_s_barrier();
+    if constexpr (kMore) {
+      wait_vmcnt<kFill ? (S - 2) * T::kOps : 0>();
+      wait_lgkmcnt0();
+      asm volatile("s_barrier" ::: "memory");
       fence();
     }
-    const char* nst = lds + ((kt + 1) & 1) * kGemmStage;
+    cur = cur + 1 == S ? 0 : cur + 1;
+    fill = fill + 1 == S ? 0 : fill + 1;
+    const char* nst = lds + cur * T::kStage;
+    constexpr int kR = T::kBlocks - kQ < 4 ? T::kBlocks - kQ : 4;  // read groups
 #pragma unroll
-    for (int g = 12; g < 16; ++g) {
-      if constexpr (more) {
+    for (int g = 0; g < kR; ++g) {
+      if constexpr (kMore) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) f0[4 * (g - 12) + u] = frag(nst, 0, 4 * (g - 12) + u);
+        for (int u = g * T::kOps / kR; u < (g + 1) * T::kOps / kR; ++u) f0[u] = frag(nst, 0, u);
       }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int e = 4 * g + t, i = e >> 3, j = e & 7;
-        acc[i][j] = mfma16x16x32(f1[i], f1[8 + j], acc[i][j]);
-      }
+      mfmas(f1, kQ + g * (T::kBlocks - kQ) / kR, kQ + (g + 1) * (T::kBlocks - kQ) / kR);
       fence();
     }
   };
-  for (int kt = 0; kt + 1 < steps; ++kt) step(kt, std::true_type{});
-  step(steps - 1, std::false_type{});
-  __builtin_amdgcn_s_barrier();  // every wave is done with the stages
+  int kt = 0;
+  for (; kt + S - 1 < steps; ++kt) step(kt, std::true_type{}, std::true_type{});
+  for (; kt + 1 < steps; ++kt) step(kt, std::true_type{}, std::false_type{});
+  step(steps - 1, std::false_type{}, std::false_type{});
+
+  if constexpr (T::kSplit)
+    if (p.ksplit > 1 && !add_splits<T::kBlocks>(p, acc, t, s, xg, ti, wave, lane)) return;
+  wait_lgkmcnt0();
+  __syncthreads();  // every wave is done with the stages
   fence();
 
-  // Lane (m = 16j + fr, fg) holds C[m][16i + 4fg .. +3] of the wave's block.  Rows go
-  // through the wave's own 32 KiB of LDS (fp16, 256 bytes a row, chunk c of row m at
-  // c ^ (m % 16)) so that 16 lanes store one row's 256 bytes.
-  char* cs = lds + wave * (128 * 256);
+  // Lane (m = 16j + fr, fg) holds C[m][16i + 4fg .. +3] of the wave's tile.  Rows go through
+  // the wave's own part of the LDS (fp16, chunk c of row m at c ^ (m % chunks)) so that whole
+  // rows of the wave's tile are stored by consecutive lanes.
+  constexpr int kRow = 32 * BN, kCh = 2 * BN;
+  char* cs = lds + wave * (16 * BM * kRow);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < BM; ++j) {
     const int m = 16 * j + fr;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < BN; ++i) {
       const int c = 2 * i + (fg >> 1);
-      *(half4*)(cs + m * 256 + ((c ^ (m & 15)) << 4) + ((fg & 1) << 3)) = to_half4(acc[i][j]);
+      *(half4*)(cs + m * kRow + ((c ^ (m & (kCh - 1))) << 4) + ((fg & 1) << 3)) =
+          to_half4(acc[i * BM + j]);
     }
   }
   wave_lds_sync();
-  const int sr = lane >> 4, sc = lane & 15;
-  const int gn = n0 + 128 * wn + 8 * sc;
+  const int sr = lane / kCh, sc = lane % kCh;
+  const int gn = n0 + 16 * BN * wn + 8 * sc;
 #pragma unroll 4
-  for (int q = 0; q < 32; ++q) {
-    const int m = 4 * q + sr;
-    const u32x4 v = *(const u32x4*)(cs + m * 256 + ((sc ^ (m & 15)) << 4));
-    const int gm = m0 + 128 * wm + m;
+  for (int q = 0; q < 16 * BM * kCh / 64; ++q) {
+    const int m = (64 / kCh) * q + sr;
+    const u32x4 v = *(const u32x4*)(cs + m * kRow + ((sc ^ (m & (kCh - 1))) << 4));
+    const int gm = m0 + 16 * BM * wm + m;
     if (gm >= p.M || gn >= p.N) continue;
-    half_t* dst = p.o + (int64_t)gm * p.ldo + gn;
+    half_t* dst = p.out + (int64_t)gm * p.out_stride + gn;
     if (p.vec_out) {
       *(u32x4*)dst = v;
     } else {
@@ -889,35 +864,20 @@ __global__ __launch_bounds__(kGemmThreads, 1) void wide_gemm_kernel(GemmParams p
   }
 }
 
-// C[M, N] (ldc) = X[M, K] (ldx) * W[N, K]^T (ldw), all fp16 row-major, fp32 accumulation;
-// K a multiple of 64, rows of X and W 16-byte aligned.
-inline int f16_gemm(const half_t* x, int64_t ldx, const half_t* w, int64_t ldw, half_t* out,
-                    int64_t ldc, int64_t M, int64_t N, int64_t K, hipStream_t st) {
-  if (K % kGemmK || ((int64_t)(kGemmTile - 1) * std::max(ldx, ldw) + K) * 2 >= 0x7ffffff0) {
-    set_error("fi_int4_matmul: 256 rows of X or W span 2^31 bytes or more");
-    return FI_ERR_UNSUPPORTED;
-  }
-  GemmParams p;
-  p.x = x;
-  p.ldx = ldx;
-  p.w = w;
-  p.ldw = ldw;
-  p.o = out;
-  p.ldo = ldc;
-  p.M = (int)M;
-  p.N = (int)N;
-  p.K = (int)K;
-  p.tiles_m = (int)((M + kGemmTile - 1) / kGemmTile);
-  const int64_t tiles_n = (N + kGemmTile - 1) / kGemmTile;
-  const int64_t tiles = p.tiles_m * tiles_n;
-  if (tiles > 0x7fffffff) {
-    set_error("fi_int4_matmul: too many output tiles");
-    return FI_ERR_UNSUPPORTED;
-  }
-  p.band = p.tiles_m % 8 == 0 ? p.tiles_m / 8 : 0;
-  p.vec_out = ((uintptr_t)out & 15) == 0 && ldc % 8 == 0 && N % 8 == 0;
-  hipLaunchKernelGGL(wide_gemm_kernel, dim3((unsigned)tiles), dim3(kGemmThreads), 0, st, p);
-  return check_launch("fi_int4_matmul");
+// tile_gemm_kernel's split sums in a second launch, for streams without arrival counters: the
+// same additions in the same order.  One thread per (tile, wave, block, lane).
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void tile_reduce_kernel(Params p) {
+  constexpr int kB = BM * BN;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (int64_t)p.tiles * 4 * kB * 64) return;
+  int t, at;
+  const floatx4 sum = split_sum<kB>(p, idx, t, at);
+  const int lane = at & 63, b = (at >> 6) % kB, wave = at / (64 * kB);
+  const int tn = t / p.tiles_m, tm = t - tn * p.tiles_m;
+  const int m = tm * 32 * BM + (wave >> 1) * 16 * BM + 16 * (b % BM) + (lane & 15);
+  if (m < p.M)
+    store_half4(p, sum, m, tn * 32 * BN + (wave & 1) * 16 * BN + 16 * (b / BM) + 4 * (lane >> 4));
 }
 
 // Decode-sized calls (16 rows of X per blockIdx.y): one workgroup per 16 output columns.
@@ -1081,35 +1041,15 @@ __global__ __launch_bounds__(64 * kW, kNorm ? 1 : 2) void gemv_kernel(Params p) 
 }
 
 // out[m, n] = fp16(sum over splits of partial[s, m, n]), splits added in order.
-template <int V>
 __global__ __launch_bounds__(256) void reduce_kernel(const float* partial, int splits, int M,
                                                      int N, half_t* out, int64_t out_stride) {
-  // V consecutive outputs of one row per thread (V = 4: N % 4 == 0 and 8-byte aligned output
-  // rows).  The partials of up to 8 splits are loaded before any is added, so one memory
-  // latency covers them; the sum runs in split order from 0.f either way.
-  typedef float fv __attribute__((ext_vector_type(V)));
   const int64_t total = (int64_t)M * N;
-  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * V; i < total;
-       i += (int64_t)gridDim.x * blockDim.x * V) {
-    fv s = {};
-    for (int k0 = 0; k0 < splits; k0 += 8) {
-      fv v[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (k0 + k < splits)
-          v[k] = __builtin_nontemporal_load((const fv*)(partial + (k0 + k) * total + i));
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        if (k0 + k < splits) s += v[k];
-    }
-    const int m = (int)(i / N);
-    const int nn = (int)(i - (int64_t)m * N);
-    half_t* dst = out + (int64_t)m * out_stride + nn;
-    if constexpr (V == 4) {
-      *(half4*)dst = to_half4(s);
-    } else {
-      dst[0] = (half_t)s[0];
-    }
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    float s = 0.f;
+    for (int k = 0; k < splits; ++k) s += partial[k * total + i];
+    const int64_t m = i / N;
+    out[m * out_stride + (i - m * N)] = (half_t)s;
   }
 }
 
@@ -1173,65 +1113,117 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* packed, 
   }
 }
 
-// Kernel, tile rows and split count for an (M, N, K) call; shared by the size query and
-// the launch.  gemv_rows: X rows per gemv launch row (0 = use the tiled kernel).
+// Kernel, tile and split count for an (M, N, K) call; shared by the size query and the launch.
 struct Plan {
-  int mt;
+  bool gemv;    // gemv_kernel; otherwise mt x nt tiles:
+  bool dense;   // tile_gemm_kernel (packed weights are first unpacked into the workspace), or
+                // mid_gemm_kernel
+  int mt, nt;
   int splits;
-  int gemv_rows;
-  bool dense;  // prefill-sized: dequantize once, then a plain fp16 GEMM (f16_gemm)
-  bool sk;       // packed weights, 17..64 rows: gemm_sk_kernel (K split added in-launch)
 };
 
-// Dispatch thresholds (rows of X), chosen by measurement on MI355X: the one-pass kernel
-// up to 16 rows, the tiled split-K kernels up to 128, the plain fp16 GEMM above.
-constexpr int kGemvMaxM = 16;
+// Rows from which a call may use the dense 256 x 256 tiles; below, X rows may be any distance
+// apart, from here 256 rows of X (and of an fp16 W) have to span less than 2 GiB.
 constexpr int kDenseMinM = 129;
+constexpr int kGemvMaxM = 16;    // rows of one gemv_kernel workgroup
+constexpr int kFusedNormM = 4;   // gemv_kernel whatever its cost below (the norm is fused there)
+constexpr int kMaxSplits = 10;
+constexpr int kMaxSplitTiles = 8 * kXcdCounters;  // tiles of a split call
 
-// int4: packed weights.  cus: compute units of the device.
-inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, int cus) {
-  Plan pl;
-  pl.gemv_rows = 0;
-  pl.dense = false;
-  pl.sk = false;
-  if (M >= kDenseMinM) {
-    pl.dense = true;
-    pl.mt = 0;
-    pl.splits = 1;
-    return pl;
-  }
-  if (M <= kGemvMaxM && (M + 15) / 16 <= 65535) {
-    pl.gemv_rows = 16;
-    pl.mt = 16;
-    pl.splits = 1;
-    return pl;
-  }
+// Time of a call with one tile shape, in us, as measured on MI355X (3072, 5120 and 16384
+// columns, K 3072 and 8192, 5 to 5000 rows, cold weights, fitted by least squares; the tile
+// chosen by it is within 1.3% of the fastest measured on average):
+//   fixed + groups per split x (full rounds x load[per_cu] + load[workgroups of the last round
+//   on a CU]) + (K split: split + per_split x splits)
+// where a round is per_cu workgroups on every CU, and load[n] the time of one 128-wide K group
+// with n workgroups on the CU.
+struct TileCost {
+  bool dense;
+  int mt, nt, per_cu;
+  float fixed, load[5], split, per_split;
+};
+constexpr TileCost kPackedTiles[] = {
+    {false, 16, 64, 4, 3.4f, {0, 0.46f, 0.52f, 0.74f, 1.01f}, 0.94f, 0.15f},
+    {false, 32, 64, 4, 3.4f, {0, 0.49f, 0.57f, 0.86f, 1.28f}, 1.11f, 0.24f},
+    {false, 64, 64, 4, 4.6f, {0, 0.53f, 0.73f, 1.28f, 1.67f}, 1.12f, 0.28f},
+    {false, 64, 128, 4, 6.8f, {0, 0.77f, 1.36f, 2.12f, 2.83f}, 0.54f, 0.51f},
+    {false, 128, 64, 2, 3.5f, {0, 0.82f, 1.43f}, 2.0f, 0.73f},
+    {false, 128, 128, 2, 4.8f, {0, 1.28f, 2.22f}, 3.15f, 1.22f},
+    {true, 128, 128, 2, 2.4f, {0, 1.53f, 1.82f}, 0, 0},
+    {true, 256, 256, 1, 7.1f, {0, 2.45f}, 0, 0},
+};
+constexpr TileCost kHalfTiles[] = {
+    {true, 32, 64, 2, 6.1f, {0, 0.28f, 0.55f}, 0.22f, 0.36f},
+    {true, 64, 64, 2, 6.3f, {0, 0.37f, 0.76f}, 0.61f, 0.46f},
+    {true, 64, 128, 2, 5.9f, {0, 0.63f, 1.28f}, 2.43f, 0.61f},
+    {true, 128, 64, 2, 4.8f, {0, 0.66f, 1.29f}, 2.52f, 0.73f},
+    {true, 128, 128, 2, 0.7f, {0, 1.59f, 2.09f}, 8.33f, 1.21f},
+    {true, 256, 256, 1, 0.2f, {0, 2.85f}, 0, 0},
+};
+
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The same for gemv_kernel (fits 5 to 16 rows of the shapes above): its workgroups on a CU add
+// up, and every one reads the M rows of X.
+inline float gemv_cost(int64_t M, int64_t N, int64_t groups, bool int4, int cus) {
+  const float load = (float)ceil_div(ceil_div(N, 16), cus);
+  return int4 ? 2.2f + groups * (0.1f + 0.064f * (load - 1) + 0.0055f * load * M)
+              : 1.65f + groups * (0.2f + 0.155f * (load - 1) + 0.0053f * load * M);
+}
+
+// fp32 partial sums of a tiled plan, bytes
+inline int64_t partial_bytes(int64_t M, int64_t N, const Plan& pl) {
+  return pl.splits <= 1 ? 0 : pl.splits * ceil_div(M, pl.mt) * pl.mt * ceil_div(N, pl.nt) * pl.nt * 4;
+}
+
+// The cheapest plan; split_ok false: without a K split (no workspace for its partials).
+inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, int cus, bool split_ok) {
   const int64_t groups = K / kGroup;
-  const int64_t tiles = (N + kNTile - 1) / kNTile;
-  if (int4 && M <= 64) {
-    // one workgroup per (column tile, K split), at most eight groups each, about one per CU
-    pl.sk = true;
-    pl.mt = M <= 32 ? 32 : 64;
-    const int64_t lo = (groups + kSkMaxGroups - 1) / kSkMaxGroups;
-    const int64_t s = std::max<int64_t>(lo, std::min<int64_t>(groups, cus / tiles));
-    const int64_t per = (groups + s - 1) / s;
-    pl.splits = (int)((groups + per - 1) / per);
-    return pl;
+  Plan best{true, false, 16, 16, 1};
+  if (M <= kFusedNormM) return best;
+  float best_us = M <= kGemvMaxM ? gemv_cost(M, N, groups, int4, cus) : 1e30f;
+  const TileCost* costs = int4 ? kPackedTiles : kHalfTiles;
+  const int n = int4 ? (int)(sizeof(kPackedTiles) / sizeof(TileCost))
+                     : (int)(sizeof(kHalfTiles) / sizeof(TileCost));
+  for (int c = 0; c < n; ++c) {
+    const TileCost& t = costs[c];
+    if (int4 && t.dense && M < kDenseMinM) continue;
+    const int64_t tiles = ceil_div(M, t.mt) * ceil_div(N, t.nt);
+    if (tiles > 0x7ffffff) continue;
+    const bool may_split = split_ok && (t.split > 0) && tiles <= kMaxSplitTiles;
+    for (int64_t s = 1; s <= kMaxSplits && s <= groups; ++s) {
+      if (s > 1 && (!may_split || tiles * s > 5 * (int64_t)cus)) break;
+      const int64_t per = ceil_div(groups, s), splits = ceil_div(groups, per);
+      if (splits != s) continue;  // a smaller count with the same groups per split
+      const Plan pl{false, t.dense, t.mt, t.nt, (int)splits};
+      // the partials of a call that large stay within the unpacked weight's bytes
+      if (M >= kDenseMinM && partial_bytes(M, N, pl) > N * K * 2) break;
+      const int64_t on_cu = ceil_div(tiles * splits, cus);
+      float us = t.fixed + per * ((on_cu / t.per_cu) * t.load[t.per_cu] + t.load[on_cu % t.per_cu]);
+      if (splits > 1) us += t.split + t.per_split * splits;
+      if (int4 && t.dense) us += 2.5f + 0.62e-6f * N * K;  // unpacking the weight first
+      if (us < best_us) {
+        best_us = us;
+        best = pl;
+      }
+    }
   }
-  pl.mt = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : 128;
-  const int64_t wgs = ((N + kNTile - 1) / kNTile) * ((M + pl.mt - 1) / pl.mt);
-  int64_t s = 1;
-  if (wgs < 256) {
-    s = (512 + wgs - 1) / wgs;
-    // keep the fp32 partials (written and read once) below the weight bytes
-    const int64_t cap = std::max<int64_t>(1, K / (16 * std::max<int64_t>(M, 1)));
-    s = std::min<int64_t>(std::min<int64_t>(s, cap), groups);
-  }
-  // every split gets the same whole number of groups
-  const int64_t per = (groups + s - 1) / std::max<int64_t>(s, 1);
-  pl.splits = (int)((groups + per - 1) / std::max<int64_t>(per, 1));
-  if (pl.splits < 1) pl.splits = 1;
-  return pl;
+  return best;
+}
+
+// choose_plan, remembered per thread for the last few sizes (it weighs some 50 plans).
+inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, int cus, bool split_ok = true) {
+  struct Entry {
+    int64_t M, N, K;
+    int form;
+    Plan pl;
+  };
+  static thread_local Entry memo[64] = {};
+  const int form = 4 * cus + 2 * int4 + split_ok;
+  Entry& e = memo[(M * 31 + N * 7 + K / kGroup * 3 + form) & 63];
+  if (e.M != M || e.N != N || e.K != K || e.form != form)
+    e = Entry{M, N, K, form, choose_plan(M, N, K, int4, cus, split_ok)};
+  return e.pl;
 }
 
 }  // namespace gemm
@@ -1240,7 +1232,6 @@ inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, int cus) {
 namespace {
 
 using fi::half_t;
-using fi::gemm::f16_gemm;
 using fi::gemm::dequantize_kernel;
 using fi::gemm::rmsnorm_kernel;
 
@@ -1285,119 +1276,106 @@ int check_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int
   return FI_OK;
 }
 
-// Arrival counters of gemm_sk_kernel for the stream `st`: one set per stream slot (other
-// streams add their splits in a second launch), each zero at load and left zero by every
-// call; only on a device where block ids congruent modulo 8 share an XCD.
-unsigned* sk_counters_for(hipStream_t st) {
-  using fi::gemm::kSkMaxTiles;
-  constexpr int kMaxDevices = 64;
-  static std::atomic<unsigned*> base[kMaxDevices];
-  if (!fi::xcd_groups_ok(st)) return nullptr;
-  const int slot = fi::xcd_stream_slot(st, 0, fi::gemm::kSkStreamSlots);
-  if (slot < 0) return nullptr;
-  hipDevice_t d;
-  if (hipStreamGetDevice(st, &d) != hipSuccess || (int)d < 0 || (int)d >= kMaxDevices) return nullptr;
-  unsigned* b = base[(int)d].load();
-  if (!b) {
-    int cur = -1;
-    if (hipGetDevice(&cur) != hipSuccess) return nullptr;
-    if (cur != (int)d && hipSetDevice((int)d) != hipSuccess) return nullptr;
-    void* addr = nullptr;
-    const bool ok = hipGetSymbolAddress(&addr, HIP_SYMBOL(fi::gemm::sk_counters)) == hipSuccess;
-    if (cur != (int)d) (void)hipSetDevice(cur);
-    if (!ok || !addr) return nullptr;
-    b = (unsigned*)addr;
-    base[(int)d].store(b);
+// mid_gemm_kernel and tile_gemm_kernel address the tile's rows of X (and tile_gemm_kernel those
+// of W) with 32-bit buffer offsets.
+bool spans_ok(const fi::gemm::Params& p, const fi::gemm::Plan& pl) {
+  const int64_t x_span = ((pl.mt - 1) * p.x_stride + p.K) * 2;
+  const int64_t w_span = pl.dense ? ((pl.nt - 1) * p.w_stride + p.K) * 2 : 0;
+  return x_span < 0x7ffffff0 && w_span < 0x7ffffff0;
+}
+
+template <typename Kernel, typename Reduce>
+void launch_tiles(Kernel kernel, Reduce reduce, const fi::gemm::Params& p, int64_t tile_floats,
+                  hipStream_t st) {
+  const dim3 grid((unsigned)(8 * p.ksplit * ((p.tiles + 7) / 8)));
+  hipLaunchKernelGGL(kernel, grid, dim3(fi::gemm::kThreads), 0, st, p);
+  if (p.ksplit > 1 && !p.counters) {
+    const int64_t threads = p.tiles * tile_floats / 4;
+    hipLaunchKernelGGL(reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, p);
   }
-  return b + (size_t)slot * kSkMaxTiles;
 }
 
-// gemm_sk_kernel addresses X and the weight tile rows with 32-bit buffer offsets.
-bool dma_ok_sk(const fi::gemm::Params& p, const fi::gemm::Plan& pl) {
+template <int TM, int NB>
+void launch_mid(const fi::gemm::Params& p, hipStream_t st) {
   using namespace fi::gemm;
-  const int64_t x_span = (int64_t)pl.mt * p.x_stride * 2 + (int64_t)p.K * 2;
-  const int64_t w_span = (int64_t)kNTile * p.w_stride + p.K / 2;
-  return x_span < (1ll << 31) - 4096 && w_span < (1ll << 31) - 4096;
+  launch_tiles(mid_gemm_kernel<TM, NB>, mid_reduce_kernel<TM, NB>, p, TM * 64 * NB, st);
 }
 
-// kNorm: the RMSNorm is fused into the decode kernel (only on the gemv path).
-template <bool kNorm>
-void launch_linear(const fi::gemm::Params& base, bool int4, const fi::gemm::Plan& pl,
-                   void* workspace, hipStream_t st) {
+template <int BM, int BN, int S>
+void launch_tile_gemm(fi::gemm::Params p, hipStream_t st) {
   using namespace fi::gemm;
-  Params p = base;
-  if (pl.sk && dma_ok_sk(p, pl)) {
-    // the split's arrival counters; without them (more than kSkMaxTiles column tiles, a
-    // stream past the per-device sets, a device whose dispatch does not group block ids by
-    // XCD, or a first call under graph capture) the workgroups only store their partials and
-    // sk_reduce_kernel adds them
-    const int groups = p.K / kGroup;
-    p.groups_per_split = (groups + pl.splits - 1) / pl.splits;
-    p.partial = (float*)workspace;
-    p.tiles = (p.N + kNTile - 1) / kNTile;
-    p.ksplit = pl.splits;
-    p.counters = pl.splits > 1 && p.tiles <= kSkMaxTiles ? sk_counters_for(st) : nullptr;
-    const dim3 grid((unsigned)(8 * pl.splits * ((p.tiles + 7) / 8)));
-    const dim3 block((kSkWaves + kSkLoaders) * 64);
-    if (pl.mt == 32)
-      hipLaunchKernelGGL(gemm_sk_kernel<32>, grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL(gemm_sk_kernel<64>, grid, block, 0, st, p);
-    if (pl.splits > 1 && !p.counters) {
-      const int64_t threads = (int64_t)p.tiles * 4 * (pl.mt / 16) * 64;
-      const dim3 rgrid((unsigned)((threads + 255) / 256));
-      if (pl.mt == 32)
-        hipLaunchKernelGGL(sk_reduce_kernel<32>, rgrid, dim3(256), 0, st, p);
-      else
-        hipLaunchKernelGGL(sk_reduce_kernel<64>, rgrid, dim3(256), 0, st, p);
+  p.band = BM == 8 && BN == 8 && p.tiles_m % 8 == 0 ? p.tiles_m / 8 : 0;
+  launch_tiles(tile_gemm_kernel<BM, BN, S>, tile_reduce_kernel<BM, BN>, p, 1024 * BM * BN, st);
+}
+
+// A tiled plan's launch.  Without arrival counters (a stream past the per-device sets, a device
+// whose dispatch does not group block ids by XCD, a first call under graph capture) the
+// workgroups only store their partials and a second launch adds them, in the same order.
+void launch_plan(fi::gemm::Params p, const fi::gemm::Plan& pl, void* workspace, hipStream_t st) {
+  using namespace fi::gemm;
+  p.groups_per_split = (int)ceil_div(p.K / kGroup, pl.splits);
+  p.partial = (float*)workspace;
+  p.tiles_m = (int)ceil_div(p.M, pl.mt);
+  p.tiles = p.tiles_m * (int)ceil_div(p.N, pl.nt);
+  p.ksplit = pl.splits;
+  if (pl.splits > 1)
+    p.counters = fi::xcd_counters(st, (p.tiles + 7) / 8, &p.counter_stride);
+  p.vec_out = ((uintptr_t)p.out & 15) == 0 && p.out_stride % 8 == 0 && p.N % 8 == 0;
+  const int tile = pl.mt * 1000 + pl.nt;
+  if (pl.dense) {
+    switch (tile) {
+      case 32064: launch_tile_gemm<1, 2, 5>(p, st); break;
+      case 64064: launch_tile_gemm<2, 2, 4>(p, st); break;
+      case 64128: launch_tile_gemm<2, 4, 3>(p, st); break;
+      case 128064: launch_tile_gemm<4, 2, 3>(p, st); break;
+      case 128128: launch_tile_gemm<4, 4, 2>(p, st); break;
+      default: launch_tile_gemm<8, 8, 2>(p, st); break;
     }
     return;
   }
-  if (kNorm || pl.gemv_rows) {
-    p.partial = nullptr;
-    p.groups_per_split = p.K / kGroup;
-    const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)((p.M + 15) / 16), 1);
-    const size_t lds = kNorm ? (size_t)std::min(p.M, 16) * p.K * sizeof(half_t) : 0;
-    // packed weights: eight waves (two per SIMD hide the dequantization's VALU latency),
-    // except with the fused norm, whose registers allow only one such workgroup per CU
-    if (int4 && !kNorm)
-      hipLaunchKernelGGL((gemv_kernel<true, 3, false, 8>), grid, dim3(512), lds, st, p);
-    else if (int4)
-      hipLaunchKernelGGL((gemv_kernel<true, 6, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
-    else
-      hipLaunchKernelGGL((gemv_kernel<false, 3, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
-    return;
+  switch (tile) {
+    case 16064: launch_mid<16, 1>(p, st); break;
+    case 32064: launch_mid<32, 1>(p, st); break;
+    case 64064: launch_mid<64, 1>(p, st); break;
+    case 64128: launch_mid<64, 2>(p, st); break;
+    case 128064: launch_mid<128, 1>(p, st); break;
+    default: launch_mid<128, 2>(p, st); break;
   }
-  p.partial = pl.splits > 1 ? (float*)workspace : nullptr;
-  const int groups = p.K / kGroup;
-  p.groups_per_split = (groups + pl.splits - 1) / pl.splits;
-  const dim3 grid((unsigned)((p.N + kNTile - 1) / kNTile), (unsigned)((p.M + pl.mt - 1) / pl.mt),
-                  (unsigned)pl.splits);
-#define FI_GEMM_LAUNCH(MT)                                                                    \
-  do {                                                                                      \
-    if (int4)                                                                               \
-      hipLaunchKernelGGL((gemm_kernel<MT, true>), grid, dim3(kThreads), 0, st, p);           \
-    else                                                                                    \
-      hipLaunchKernelGGL((gemm_kernel<MT, false>), grid, dim3(kThreads), 0, st, p);          \
-  } while (0)
-  switch (pl.mt) {
-    case 16: FI_GEMM_LAUNCH(16); break;
-    case 32: FI_GEMM_LAUNCH(32); break;
-    case 64: FI_GEMM_LAUNCH(64); break;
-    default: FI_GEMM_LAUNCH(128); break;
-  }
-#undef FI_GEMM_LAUNCH
-  if (pl.splits > 1) {
-    const int64_t total = (int64_t)p.M * p.N;
-    const bool v4 = p.N % 4 == 0 && p.out_stride % 4 == 0 && ((uintptr_t)p.out & 7) == 0;
-    const int64_t blocks = std::min<int64_t>((total / (v4 ? 4 : 1) + 255) / 256, 4096);
-    if (v4)
-      hipLaunchKernelGGL(reduce_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, st,
-                         (const float*)workspace, pl.splits, p.M, p.N, p.out, p.out_stride);
-    else
-      hipLaunchKernelGGL(reduce_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, st,
-                         (const float*)workspace, pl.splits, p.M, p.N, p.out, p.out_stride);
-  }
+}
+
+// gemv_kernel; kNorm: with the RMSNorm fused into it.
+template <bool kNorm>
+void launch_gemv(fi::gemm::Params p, bool int4, hipStream_t st) {
+  using namespace fi::gemm;
+  p.groups_per_split = p.K / kGroup;
+  const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)((p.M + 15) / 16), 1);
+  const size_t lds = kNorm ? (size_t)std::min(p.M, 16) * p.K * sizeof(half_t) : 0;
+  // packed weights: eight waves (two per SIMD hide the dequantization's VALU latency),
+  // except with the fused norm, whose registers allow only one such workgroup per CU
+  if (int4 && !kNorm)
+    hipLaunchKernelGGL((gemv_kernel<true, 3, false, 8>), grid, dim3(512), lds, st, p);
+  else if (int4)
+    hipLaunchKernelGGL((gemv_kernel<true, 6, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
+  else
+    hipLaunchKernelGGL((gemv_kernel<false, 3, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
+}
+
+// gemm_kernel: calls of 17 to 128 rows whose rows lie too far apart for 32-bit offsets, with
+// the K splits (and workspace) of their plan.
+void launch_far_rows(fi::gemm::Params p, bool int4, int splits, void* workspace, hipStream_t st) {
+  using namespace fi::gemm;
+  p.partial = splits > 1 ? (float*)workspace : nullptr;
+  p.groups_per_split = (int)ceil_div(p.K / kGroup, splits);
+  const dim3 grid((unsigned)ceil_div(p.N, kNTile), (unsigned)ceil_div(p.M, 32), (unsigned)splits);
+  if (int4)
+    hipLaunchKernelGGL((gemm_kernel<32, true>), grid, dim3(kThreads), 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_kernel<32, false>), grid, dim3(kThreads), 0, st, p);
+  if (splits == 1) return;
+  const int64_t total = (int64_t)p.M * p.N;
+  const int64_t blocks = std::min<int64_t>((total + 255) / 256, 4096);
+  hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
+                     (const float*)workspace, splits, p.M, p.N, p.out, p.out_stride);
 }
 
 fi::gemm::Params make_params(const void* x, int64_t x_stride, int64_t M, int64_t K,
@@ -1420,18 +1398,13 @@ fi::gemm::Params make_params(const void* x, int64_t x_stride, int64_t M, int64_t
   p.norm_w = nullptr;
   p.eps = 0.f;
   p.tiles = 0;
+  p.tiles_m = 1;
   p.ksplit = 1;
   p.counters = nullptr;
+  p.counter_stride = 0;
+  p.band = 0;
+  p.vec_out = 0;
   return p;
-}
-
-// fp32 partials of a split call: gemm_sk_kernel's [tile][split][MT x 64] blocks, which also
-// hold the two-launch path's [split][M][N] for the same split
-size_t split_bytes(int64_t M, int64_t N, const fi::gemm::Plan& pl) {
-  using fi::gemm::kNTile;
-  if (pl.splits <= 1) return 0;
-  if (pl.sk) return (size_t)pl.splits * ((N + kNTile - 1) / kNTile) * pl.mt * kNTile * sizeof(float);
-  return (size_t)pl.splits * M * N * sizeof(float);
 }
 
 // The norm is fused into the decode kernel for a few rows (each workgroup normalizes them
@@ -1440,35 +1413,39 @@ size_t split_bytes(int64_t M, int64_t N, const fi::gemm::Plan& pl) {
 bool fuse_norm(int64_t M, int64_t K, const fi::gemm::Plan& pl) {
   // up to 4 rows (measured: the fused call is faster than norm pass + GEMM there); the
   // decode kernel keeps its normalized rows in LDS: at most 64 KB of them
-  constexpr int64_t kFuseMaxM = 4;
-  return pl.gemv_rows && M <= kFuseMaxM && std::min<int64_t>(M, 16) * K * 2 <= 65536;
+  return pl.gemv && M <= fi::gemm::kFusedNormM && M * K * 2 <= 65536;
 }
 
 size_t round256(int64_t n) { return (size_t)((n + 255) / 256 * 256); }
 
 size_t norm_rows_bytes(int64_t M, int64_t K) { return round256(M * K * 2); }
 
-// Workspace layout of a call: [normalized rows (separate norm pass)] [dequantized weight
-// (dense path, packed weights)] [fp32 partials (split K)], each 256-byte aligned.
+// Workspace layout of a call: [normalized rows (separate norm pass)] [the unpacked weight
+// (dense plan, packed weights) or the fp32 partials (split K)], each 256-byte aligned.
 struct Layout {
-  size_t rows, weight, split, total;
+  size_t rows, rest, total;
 };
 
 Layout layout(int64_t M, int64_t N, int64_t K, const fi::gemm::Plan& pl, bool int4, bool norm) {
+  using namespace fi::gemm;
   Layout l;
   l.rows = norm && !fuse_norm(M, K, pl) ? norm_rows_bytes(M, K) : 0;
-  l.weight = pl.dense && int4 ? round256(N * K * 2) : 0;
-  l.split = round256((int64_t)split_bytes(M, N, pl));
-  l.total = l.rows + l.weight + l.split;
+  l.rest = pl.gemv ? 0
+           : pl.dense && int4 ? round256(N * K * 2)
+                              : round256(partial_bytes(M, N, pl));
+  l.total = l.rows + l.rest;
   return l;
 }
 
-// What the size queries report: the larger of the packed and the fp16 weight forms.
+// What the size queries report: the larger of the packed and the fp16 weight forms; from
+// kDenseMinM rows, room for the unpacked weight (which also holds any plan's partials).
 size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, bool norm) {
-  using fi::gemm::plan;
+  using namespace fi::gemm;
   const int cus = fi::device_cu_count(nullptr);
-  return std::max(layout(M, N, K, plan(M, N, K, true, cus), true, norm).total,
-                  layout(M, N, K, plan(M, N, K, false, cus), false, norm).total);
+  const Layout packed = layout(M, N, K, plan(M, N, K, true, cus), true, norm);
+  const Layout half = layout(M, N, K, plan(M, N, K, false, cus), false, norm);
+  if (M >= kDenseMinM) return packed.rows + round256(N * K * 2);
+  return std::max(packed.total, half.total);
 }
 
 // One linear-layer call on any path; norm_w non-null applies RMSNorm to X first.
@@ -1480,22 +1457,39 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   using namespace fi::gemm;
   const bool int4 = scales != nullptr;
   const bool norm = norm_w != nullptr;
-  const Plan pl = plan(M, N, K, int4, device_cu_count(st));
-  const Layout l = layout(M, N, K, pl, int4, norm);
-  if (l.total && (!workspace || workspace_bytes < l.total || ((uintptr_t)workspace & 255))) {
-    set_error("%s: workspace of %zu bytes (256-byte aligned) needed, %zu given", fn, l.total,
-              workspace ? workspace_bytes : (size_t)0);
+  const int cus = device_cu_count(st);
+  if (!workspace || ((uintptr_t)workspace & 255)) workspace_bytes = 0;
+  Plan pl = plan(M, N, K, int4, cus);
+  Layout l = layout(M, N, K, pl, int4, norm);
+  // Up to kGemvMaxM rows, and fp16 weights from kDenseMinM rows, a call without room for the
+  // partials runs unsplit; packed weights from kDenseMinM rows always need the size queried.
+  size_t need = l.total;
+  if (M >= kDenseMinM && int4) need = l.rows + round256(N * K * 2);
+  if (workspace_bytes < l.total && (M <= kGemvMaxM || (M >= kDenseMinM && !int4))) {
+    pl = M <= kGemvMaxM ? Plan{true, false, 16, 16, 1} : plan(M, N, K, int4, cus, false);
+    l = layout(M, N, K, pl, int4, norm);
+    need = l.total;
+  }
+  if (workspace_bytes < need) {
+    set_error("%s: workspace of %zu bytes (256-byte aligned) needed, %zu given", fn, need,
+              workspace_bytes);
     return FI_ERR_WORKSPACE;
   }
-  if (!pl.dense && (M + (pl.mt ? pl.mt : 16) - 1) / (pl.mt ? pl.mt : 16) > 65535) {
-    set_error("%s: M %lld too large", fn, (long long)M);
+  // from kDenseMinM rows every plan keeps the limit of the 256-row tiles
+  if (M >= kDenseMinM &&
+      (255 * std::max(norm ? K : x_stride, int4 ? K : w_stride) + K) * 2 >= 0x7ffffff0) {
+    set_error("fi_int4_matmul: 256 rows of X or W span 2^31 bytes or more");
+    return FI_ERR_UNSUPPORTED;
+  }
+  if (!pl.gemv && ceil_div(M, pl.mt) * ceil_div(N, pl.nt) > 0x7ffffff) {
+    set_error("fi_int4_matmul: too many output tiles");
     return FI_ERR_UNSUPPORTED;
   }
   // the decode kernel addresses a workgroup's 16 X rows through one buffer descriptor whose
   // size must stay below the offset its idle lanes use (0x7ffffff0)
   const bool fused = norm && fuse_norm(M, K, pl);
   const int64_t gemv_x_stride = norm && !fused ? K : x_stride;
-  if (pl.gemv_rows && (std::min<int64_t>(M, 16) - 1) * gemv_x_stride * 2 + K * 2 > 0x7ffffff0) {
+  if (M <= kGemvMaxM && (M - 1) * gemv_x_stride * 2 + K * 2 > 0x7ffffff0) {
     set_error("%s: 16 rows of X span 2^31 bytes or more (x_stride %lld)", fn,
               (long long)x_stride);
     return FI_ERR_UNSUPPORTED;
@@ -1505,7 +1499,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   if (fused) {
     p.norm_w = (const half_t*)norm_w;
     p.eps = eps;
-    launch_linear<true>(p, int4, pl, nullptr, st);
+    launch_gemv<true>(p, int4, st);
     return check_launch(fn);
   }
   if (norm) {  // separate norm pass into the workspace
@@ -1516,24 +1510,26 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
     p.x = normed;
     p.x_stride = K;
   }
-  if (pl.dense) {
-    const half_t* w16 = (const half_t*)w;
-    int64_t ldw = w_stride;
-    if (int4) {  // dequantize once into the workspace
-      half_t* deq = (half_t*)(ws + l.rows);
-      const int64_t items = N * (K / 8);
-      const int64_t blocks = std::min<int64_t>((items + 255) / 256, 65536);
-      hipLaunchKernelGGL(dequantize_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
-                         (const uint8_t*)w, w_stride, (const half_t*)scales, s_stride, (int)N,
-                         (int)K, kGroup, deq, K);
-      w16 = deq;
-      ldw = K;
-    }
-    const int rc = check_launch(fn);
-    if (rc != FI_OK) return rc;
-    return f16_gemm(p.x, p.x_stride, w16, ldw, (half_t*)out, out_stride, M, N, K, st);
+  if (pl.gemv) {
+    launch_gemv<false>(p, int4, st);
+    return check_launch(fn);
   }
-  launch_linear<false>(p, int4, pl, ws + l.rows + l.weight, st);
+  if (pl.dense && int4) {  // unpack the weight into the workspace
+    half_t* deq = (half_t*)(ws + l.rows);
+    const int64_t items = N * (K / 8);
+    const int64_t blocks = std::min<int64_t>((items + 255) / 256, 65536);
+    hipLaunchKernelGGL(dequantize_kernel, dim3((unsigned)blocks), dim3(256), 0, st,
+                       (const uint8_t*)w, w_stride, (const half_t*)scales, s_stride, (int)N,
+                       (int)K, kGroup, deq, K);
+    p.w = (const uint8_t*)deq;
+    p.w_stride = K;
+  }
+  if (spans_ok(p, pl))
+    launch_plan(p, pl, ws + l.rows, st);
+  else if (M <= kGemvMaxM)
+    launch_gemv<false>(p, int4, st);
+  else
+    launch_far_rows(p, int4, pl.splits, ws + l.rows, st);
   return check_launch(fn);
 }
 

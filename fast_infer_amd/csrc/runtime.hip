@@ -1,5 +1,5 @@
 // Library-wide host helpers: error strings, version, the CU count per device, the XCD-group
-// check and per-stream slots of the kernels that share partial results within an XCD, and the
+// check and arrival counters of the kernels that share partial results within an XCD, and the
 // MFMA layout self-test.
 #include <stdarg.h>
 
@@ -71,10 +71,22 @@ __global__ __launch_bounds__(64) void xcd_probe_kernel(unsigned* out) {
   }
 }
 
+// Arrival counters, zero at load and left zero by every launch.  Launches on one stream follow
+// one another, so they share the stream's set (one per stream, in order of first use, up to
+// kXcdStreams streams).  A captured launch may be replayed beside any stream: each gets
+// counters of its own, from a part of the array that is only ever handed out once (16 MiB,
+// some 8000 launches; captures past it use the second launch).
+constexpr int kXcdStreams = 16;
+constexpr int kXcdSet = 8 * kXcdCounters;
+constexpr int kXcdCaptured = 4 << 20;
+__device__ __attribute__((aligned(256))) unsigned g_xcd_counters[kXcdStreams * kXcdSet + kXcdCaptured];
+
 struct XcdDevice {
   int state = 0;  // 0: not probed, 1: groups share an XCD, -1: they do not (or no answer)
-  hipStream_t streams[kXcdPurposes][kXcdMaxSlots] = {};
-  int used[kXcdPurposes] = {};
+  unsigned* counters = nullptr;
+  hipStream_t streams[kXcdStreams] = {};
+  int used = 0;      // streams with a set
+  int captured = 0;  // counters handed to captured launches
 };
 
 static std::mutex& xcd_mutex() {
@@ -110,36 +122,59 @@ static bool xcd_probe(hipStream_t st) {
   return ok;
 }
 
-bool xcd_groups_ok(hipStream_t st) {
-  const int dev = stream_device(st);
-  if (dev < 0) return false;
-  std::lock_guard<std::mutex> lock(xcd_mutex());
-  XcdDevice& xd = xcd_device(dev);
+// Whether workgroups whose block ids are congruent modulo 8 run on one XCD of `dev` (one probe
+// launch and a synchronous copy on `st` at the device's first call; false, and not yet probed,
+// while `st` is being captured).
+static bool xcd_ready(XcdDevice& xd, int dev, hipStream_t st) {
   if (xd.state == 0) {
     // the probe synchronizes: not while `st` is being captured or an error is pending
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone ||
-        hipPeekAtLastError() != hipSuccess)
+    if (hipPeekAtLastError() != hipSuccess) return false;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+      (void)hipGetLastError();
       return false;
+    }
+    if (cs != hipStreamCaptureStatusNone) return false;
     int cur = -1;
     if (hipGetDevice(&cur) != hipSuccess) return false;
     if (cur != dev && hipSetDevice(dev) != hipSuccess) return false;
-    xd.state = xcd_probe(st) ? 1 : -1;
+    void* addr = nullptr;
+    const bool ok = hipGetSymbolAddress(&addr, HIP_SYMBOL(g_xcd_counters)) == hipSuccess && addr;
+    xd.counters = (unsigned*)addr;
+    xd.state = ok && xcd_probe(st) ? 1 : -1;
     if (cur != dev) (void)hipSetDevice(cur);
   }
   return xd.state == 1;
 }
 
-int xcd_stream_slot(hipStream_t st, int purpose, int slots) {
+unsigned* xcd_counters(hipStream_t st, int per_group, int* stride) {
+  // hipStreamPerThread names another stream in every thread
+  if (per_group > kXcdCounters || st == hipStreamPerThread) return nullptr;
   const int dev = stream_device(st);
-  if (dev < 0 || purpose < 0 || purpose >= kXcdPurposes || slots > kXcdMaxSlots) return -1;
+  if (dev < 0) return nullptr;
   std::lock_guard<std::mutex> lock(xcd_mutex());
   XcdDevice& xd = xcd_device(dev);
-  for (int i = 0; i < xd.used[purpose]; ++i)
-    if (xd.streams[purpose][i] == st) return i;
-  if (xd.used[purpose] >= slots) return -1;
-  xd.streams[purpose][xd.used[purpose]] = st;
-  return xd.used[purpose]++;
+  if (!xcd_ready(xd, dev, st)) return nullptr;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (st != nullptr && hipStreamIsCapturing(st, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (cs != hipStreamCaptureStatusNone) {
+    *stride = (per_group + 63) / 64 * 64;
+    if (xd.captured + 8 * *stride > kXcdCaptured) return nullptr;
+    unsigned* c = xd.counters + kXcdStreams * kXcdSet + xd.captured;
+    xd.captured += 8 * *stride;
+    return c;
+  }
+  *stride = kXcdCounters;
+  int i = 0;
+  while (i < xd.used && xd.streams[i] != st) ++i;
+  if (i == xd.used) {
+    if (i == kXcdStreams) return nullptr;
+    xd.streams[xd.used++] = st;
+  }
+  return xd.counters + i * kXcdSet;
 }
 
 // One wave: c = mfma16x16x32(a, b, 0) with the lane-major fragments of the header.

@@ -396,3 +396,142 @@ def test_int4_split_k_streams_past_the_counter_sets(hip):
         st.synchronize()
     for out in outs:
         _check(out, x.numpy(), w16)
+
+
+def _check_device(out, x, w16):
+    """_check on the GPU: the float64 product and the bound of oracle.int4.matmul_bound."""
+    x, w = x.double(), w16.double()
+    exact = x @ w.t()
+    steps = x.shape[1] / 32 + 16
+    bound = exact.abs() * 2.0 ** -11 + (x.abs() @ w.t().abs()) * steps * 2.0 ** -24 + 2.0 ** -24
+    over = ((out.double() - exact).abs() - bound).max().item()
+    assert over <= 0, over
+
+
+# Both tiled kernels (mid_gemm_kernel and, for fp16 weights, tile_gemm_kernel) over the rows at
+# which their tiles change: one row more or less than a tile, row counts that leave a nearly
+# empty last tile, column counts that do the same (200, 130 with scalar stores) or fill the
+# chip, K of one and of many groups, with and without K splits.
+@pytest.mark.parametrize("M", [5, 16, 17, 33, 65, 128, 129, 257, 509, 700, 1100])
+@pytest.mark.parametrize("N,K", [(5120, 3072), (3072, 8192), (200, 1280), (130, 128), (2049, 640)])
+def test_tiled_kernels(hip, M, N, K):
+    banner(f"tiled linear kernels M={M} N={N} K={K}")
+    from fast_infer_amd import _lib, dequantize_int4
+
+    lib = _lib.load()
+    packed, scales = _packed(M + N + K, N, K)
+    w16 = dequantize_int4(packed, scales)
+    g = torch.Generator(device=DEV).manual_seed(M * 3 + N)
+    big = torch.full((M + 300, K + 16), float("nan"), device=DEV).half()
+    big[:M, 8:8 + K] = torch.randn(M, K, device=DEV, generator=g).half()
+    x = big[:M, 8:8 + K]  # NaN around the rows: nothing past them may be used
+    ws = torch.empty(lib.fi_int4_matmul_workspace_size(M, N, K), dtype=torch.uint8, device=DEV)
+    st = _lib.stream_handle(torch.device(DEV))
+    for form in ("packed", "fp16"):
+        outs = []
+        for _ in range(2):  # twice: the counters are back at zero after a call
+            ws.fill_(255)
+            buf = torch.full((M * N + 16,), float("nan"), device=DEV).half()
+            w = (packed.data_ptr(), K // 2, scales.data_ptr(), K // 128) if form == "packed" else \
+                (w16.data_ptr(), K, None, 0)
+            rc = lib.fi_int4_matmul(x.data_ptr(), x.stride(0), M, K, *w, N, 128, buf.data_ptr(), N,
+                                    ws.data_ptr() if ws.numel() else None, ws.numel(), st)
+            _lib.check(rc, "fi_int4_matmul")
+            assert torch.isnan(buf[M * N:]).all()
+            outs.append(buf[:M * N].view(M, N))
+        assert torch.equal(*outs)
+        _check_device(outs[0], x, w16)
+
+
+def test_tiled_kernels_two_launch_path(hip):
+    """A stream without counters (hipStreamPerThread is never given any) adds the K splits in a
+    second launch: the same bits as the in-launch sum, both weight forms."""
+    banner("tiled linear kernels: second launch")
+    from fast_infer_amd import _lib, dequantize_int4
+
+    lib = _lib.load()
+    per_thread = 2  # hipStreamPerThread
+    for M, N, K in ((16, 5120, 3072), (40, 3072, 3072), (100, 3072, 8192), (500, 3072, 8192)):
+        packed, scales = _packed(M, N, K)
+        w16 = dequantize_int4(packed, scales)
+        x = torch.randn(M, K, device=DEV).half()
+        ws = torch.empty(lib.fi_int4_matmul_workspace_size(M, N, K), dtype=torch.uint8, device=DEV)
+        for w in ((packed.data_ptr(), K // 2, scales.data_ptr(), K // 128), (w16.data_ptr(), K, None, 0)):
+            outs = []
+            for stream in (_lib.stream_handle(torch.device(DEV)), per_thread):
+                out = torch.empty(M, N, dtype=torch.float16, device=DEV)
+                torch.cuda.synchronize()
+                rc = lib.fi_int4_matmul(x.data_ptr(), K, M, K, *w, N, 128, out.data_ptr(), N,
+                                        ws.data_ptr(), ws.numel(), stream)
+                _lib.check(rc, "fi_int4_matmul")
+                torch.cuda.synchronize()
+                outs.append(out)
+            assert torch.equal(*outs), (M, N, K)
+
+
+def test_captured_split_beside_eager_calls(hip):
+    """A captured split-K call replayed on one stream while eager calls run on the stream it was
+    captured on (each with its own workspace): both keep their results."""
+    banner("captured split-K call beside eager calls on its capture stream")
+    from fast_infer_amd import _lib, int4_matmul
+
+    M, N, K = 100, 3072, 8192
+    lib = _lib.load()
+    w = _packed(61, N, K)
+    x = torch.randn(M, K, device=DEV).half()
+    ref = int4_matmul(x, w)
+    need = lib.fi_int4_matmul_workspace_size(M, N, K)
+    ws = [torch.empty(need, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    torch.cuda.synchronize()
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = int4_matmul(x, w, workspace=ws[0])
+    torch.cuda.synchronize()
+    for _ in range(5):
+        eager = []
+        for _ in range(8):
+            with torch.cuda.stream(other):
+                graph.replay()
+            with torch.cuda.stream(side):
+                eager.append(int4_matmul(x, w, workspace=ws[1]))
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and all(torch.equal(e, ref) for e in eager)
+
+
+def test_calls_without_room_for_partials(hip):
+    """Calls that never needed a workspace keep running without one: up to 16 rows, and fp16
+    weights from 129 rows; packed weights from 129 rows are refused as before."""
+    banner("linear calls without a workspace")
+    from fast_infer_amd import _lib, dequantize_int4
+
+    lib = _lib.load()
+    N, K = 3072, 8192
+    packed, scales = _packed(71, N, K)
+    w16 = dequantize_int4(packed, scales)
+    p_args, h_args = (packed.data_ptr(), K // 2, scales.data_ptr(), K // 128), (w16.data_ptr(), K, None, 0)
+    st = _lib.stream_handle(torch.device(DEV))
+    for M, w, ok in ((12, p_args, True), (16, h_args, True), (509, h_args, True), (509, p_args, False)):
+        x = torch.randn(M, K, device=DEV).half()
+        out = torch.empty(M, N, dtype=torch.float16, device=DEV)
+        rc = lib.fi_int4_matmul(x.data_ptr(), K, M, K, *w, N, 128, out.data_ptr(), N, None, 0, st)
+        assert rc == (_lib.FI_OK if ok else _lib.FI_ERR_WORKSPACE)
+        if ok:
+            _check_device(out, x, w16)
+
+
+@pytest.mark.parametrize("form", ["packed", "fp16"])
+def test_rows_too_far_apart_for_buffer_offsets(hip, form):
+    """20 rows of X spread over more than 2 GiB (gemm_kernel), K split and not."""
+    banner(f"int4_matmul, rows 128 MiB apart, {form} weights")
+    from fast_infer_amd import dequantize_int4, int4_matmul
+
+    stride = 1 << 26
+    store = torch.empty(19 * stride + 8192, dtype=torch.float16, device=DEV)
+    for N, K in ((3072, 8192), (130, 256)):
+        w = _packed(N, N, K)
+        w16 = dequantize_int4(*w)
+        x = store.as_strided((20, K), (stride, 1))
+        x.copy_(torch.randn(20, K, device=DEV))
+        out = int4_matmul(x, w if form == "packed" else w16)
+        _check_device(out, x.contiguous(), w16)
