@@ -22,6 +22,7 @@
 //     block (one descriptor per tile); any other size gives each row its own block, through
 //     per-lane offsets into a descriptor over the whole pool (pools under 4 GiB) or through
 //     one descriptor per row.
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -477,27 +478,40 @@ __global__ __launch_bounds__(kHeadDim) void merge_kernel(Params p) {
     p.o[(int64_t)b * p.o_sb + (int64_t)h * p.o_sh + d] = (half_t)(L > 0.f ? O / L : 0.f);
 }
 
-// Partition size (tokens, a multiple of kWgTokens) for a call: about kTargetWgs
-// workgroups in total if every row had the maximum length, 128..384 tokens each (short
-// partitions keep every CU streaming at small batch; longer ones amortise the
-// workgroup's table and merge work; the merge reads ~0.5 KiB per partition and head).
-// A context of at most 512 tokens is one partition with no merge.
-static int tokens_per_split(int64_t batch, int64_t wg_per_row, int64_t num_tokens) {
-  constexpr int64_t target = 2048;
+// Partition size (tokens, a multiple of kWgTokens) for a call of `units` = rows x head groups.
+// 256 CUs hold two workgroups each, and a second round of them, however small, costs a whole
+// workgroup's time (about 4 us of latency before it streams): the smallest partitions whose
+// workgroups fit one round, else the cap.  Workgroups are counted with every row at the maximum
+// length; with per-row lengths about a third of them is taken to be empty.  64-token partitions
+// pay only while half the slots stay free, and the merge reads 0.5 KiB per partition and head.
+// Measured against the smallest partition of at least 128 tokens that gave 2048 workgroups:
+// 1 row of 1024 tokens 9.5 -> 9.0 us (64 tokens, was 128), 4 of 4096 23.0 -> 17.4 (256, was
+// 128), 7 of 100..3001 18.1 -> 15.2 (256, was 128), 16 of 1024 21.7 -> 18.1 (256, was 128), 64 of
+// 4096 184 -> 171 (512, was 384); 32 of 512..4096 stays at 384 (50.6 us; 51.6 with 320, 52.4
+// with 512).
+// Up to kDirectTokens a call is one partition with no merge, except that the longer ones of few
+// units are cut into 64-token partitions (1 row of 500: 8.6 us against 10.4, 8 of 512 10.4
+// against 11.5, but 32 of 500 24.0 against 13.6).
+constexpr int64_t kDirectTokens = 512;
+constexpr int64_t kUnsplitTokens = 320;  // at most this: always one partition
+constexpr int64_t kRoundWgs = 512;       // workgroups of one round
+constexpr int64_t kRoundWgsLens = 704;   // the same with per-row lengths
+static int tokens_per_split(int64_t units, int64_t num_tokens, bool lens) {
+  auto wgs = [&](int64_t tps) { return units * ((num_tokens + tps - 1) / tps); };
+  const int64_t most = lens ? kRoundWgsLens : kRoundWgs;
   int64_t tps;
-  if (num_tokens <= 512) {
-    tps = num_tokens;
+  if (num_tokens <= kDirectTokens) {
+    tps = num_tokens > kUnsplitTokens && wgs(64) <= kRoundWgs ? 64 : num_tokens;
+  } else if (wgs(64) <= kRoundWgs / 2) {
+    tps = 64;
   } else {
-    const int64_t per_row = batch * wg_per_row;
-    int64_t want = (target + per_row - 1) / per_row;
-    if (want < 1) want = 1;
-    tps = (num_tokens + want - 1) / want;
-    if (tps > 384) tps = 384;
+    tps = 128;
+    while (tps < 512 && wgs(tps) > most) tps += tps < 384 ? 64 : 128;
+    if (wgs(tps) > most) tps = lens ? 384 : 512;
   }
   const int64_t min_tps = (num_tokens + kMaxSplits - 1) / kMaxSplits;
   if (tps < min_tps) tps = min_tps;
   tps = (tps + kWgTokens - 1) / kWgTokens * kWgTokens;
-  if (tps < 128) tps = 128;
   if (tps > kMaxSplitTokens) tps = kMaxSplitTokens;
   return (int)tps;
 }
@@ -520,8 +534,13 @@ extern "C" size_t fi_paged_attention_workspace_size(int64_t batch, int64_t num_q
     return 0;
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t wg_per_row = num_kv_heads * (group / heads_per_wg(group));
-  const int64_t tps = tokens_per_split(batch, wg_per_row, max_num_tokens);
-  const int64_t splits = (max_num_tokens + tps - 1) / tps;
+  if (max_num_tokens <= kUnsplitTokens) return 0;
+  // enough for any num_tokens up to this one: fewer tokens may be cut into more partitions
+  const int64_t units = batch * wg_per_row;
+  const int64_t tps = std::min(tokens_per_split(units, max_num_tokens, false),
+                               tokens_per_split(units, max_num_tokens, true));
+  const int64_t splits = std::max((max_num_tokens + tps - 1) / tps,
+                                  std::min((max_num_tokens + 63) / 64, kRoundWgsLens / units));
   if (splits <= 1) return 0;
   return (size_t)(batch * num_q_heads * splits * (fi::kHeadDim + 2) * sizeof(float));
 }
@@ -595,7 +614,13 @@ int paged_fwd(const char* fn, const void* q, int64_t q_sb, int64_t q_sh, const v
   p.heads_per_wg = heads_per_wg(group);
   p.scale_log2 = sm_scale * kLog2e;
   const int64_t wg_per_row = num_kv_heads * (group / p.heads_per_wg);
-  p.tokens_per_split = tokens_per_split(batch, wg_per_row, num_tokens > 0 ? num_tokens : 1);
+  const size_t need =
+      fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads, num_tokens, head_dim);
+  p.tokens_per_split = tokens_per_split(batch * wg_per_row, num_tokens > 0 ? num_tokens : 1,
+                                        context_lens != nullptr);
+  // calls of up to kDirectTokens tokens run without a workspace too, as one partition
+  if (num_tokens <= kDirectTokens && (!workspace || workspace_bytes < need))
+    p.tokens_per_split = (int)kDirectTokens;
   int64_t splits = (num_tokens + p.tokens_per_split - 1) / p.tokens_per_split;
   if (splits < 1) splits = 1;
   p.max_splits = (int)splits;
@@ -617,8 +642,6 @@ int paged_fwd(const char* fn, const void* q, int64_t q_sb, int64_t q_sh, const v
   p.part_o = nullptr;
   p.part_ml = nullptr;
   if (!p.direct) {
-    const size_t need =
-        fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads, num_tokens, head_dim);
     if (!workspace || workspace_bytes < need) {
       set_error("%s: workspace of %zu bytes needed, %zu given", fn, need,
                 workspace ? workspace_bytes : (size_t)0);
@@ -710,7 +733,8 @@ extern "C" int fi_paged_attention_fwd_noalloc(const void* q, int64_t q_sb, int64
   using namespace fi;
   static const char* fn = "fi_paged_attention_fwd_noalloc";
   clear_error();
-  const size_t need = batch > 0 && num_tokens > 0
+  // up to kDirectTokens tokens: one partition, which leaves the shared scratch alone
+  const size_t need = batch > 0 && num_tokens > decode::kDirectTokens
                           ? fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads,
                                                               num_tokens, head_dim)
                           : 0;

@@ -237,3 +237,23 @@ def test_workspace_size(lib):
 
     assert rc == _lib.FI_ERR_WORKSPACE
     assert ctypes.c_size_t(n).value == n
+
+
+def test_paged_workspace_size_covers_smaller_calls(lib):
+    """A workspace sized for a bound serves any smaller num_tokens, calls of up to 320 tokens
+    need none, and no call outgrows the allocation-free entry point's scratch that fitted it with
+    partitions of at least 128 tokens in at most 2048 workgroups."""
+    size = lib.fi_paged_attention_workspace_size
+    scratch = 32 << 20
+    for kv, group in ((8, 3), (1, 8), (32, 1), (4, 32)):
+        per_row = kv * (group // (16 if group == 32 else group))
+        for batch in (1, 2, 3, 7, 12, 33, 64, 200, 1000):
+            last = 0
+            for n in list(range(1, 1200, 13)) + list(range(1200, 70000, 997)):
+                need = size(batch, kv * group, kv, n, 128)
+                assert need >= last and (n > 320 or need == 0)
+                last = need
+                want = -(-2048 // (batch * per_row))
+                tps = max(128, -(-max(min(384, -(-n // want)), -(-n // 1024)) // 64) * 64)
+                before = batch * kv * group * -(-n // tps) * 130 * 4
+                assert n <= 512 or before > scratch or need <= scratch, (batch, kv, group, n)

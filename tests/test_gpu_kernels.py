@@ -482,3 +482,61 @@ def test_kvcache_device_table_keeps_in_place_writes(hip):
     assert cache.host_block_table()[1, 5] == -1   # not seen by the allocator
     cache.reset()
     assert bool((cache.block_table == -1).all())
+
+
+# Decode partitions: the sizes at which the partition size changes (64 to 512 tokens, one
+# partition, 64-token partitions below 512 tokens), each with one shared length and with ragged
+# rows whose lengths end at, before and after partition and tile edges (and an empty row).
+@pytest.mark.parametrize("batch,tokens", [(1, 320), (1, 321), (2, 512), (40, 512), (1, 513), (1, 2048),
+                                          (2, 2049), (3, 1536), (4, 2100), (5, 4096), (9, 2500),
+                                          (12, 4096), (70, 600)])
+def test_paged_decode_partition_sizes(hip, batch, tokens):
+    banner(f"paged decode partitions batch {batch} tokens {tokens}")
+    from fast_infer_amd import paged_attention
+
+    hq, hkv, d, bs = 24, 8, 128, 16
+    blocks = -(-tokens // bs)
+    g = torch.Generator(device="cuda:0").manual_seed(batch + tokens)
+    kc, vc = (torch.randn(batch * blocks, bs, hkv, d, device="cuda:0", generator=g).half()
+              for _ in range(2))
+    q = torch.randn(batch, hq, d, device="cuda:0", generator=g).half()
+    table = torch.randperm(batch * blocks, device="cuda:0", generator=g).int().view(batch, blocks)
+    edges = [0, 1, 63, 64, 65, 128, 191, 193, 256, 321, 384, 512, 513, tokens - 1, tokens]
+    lens = [min(edges[-1 - i % len(edges)], tokens) for i in range(batch)]
+    for cl in (None, torch.tensor(lens, dtype=torch.int32, device="cuda:0")):
+        out = paged_attention(q, kc, vc, table, bs, tokens, context_lens=cl)
+        for b in sorted({0, batch - 1, *range(min(batch, len(edges)))}):
+            n = tokens if cl is None else lens[b]
+            if n == 0:
+                assert not out[b].any()
+                continue
+            k, v = (c[table[b].long()].flatten(0, 1)[:n].float() for c in (kc, vc))
+            s = torch.einsum("kgd,nkd->kgn", q[b].float().view(hkv, 3, d), k) * d ** -0.5
+            ref = torch.einsum("kgn,nkd->kgd", s.softmax(-1), v).reshape(hq, d)
+            assert float((out[b].float() - ref).abs().max()) <= ATOL, (b, n)
+
+
+def test_paged_decode_short_calls_without_workspace(hip):
+    """Up to 512 tokens a C call without a workspace runs as one partition: within the tolerance
+    of the call with one, which cuts this length into partitions."""
+    banner("paged decode 500 tokens with and without workspace")
+    from fast_infer_amd import _lib
+
+    lib = _lib.load()
+    b, n, hq, hkv, d, bs = 2, 500, 24, 8, 128, 64
+    kc, vc = (torch.randn(16, bs, hkv, d, device="cuda:0").half() for _ in range(2))
+    q = torch.randn(b, hq, d, device="cuda:0").half()
+    table = torch.randperm(16, device="cuda:0").int().view(b, 8)
+    need = lib.fi_paged_attention_workspace_size(b, hq, hkv, n, d)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    outs = []
+    for ptr, nbytes in ((ws.data_ptr(), need), (None, 0), (ws.data_ptr(), need - 4)):
+        out = torch.empty_like(q)
+        rc = lib.fi_paged_attention_fwd(
+            q.data_ptr(), hq * d, d, kc.data_ptr(), vc.data_ptr(), 16, bs, hkv, table.data_ptr(), 8, 8,
+            None, n, out.data_ptr(), hq * d, d, b, hq, d, d ** -0.5, ptr, nbytes,
+            _lib.stream_handle(q.device))
+        _lib.check(rc, "fi_paged_attention_fwd")
+        outs.append(out.float())
+    assert float((outs[0] - outs[1]).abs().max()) <= ATOL and torch.equal(outs[1], outs[2])
