@@ -62,10 +62,38 @@ __device__ __forceinline__ half_t rot1(half_t x, half_t c, half_t y, half_t s) {
   return (half_t)((float)a + (float)b);
 }
 
+template <bool kNt>
+__device__ __forceinline__ u32x4 load16(const half_t* p) {
+  return kNt ? __builtin_nontemporal_load((const u32x4*)p) : *(const u32x4*)p;
+}
+template <bool kNt>
+__device__ __forceinline__ void store16(half_t* p, u32x4 v) {
+  if (kNt)
+    __builtin_nontemporal_store(v, (u32x4*)p);
+  else
+    *(u32x4*)p = v;
+}
+
+// Cache policy, by the size of the call.  Bound by memory; 24/8 heads, D 128, pool written:
+//   kKeep     small calls: default loads and stores;
+//   kStream   from kStreamItems: non-temporal stores, which leave the L2 to the rows still to be
+//             read: 1024 tokens 6.7 -> 5.6 us, 2 x 4096 (no k out) 32.0 -> 28.2; a projection,
+//             this call and attention in a row take the same time or less (4096 tokens 313 ->
+//             305 us);
+//   kStreamIn from kStreamInBytes of q, k and v, more than the last-level cache holds beside
+//             the outputs: non-temporal loads too, and the pools written back by default:
+//             4 x 4096 68.5 -> 58.6 us (6.3 TB/s; kStream 63.1).  Below, loads find the
+//             projection's output in the cache: 4096 tokens 17.0 us, 19.3 with them.
+enum Policy { kKeep, kStream, kStreamIn };
+constexpr int64_t kStreamItems = 1 << 17;  // about 410 tokens
+constexpr int64_t kStreamInBytes = 144 << 20;
+
 // Index is uint32_t whenever the work items fit (32-bit division by the runtime head and
 // token counts is a short sequence; 64-bit division is a long software routine).
-template <typename Index>
+template <typename Index, int kPolicy>
 __global__ __launch_bounds__(256) void rope_store_kernel(Params p) {
+  constexpr bool kNtIn = kPolicy == kStreamIn, kNtOut = kPolicy != kKeep;
+  constexpr bool kNtPool = kPolicy == kStream;
   const Index heads = (Index)p.heads;
   const Index items = (Index)p.items;
   for (Index it = (Index)blockIdx.x * blockDim.x + threadIdx.x; it < items;
@@ -97,8 +125,8 @@ __global__ __launch_bounds__(256) void rope_store_kernel(Params p) {
       if (dst < 0) continue;
       const int hk = hh - p.num_q_heads - p.num_kv_heads;
       const half_t* src = p.v + (int64_t)b * p.v_sb + (int64_t)t * p.v_st + (int64_t)hk * p.v_sh;
-      *(u32x4*)(p.v_cache + dst + 8 * c) = *(const u32x4*)(src + 8 * c);
-      *(u32x4*)(p.v_cache + dst + p.half + 8 * c) = *(const u32x4*)(src + p.half + 8 * c);
+      store16<kNtPool>(p.v_cache + dst + 8 * c, load16<kNtIn>(src + 8 * c));
+      store16<kNtPool>(p.v_cache + dst + p.half + 8 * c, load16<kNtIn>(src + p.half + 8 * c));
       continue;
     }
 
@@ -106,8 +134,8 @@ __global__ __launch_bounds__(256) void rope_store_kernel(Params p) {
     const half_t* src = is_q ? p.q + (int64_t)b * p.q_sb + (int64_t)t * p.q_st + (int64_t)hh * p.q_sh
                              : p.k + (int64_t)b * p.k_sb + (int64_t)t * p.k_st +
                                    (int64_t)(hh - p.num_q_heads) * p.k_sh;
-    const half8 lo = as_half8(*(const u32x4*)(src + 8 * c));        // x[8c .. 8c+7]
-    const half8 hi = as_half8(*(const u32x4*)(src + p.half + 8 * c));  // x[D/2+8c .. +7]
+    const half8 lo = as_half8(load16<kNtIn>(src + 8 * c));           // x[8c .. 8c+7]
+    const half8 hi = as_half8(load16<kNtIn>(src + p.half + 8 * c));  // x[D/2+8c .. +7]
     const half_t* cr = p.cos_t + (int64_t)pos * p.head_dim;
     const half_t* sr = p.sin_t + (int64_t)pos * p.head_dim;
     const half8 clo = as_half8(*(const u32x4*)(cr + 8 * c));
@@ -122,18 +150,18 @@ __global__ __launch_bounds__(256) void rope_store_kernel(Params p) {
     }
     if (is_q) {
       half_t* o = p.q_out + (int64_t)b * p.qo_sb + (int64_t)t * p.qo_st + (int64_t)hh * p.qo_sh;
-      *(u32x4*)(o + 8 * c) = as_u32x4(olo);
-      *(u32x4*)(o + p.half + 8 * c) = as_u32x4(ohi);
+      store16<kNtOut>(o + 8 * c, as_u32x4(olo));
+      store16<kNtOut>(o + p.half + 8 * c, as_u32x4(ohi));
     } else {
       if (p.k_out) {
         half_t* o = p.k_out + (int64_t)b * p.ko_sb + (int64_t)t * p.ko_st +
                     (int64_t)(hh - p.num_q_heads) * p.ko_sh;
-        *(u32x4*)(o + 8 * c) = as_u32x4(olo);
-        *(u32x4*)(o + p.half + 8 * c) = as_u32x4(ohi);
+        store16<kNtOut>(o + 8 * c, as_u32x4(olo));
+        store16<kNtOut>(o + p.half + 8 * c, as_u32x4(ohi));
       }
       if (dst >= 0) {
-        *(u32x4*)(p.k_cache + dst + 8 * c) = as_u32x4(olo);
-        *(u32x4*)(p.k_cache + dst + p.half + 8 * c) = as_u32x4(ohi);
+        store16<kNtPool>(p.k_cache + dst + 8 * c, as_u32x4(olo));
+        store16<kNtPool>(p.k_cache + dst + p.half + 8 * c, as_u32x4(ohi));
       }
     }
   }
@@ -230,11 +258,16 @@ extern "C" int fi_rope_store_kv(const void* q, int64_t q_sb, int64_t q_st, int64
   if (p.items == 0) return FI_OK;
   const int64_t blocks = (p.items + 255) / 256;
   const unsigned grid = (unsigned)(blocks < 65536 ? blocks : 65536);
-  if (p.items < (1ll << 31))
-    hipLaunchKernelGGL(rope_store_kernel<uint32_t>, dim3(grid), dim3(256), 0,
-                       (hipStream_t)stream, p);
+  const int64_t in_bytes = batch * num_tokens * p.heads * head_dim * 2;
+  const hipStream_t st = (hipStream_t)stream;
+  const dim3 block(256);
+  if (p.items >= (1ll << 31))
+    hipLaunchKernelGGL((rope_store_kernel<int64_t, kStreamIn>), dim3(grid), block, 0, st, p);
+  else if (in_bytes >= kStreamInBytes)
+    hipLaunchKernelGGL((rope_store_kernel<uint32_t, kStreamIn>), dim3(grid), block, 0, st, p);
+  else if (p.items >= kStreamItems)
+    hipLaunchKernelGGL((rope_store_kernel<uint32_t, kStream>), dim3(grid), block, 0, st, p);
   else
-    hipLaunchKernelGGL(rope_store_kernel<int64_t>, dim3(grid), dim3(256), 0,
-                       (hipStream_t)stream, p);
+    hipLaunchKernelGGL((rope_store_kernel<uint32_t, kKeep>), dim3(grid), block, 0, st, p);
   return check_launch("fi_rope_store_kv");
 }

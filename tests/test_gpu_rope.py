@@ -190,3 +190,37 @@ def test_rope_store_kv_batch4_seq4096_full_size(hip):
                                cos[t0:t0 + 64].cpu().numpy(), sin[t0:t0 + 64].cpu().numpy())
         assert np.array_equal(_bits(qr[b:b + 1, t0:t0 + 64]), _bits(eq))
         assert np.array_equal(_bits(kr[b:b + 1, t0:t0 + 64]), _bits(ek))
+
+
+@pytest.mark.parametrize("B,T,keep_k", [(1, 409, True), (1, 410, True), (3, 333, False), (4, 3670, True),
+                                        (4, 3700, False)])
+def test_rope_store_kv_cache_policies(hip, B, T, keep_k):
+    """The three cache policies, at sizes on both sides of each switch (24/8 heads with a pool),
+    rows starting apart, a hole in the table: the same bits as eager torch ops."""
+    banner(f"rope_store_kv cache policies B={B} T={T} keep_k={keep_k}")
+    from fast_infer_amd import rope_store_kv
+
+    bs, rows = 16, 4096
+    q, k, v = _qkv(B, T, 24, 8, seed=B + T)
+    cos, sin = _tables(rows)
+    width = -(-(T + 100) // bs)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    table = torch.randperm(B * width, device=DEV, generator=g).int().view(B, width)
+    table[0, 3] = -1
+    starts = [(37 * b) % 100 for b in range(B)]
+    kp = torch.full((B * width, bs, 8, 128), 7.0, dtype=torch.float16, device=DEV)
+    vp = torch.full_like(kp, -7.0)
+    ekp, evp = kp.clone(), vp.clone()
+    qr, kr = rope_store_kv(q, k, v, cos, sin, 0, kp, vp, table, return_k=keep_k,
+                           start_positions=torch.tensor(starts, dtype=torch.int32, device=DEV))
+    assert (kr is None) == (not keep_k)
+    for b, st in enumerate(starts):
+        pos = torch.arange(st, st + T, device=DEV)
+        ek = _torch_rope(k[b], cos[pos], sin[pos])
+        assert torch.equal(qr[b], _torch_rope(q[b], cos[pos], sin[pos]))
+        assert kr is None or torch.equal(kr[b], ek)
+        blocks = table[b].long()[pos // bs]
+        ok = blocks >= 0
+        ekp[blocks[ok], pos[ok] % bs] = ek[ok]
+        evp[blocks[ok], pos[ok] % bs] = v[b][ok]
+    assert torch.equal(kp, ekp) and torch.equal(vp, evp)
