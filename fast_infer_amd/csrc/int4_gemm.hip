@@ -9,7 +9,7 @@
 //
 // C[m, n] = fp16( sum_k X[m, k] * W[n, k] ), fp32 accumulation (matmul.py:14-132,
 // :135-186).  By the rows M of X and the measured costs in plan():
-//   up to 4 rows, and up to 16 where it is the fastest:
+//   up to 16 rows where it is the fastest, and up to 4 with a fused norm:
 //                     gemv_kernel: one workgroup per 16 output columns, K split over its waves;
 //   packed weights:   mid_gemm_kernel, which unpacks them in registers, and for many row tiles
 //                     one unpacking into the workspace followed by tile_gemm_kernel;
@@ -31,6 +31,7 @@ constexpr int kThreads = 256;
 constexpr int kNTile = 64;
 constexpr int kGroup = 128;     // K per scale group and per pipeline step
 constexpr int kLdsRow = 136;    // halves per staged X row (128 + 8 pad)
+constexpr int kFusedNormM = 4;  // rows up to which gemv_kernel takes the RMSNorm in
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
@@ -880,14 +881,27 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(Params p) {
     store_half4(p, sum, m, tn * 32 * BN + (wave & 1) * 16 * BN + 16 * (b / BM) + 4 * (lane >> 4));
 }
 
+// A barrier for data passed through LDS only: __syncthreads would also wait for the weight loads
+// in flight.
+__device__ __forceinline__ void lds_barrier() {
+  wait_lgkmcnt0();
+  asm volatile("s_barrier" ::: "memory");
+}
+
 // Decode-sized calls (16 rows of X per blockIdx.y): one workgroup per 16 output columns.
 // The kW waves take interleaved groups (g = wave, wave + kW, ...), so K is split inside
 // the workgroup and no partials leave it.  Each lane issues the loads of kChunk groups at
 // once (16 weight bytes, the scale, and 64 bytes of its X row per group) before any math,
 // so one memory latency covers the chunk; the kW waves' sums are added through LDS in
 // a fixed order.
-template <bool kInt4, int kChunk, bool kNorm, int kW>
-__global__ __launch_bounds__(64 * kW, kNorm ? 1 : 2) void gemv_kernel(Params p) {
+//
+// kNormRows > 0: the RMSNorm of up to that many rows fused, shared out over the workgroup (packed
+// weights, 1 or 2 rows) or a row per wave.  5120 columns, K 3072, packed, cold weights: 1 row
+// 8.0 us, 8.8 a row per wave; 16384 columns 12.2 against 15.2 and, 2 rows, 13.6 against 15.1.  4
+// rows shared out take 10.9 against 9.1, and fp16 weights, bound by their stream, lose too.
+template <bool kInt4, int kChunk, int kNormRows, int kW>
+__global__ __launch_bounds__(64 * kW, kNormRows == kFusedNormM ? 1 : 2) void gemv_kernel(Params p) {
+  constexpr bool kNorm = kNormRows > 0;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int row = lane & 15;
@@ -944,7 +958,65 @@ __global__ __launch_bounds__(64 * kW, kNorm ? 1 : 2) void gemv_kernel(Params p) 
   // the first chunk's weights are in flight while the rows are normalized; the scheduling
   // barriers keep every load of a chunk ahead of its math (the scheduler would otherwise
   // start the math after the first few loads and issue the rest one latency later)
-  if constexpr (kNorm) {
+  if constexpr (kNorm && kNormRows < kFusedNormM) {
+    // Every thread takes a few elements of every row: a row's sum of squares is the sum of the
+    // waves' parts (through LDS), and no wave holds a whole row in registers, so two
+    // eight-wave workgroups fit a CU.  x and the norm weight are loaded before the first
+    // chunk's weights: loads complete in issue order, so the norm waits for its own data only
+    // and runs while the weights stream in.  Rows longer than kLongRow are normalized after
+    // the weights' loads, a wave per row.
+    constexpr int kLongRow = 8192, kSpan = kW * 512, kParts = kLongRow / kSpan;
+    if (p.K <= kLongRow) {  // uniform
+      __shared__ float part[kNormRows][kW];
+      u32x4 xr_v[kNormRows][kParts], nw_v[kParts];
+      // elements past K and rows past M read zeros through the buffer bounds
+      const __amdgpu_buffer_rsrc_t nw_rsrc =
+          __builtin_amdgcn_make_buffer_rsrc((void*)p.norm_w, (short)0, p.K * 2, 0x00020000);
+#pragma unroll
+      for (int i = 0; i < kParts; ++i) {
+        const int k2 = (threadIdx.x * 8 + i * kSpan) * 2;
+#pragma unroll
+        for (int r = 0; r < kNormRows; ++r)
+          xr_v[r][i] = __builtin_bit_cast(
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                         xr_rsrc, k2 < 2 * p.K && r < rows_n ? r * (int)(p.x_stride * 2) + k2 : 0x7ffffff0,
+                         0, 0));
+        nw_v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(nw_rsrc, k2, 0, 0));
+      }
+      load_chunk(wave);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < kNormRows; ++r) {
+        float sq = 0.f;
+#pragma unroll
+        for (int i = 0; i < kParts; ++i) sq += sum_sq8(xr_v[r][i]);
+        sq = wave_sum(sq);
+        if (lane == 0) part[r][wave] = sq;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int r = 0; r < kNormRows; ++r) {
+        if (r < rows_n) {  // uniform
+          float sq = 0.f;
+#pragma unroll
+          for (int w = 0; w < kW; ++w) sq += part[r][w];
+          const float rs = rsqrtf(sq / (float)p.K + p.eps);
+#pragma unroll
+          for (int i = 0; i < kParts; ++i) {
+            const int k = threadIdx.x * 8 + i * kSpan;
+            if (k < p.K) *(u32x4*)(xn + r * p.K + k) = norm8(xr_v[r][i], rs, nw_v[i]);
+          }
+        }
+      }
+    } else {
+      load_chunk(wave);
+      __builtin_amdgcn_sched_barrier(0);
+      for (int r = wave; r < rows_n; r += kW)
+        norm_row_to(p.x + (int64_t)(blockIdx.y * 16 + r) * p.x_stride, p.norm_w, p.K, p.eps,
+                    xn + r * p.K, lane);
+    }
+    lds_barrier();
+  } else if constexpr (kNorm) {
     // Wave r normalizes row r.  Its x row and the norm weight are loaded before the first
     // chunk's weights: loads complete in issue order, so the norm waits for its own data
     // only and runs while the weights stream in.  Rows longer than kRowChunks * 512, and rows
@@ -1126,7 +1198,6 @@ struct Plan {
 // apart, from here 256 rows of X (and of an fp16 W) have to span less than 2 GiB.
 constexpr int kDenseMinM = 129;
 constexpr int kGemvMaxM = 16;    // rows of one gemv_kernel workgroup
-constexpr int kFusedNormM = 4;   // gemv_kernel whatever its cost below (the norm is fused there)
 constexpr int kMaxSplits = 10;
 constexpr int kMaxSplitTiles = 8 * kXcdCounters;  // tiles of a split call
 
@@ -1176,11 +1247,15 @@ inline int64_t partial_bytes(int64_t M, int64_t N, const Plan& pl) {
   return pl.splits <= 1 ? 0 : pl.splits * ceil_div(M, pl.mt) * pl.mt * ceil_div(N, pl.nt) * pl.nt * 4;
 }
 
-// The cheapest plan; split_ok false: without a K split (no workspace for its partials).
-inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, int cus, bool split_ok) {
+// The cheapest plan; split_ok false: without a K split (no workspace for its partials).  Up to
+// kFusedNormM rows it is gemv_kernel where the norm is fused or its workgroups fill the CUs; a
+// narrow deep weight is better split (3072 columns, K 8192: 4 rows packed 10.6 -> 9.6 us, 1
+// row fp16 16.3 -> 14.3; 16384 columns fp16 20.0 us, 20.9 tiled).
+inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus,
+                        bool split_ok) {
   const int64_t groups = K / kGroup;
   Plan best{true, false, 16, 16, 1};
-  if (M <= kFusedNormM) return best;
+  if (M <= kFusedNormM && (norm || ceil_div(N, 16) > cus)) return best;
   float best_us = M <= kGemvMaxM ? gemv_cost(M, N, groups, int4, cus) : 1e30f;
   const TileCost* costs = int4 ? kPackedTiles : kHalfTiles;
   const int n = int4 ? (int)(sizeof(kPackedTiles) / sizeof(TileCost))
@@ -1212,17 +1287,18 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, int cus, boo
 }
 
 // choose_plan, remembered per thread for the last few sizes (it weighs some 50 plans).
-inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, int cus, bool split_ok = true) {
+inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus,
+                 bool split_ok = true) {
   struct Entry {
     int64_t M, N, K;
     int form;
     Plan pl;
   };
   static thread_local Entry memo[64] = {};
-  const int form = 4 * cus + 2 * int4 + split_ok;
+  const int form = 8 * cus + 4 * norm + 2 * int4 + split_ok;
   Entry& e = memo[(M * 31 + N * 7 + K / kGroup * 3 + form) & 63];
   if (e.M != M || e.N != N || e.K != K || e.form != form)
-    e = Entry{M, N, K, form, choose_plan(M, N, K, int4, cus, split_ok)};
+    e = Entry{M, N, K, form, choose_plan(M, N, K, int4, norm, cus, split_ok)};
   return e.pl;
 }
 
@@ -1343,21 +1419,26 @@ void launch_plan(fi::gemm::Params p, const fi::gemm::Plan& pl, void* workspace, 
   }
 }
 
-// gemv_kernel; kNorm: with the RMSNorm fused into it.
-template <bool kNorm>
-void launch_gemv(fi::gemm::Params p, bool int4, hipStream_t st) {
+// gemv_kernel; `norm`: with the RMSNorm fused into it.  Packed weights: eight waves (two per SIMD
+// hide the unpacking's VALU latency), except with a row of the norm per wave, whose registers
+// allow only one such workgroup per CU.
+void launch_gemv(const fi::gemm::Params& p, bool int4, bool norm, hipStream_t st) {
   using namespace fi::gemm;
-  p.groups_per_split = p.K / kGroup;
   const dim3 grid((unsigned)((p.N + 15) / 16), (unsigned)((p.M + 15) / 16), 1);
-  const size_t lds = kNorm ? (size_t)std::min(p.M, 16) * p.K * sizeof(half_t) : 0;
-  // packed weights: eight waves (two per SIMD hide the dequantization's VALU latency),
-  // except with the fused norm, whose registers allow only one such workgroup per CU
-  if (int4 && !kNorm)
-    hipLaunchKernelGGL((gemv_kernel<true, 3, false, 8>), grid, dim3(512), lds, st, p);
-  else if (int4)
-    hipLaunchKernelGGL((gemv_kernel<true, 6, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
+  const size_t lds = norm ? (size_t)p.M * p.K * sizeof(half_t) : 0;
+  const dim3 four(256), eight(512);
+  if (!norm && int4)
+    hipLaunchKernelGGL((gemv_kernel<true, 3, 0, 8>), grid, eight, lds, st, p);
+  else if (!norm)
+    hipLaunchKernelGGL((gemv_kernel<false, 3, 0, 4>), grid, four, lds, st, p);
+  else if (!int4)
+    hipLaunchKernelGGL((gemv_kernel<false, 3, 4, 4>), grid, four, lds, st, p);
+  else if (p.M == 1)
+    hipLaunchKernelGGL((gemv_kernel<true, 3, 1, 8>), grid, eight, lds, st, p);
+  else if (p.M == 2)
+    hipLaunchKernelGGL((gemv_kernel<true, 3, 2, 8>), grid, eight, lds, st, p);
   else
-    hipLaunchKernelGGL((gemv_kernel<false, 3, kNorm, 4>), grid, dim3(kThreads), lds, st, p);
+    hipLaunchKernelGGL((gemv_kernel<true, 6, 4, 4>), grid, four, lds, st, p);
 }
 
 // gemm_kernel: calls of 17 to 128 rows whose rows lie too far apart for 32-bit offsets, with
@@ -1442,8 +1523,8 @@ Layout layout(int64_t M, int64_t N, int64_t K, const fi::gemm::Plan& pl, bool in
 size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, bool norm) {
   using namespace fi::gemm;
   const int cus = fi::device_cu_count(nullptr);
-  const Layout packed = layout(M, N, K, plan(M, N, K, true, cus), true, norm);
-  const Layout half = layout(M, N, K, plan(M, N, K, false, cus), false, norm);
+  const Layout packed = layout(M, N, K, plan(M, N, K, true, norm, cus), true, norm);
+  const Layout half = layout(M, N, K, plan(M, N, K, false, norm, cus), false, norm);
   if (M >= kDenseMinM) return packed.rows + round256(N * K * 2);
   return std::max(packed.total, half.total);
 }
@@ -1459,14 +1540,14 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   const bool norm = norm_w != nullptr;
   const int cus = device_cu_count(st);
   if (!workspace || ((uintptr_t)workspace & 255)) workspace_bytes = 0;
-  Plan pl = plan(M, N, K, int4, cus);
+  Plan pl = plan(M, N, K, int4, norm, cus);
   Layout l = layout(M, N, K, pl, int4, norm);
   // Up to kGemvMaxM rows, and fp16 weights from kDenseMinM rows, a call without room for the
   // partials runs unsplit; packed weights from kDenseMinM rows always need the size queried.
   size_t need = l.total;
   if (M >= kDenseMinM && int4) need = l.rows + round256(N * K * 2);
   if (workspace_bytes < l.total && (M <= kGemvMaxM || (M >= kDenseMinM && !int4))) {
-    pl = M <= kGemvMaxM ? Plan{true, false, 16, 16, 1} : plan(M, N, K, int4, cus, false);
+    pl = M <= kGemvMaxM ? Plan{true, false, 16, 16, 1} : plan(M, N, K, int4, norm, cus, false);
     l = layout(M, N, K, pl, int4, norm);
     need = l.total;
   }
@@ -1499,7 +1580,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   if (fused) {
     p.norm_w = (const half_t*)norm_w;
     p.eps = eps;
-    launch_gemv<true>(p, int4, st);
+    launch_gemv(p, int4, true, st);
     return check_launch(fn);
   }
   if (norm) {  // separate norm pass into the workspace
@@ -1511,7 +1592,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
     p.x_stride = K;
   }
   if (pl.gemv) {
-    launch_gemv<false>(p, int4, st);
+    launch_gemv(p, int4, false, st);
     return check_launch(fn);
   }
   if (pl.dense && int4) {  // unpack the weight into the workspace
@@ -1527,7 +1608,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   if (spans_ok(p, pl))
     launch_plan(p, pl, ws + l.rows, st);
   else if (M <= kGemvMaxM)
-    launch_gemv<false>(p, int4, st);
+    launch_gemv(p, int4, false, st);
   else
     launch_far_rows(p, int4, pl.splits, ws + l.rows, st);
   return check_launch(fn);

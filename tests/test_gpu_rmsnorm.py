@@ -87,3 +87,26 @@ def test_rms_norm_int4_matmul_vs_oracle(hip, M, packed_weights):
     for got in (out, two_step):
         g = got.float().cpu().numpy().astype(np.float64)
         assert np.all(np.abs(g - exact) <= bound), float(np.max(np.abs(g - exact) - bound))
+
+
+# The norm shared out over the workgroup (1 and 2 rows, packed weights): rows of one load and of
+# several per thread, a length that leaves threads idle, the longest shared-out row, one past it,
+# strided rows, and a last column tile with one column.
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("K,pad", [(128, 0), (3072, 8), (4096, 0), (4224, 64), (8192, 0), (8320, 0)])
+def test_rms_norm_int4_matmul_few_rows(hip, M, K, pad):
+    banner(f"rms_norm_int4_matmul M={M} K={K} row pad {pad}")
+    from fast_infer_amd import dequantize_int4, quantize_int4_groupwise, rms_norm_int4_matmul
+
+    N = 145
+    x, nw = _inputs(M + K, M, K, 2.0)
+    w = (np.random.default_rng(K).standard_normal((N, K)) * 0.02).astype(np.float16)
+    weight = quantize_int4_groupwise(torch.from_numpy(w).to(DEV))
+    big = torch.full((M + 1, K + pad), float("nan"), dtype=torch.float16, device=DEV)
+    big[:M, :K] = torch.from_numpy(x).to(DEV)
+    out = rms_norm_int4_matmul(big[:M, :K], torch.from_numpy(nw).to(DEV), weight)
+    xn, w16 = ON.rms_norm(x, nw), dequantize_int4(*weight).cpu().numpy()
+    mag = np.abs(xn.astype(np.float64)) @ np.abs(w16.astype(np.float64)).T
+    bound = OI.matmul_bound(xn, w16) + mag * 2.0 ** -10  # an fp16 ulp in a normalized element
+    got = out.float().cpu().numpy().astype(np.float64)
+    assert np.all(np.abs(got - OI.matmul_exact(xn, w16)) <= bound)
