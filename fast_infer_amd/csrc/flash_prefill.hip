@@ -19,6 +19,8 @@
 //   * the diagonal tile is processed first; when a pool is given, the workgroup that
 //     owns a 64-token tile of K/V also copies it into the paged pool (the write of
 //     model.py:176-183, any block size), so the scatter costs no extra read.
+#include <algorithm>
+
 #include "common.h"
 
 namespace fi {
@@ -58,7 +60,7 @@ struct Params {
   float lazy_log2;   // lazy_raw * scale_log2 (about kLazyLog2)
   uint32_t q_sign;   // 0x80008000 when sm_scale < 0: Q is negated instead of the scale
   int q_rows;        // rows of Q loaded: seq_len, or 0 when sm_scale == 0 (Q read as zeros)
-  int num_q_tiles;
+  int num_q_tiles;   // HPW > 1: + 65536 * the grid row from which tiles go lightest first
   int k_records;     // bytes addressable from one (batch, kv head) base of k
   int v_records;
   int k_row_bytes;   // k_ss * 2 (spans are checked to fit 31 bits)
@@ -431,7 +433,14 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_kernel(Params p) {
   const int col = lane & 15;
   const int g = lane >> 4;
 
-  const int qt = p.num_q_tiles - 1 - (int)blockIdx.y;  // heaviest tiles first
+  // Heaviest tiles first; from grid row `fold` on lightest first.  (Written as a choice of the
+  // row: a choice between two forms of qt makes the compiler spill 104 registers.  Packed into
+  // one argument: a field of its own cost the one-head kernel, which has no fold, 0.2 us.)
+  const int num_q_tiles = HPW == 1 ? p.num_q_tiles : p.num_q_tiles & 0xffff;
+  const int fold = (int)((uint32_t)p.num_q_tiles >> 16);
+  const int row = HPW == 1 || (int)blockIdx.y < fold ? (int)blockIdx.y
+                                                     : num_q_tiles - 1 + fold - (int)blockIdx.y;
+  const int qt = num_q_tiles - 1 - row;
   const int q0 = qt * kQTile;
   const int hg_total = p.num_kv_heads * p.hg_per_kv;
   const int b = blockIdx.x / hg_total;
@@ -631,13 +640,16 @@ extern "C" int fi_flash_attention_fwd(const void* q, const void* k, const void* 
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t q_tiles = (seq_len + kQTile - 1) / kQTile;
   // Several query heads per workgroup share each staged K/V tile, but make the grid that
-  // many times smaller.  A grid below two workgroups per CU leaves slots idle for the whole
-  // call: one head per workgroup is then faster (batch 1 x 512: 12.8 against 22.4 us;
-  // batch 1 x 3072: 93 against 101 us; from two per CU up, several heads win).
+  // many times smaller, and a small grid leaves workgroup slots (two per CU) idle for the whole
+  // call: below one and a half workgroups per CU one head per workgroup is faster (3 heads and 1
+  // head: batch 1 x 512 20.6 and 13.0 us, 3 x 700 29.1 and 26.5, 4 x 512 (one per CU) 23.5 and
+  // 22.6, 1 x 3000 (376 workgroups) 92.8 and 90.5; but 6 x 512 (384) 25.0 and 30.3, 3 x 1111
+  // (432) 42.5 and 49.7), except that prompts of a few tiles gain from one per CU (8 x 200 14.8
+  // and 16.7).
+  const int64_t cus = device_cu_count((hipStream_t)stream);
   int hpw = heads_per_wg(group);
-  if (hpw > 1 && batch * num_kv_heads * (group / hpw) * q_tiles <
-                     2 * (int64_t)device_cu_count((hipStream_t)stream))
-    hpw = 1;
+  const int64_t hpw_wgs = batch * num_kv_heads * (group / hpw) * q_tiles;
+  if (hpw > 1 && hpw_wgs < (q_tiles <= 4 ? cus : cus + cus / 2)) hpw = 1;
   Params p;
   p.q = (const half_t*)q;
   p.k = (const half_t*)k;
@@ -682,11 +694,17 @@ extern "C" int fi_flash_attention_fwd(const void* q, const void* k, const void* 
   p.v_row_bytes = (int)(v_ss * 2);
 
   const int64_t gx = batch * num_kv_heads * p.hg_per_kv;
-  if (gx > 0x7fffffff || p.num_q_tiles > 65535) {
+  if (gx > 0x7fffffff || q_tiles > 65535) {
     set_error("fi_flash_attention_fwd: grid too large");
     return FI_ERR_UNSUPPORTED;
   }
-  const dim3 grid((unsigned)gx, (unsigned)p.num_q_tiles);
+  // A grid of up to two workgroups per CU is resident as a whole: its second half, on the CUs
+  // that hold the heaviest tiles, starts with the lightest (batch 1 x 4096 132.0 -> 126.9 us, 2 x
+  // 2048 73.8 -> 70.2, 4 x 1024 40.8 -> 39.5; with one head per workgroup no difference, and the
+  // kernel does not read it).
+  const dim3 grid((unsigned)gx, (unsigned)q_tiles);
+  const int64_t fold = gx * q_tiles <= 2 * cus ? std::min((cus + gx - 1) / gx, q_tiles) : q_tiles;
+  if (hpw > 1) p.num_q_tiles = (int)(uint32_t)(fold << 16 | q_tiles);
   const dim3 block(kThreads);
   const bool rows = k_cache && block_size != kPoolBlock;
   const hipStream_t st = (hipStream_t)stream;

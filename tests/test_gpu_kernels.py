@@ -540,3 +540,29 @@ def test_paged_decode_short_calls_without_workspace(hip):
         _lib.check(rc, "fi_paged_attention_fwd")
         outs.append(out.float())
     assert float((outs[0] - outs[1]).abs().max()) <= ATOL and torch.equal(outs[1], outs[2])
+
+
+# Prefill grids around the switches of the launch: one head per workgroup below one and a half
+# workgroups per CU (one, up to four query tiles), the lightest-first second half up to two per
+# CU (its first row inside, at the end of and past the grid), and grids past both.
+@pytest.mark.parametrize("B,S", [(8, 200), (8, 256), (8, 257), (6, 511), (6, 513), (4, 1023), (1, 3072),
+                                 (1, 4033), (5, 800), (17, 65)])
+def test_prefill_grid_switches(hip, B, S):
+    banner(f"prefill grid switches B={B} S={S}")
+    from fast_infer_amd import flash_attention
+
+    g = torch.Generator(device="cuda:0").manual_seed(B * S)
+    q, k, v = (torch.randn(B, S, h, 128, device="cuda:0", generator=g).half().transpose(1, 2)
+               for h in (24, 8, 8))
+    blocks = -(-S // 64)
+    table = torch.randperm(B * blocks, device="cuda:0", generator=g).int().view(B, blocks)
+    kc, vc = (torch.zeros(B * blocks, 64, 8, 128, dtype=torch.float16, device="cuda:0") for _ in range(2))
+    out = flash_attention(q, k, v, k_cache=kc, v_cache=vc, block_table=table)
+    mask = torch.ones(S, S, dtype=torch.bool, device="cuda:0").triu_(1)
+    for b in sorted({0, B // 2, B - 1}):
+        for h in (0, 1, 23):
+            s = q[b, h].float() @ k[b, h // 3].float().t().contiguous() * 128 ** -0.5
+            ref = s.masked_fill_(mask, -math.inf).softmax(-1) @ v[b, h // 3].float()
+            assert float((out[b, h].float() - ref).abs().max()) <= ATOL, (b, h)
+        for pool, x in ((kc, k), (vc, v)):
+            assert torch.equal(pool[table[b].long()].flatten(0, 1)[:S], x[b].transpose(0, 1))
