@@ -213,6 +213,47 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const half_t* x, int64_t x
     *(u32x4*)(o + k) = norm8(*(const u32x4*)(xr + k), r, *(const u32x4*)(w + k));
 }
 
+// rmsnorm_kernel with a workgroup per row (K up to 8192): every thread takes a few elements, the
+// waves' sums of squares meet in LDS.  A wave per row left few rows on a quarter of the
+// workgroups and loaded its 16 chunks one guarded load after another: rows of 3072 elements
+// 5.0 -> 3.4 us for 64 rows, 5.8 -> 5.1 for 1000, 37.5 -> 35.6 (5.7 TB/s) for 16384; of 8192 7.6 ->
+// 3.8 for 64.  Rows of up to 2048 elements leave threads idle, which many of them notice: 768
+// elements 4.5 -> 4.2 us for 1000 rows, but 17.3 against 21.2 for 16384, so they stay with
+// rmsnorm_kernel from kWaveRows rows.
+constexpr int kRowParts = 4;
+constexpr int kWaveRows = 1024;
+__global__ __launch_bounds__(256) void rmsnorm_row_kernel(const half_t* x, int64_t x_stride, int K,
+                                                          const half_t* w, float eps, half_t* out,
+                                                          int64_t out_stride) {
+  __shared__ float part[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // elements past K read zeros through the buffer bounds
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(x + (int64_t)blockIdx.x * x_stride), (short)0, K * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, K * 2, 0x00020000);
+  u32x4 v[kRowParts], wv[kRowParts];
+#pragma unroll
+  for (int i = 0; i < kRowParts; ++i) {
+    const int k2 = (threadIdx.x * 8 + i * 2048) * 2;
+    v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, k2, 0, 0));
+    wv[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, k2, 0, 0));
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < kRowParts; ++i) s += sum_sq8(v[i]);
+  s = wave_sum(s);
+  if (lane == 0) part[wave] = s;
+  __syncthreads();
+  const float r = rsqrtf((part[0] + part[1] + part[2] + part[3]) / (float)K + eps);
+  half_t* o = out + (int64_t)blockIdx.x * out_stride;
+#pragma unroll
+  for (int i = 0; i < kRowParts; ++i) {
+    const int k = threadIdx.x * 8 + i * 2048;
+    if (k < K) *(u32x4*)(o + k) = norm8(v[i], r, wv[i]);
+  }
+}
+
 // One row normalized by the calling wave into dst (LDS or global), K a multiple of 8.
 __device__ __forceinline__ void norm_row_to(const half_t* xr, const half_t* w, int K, float eps,
                                             half_t* dst, int lane) {
@@ -1309,7 +1350,6 @@ namespace {
 
 using fi::half_t;
 using fi::gemm::dequantize_kernel;
-using fi::gemm::rmsnorm_kernel;
 
 // Shared validation for the linear-layer entry points; FI_OK when the operands are usable.
 int check_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64_t K,
@@ -1417,6 +1457,17 @@ void launch_plan(fi::gemm::Params p, const fi::gemm::Plan& pl, void* workspace, 
     case 128064: launch_mid<128, 1>(p, st); break;
     default: launch_mid<128, 2>(p, st); break;
   }
+}
+
+void launch_rmsnorm(const half_t* x, int64_t x_stride, int64_t M, int64_t K, const half_t* w,
+                    float eps, half_t* out, int64_t out_stride, hipStream_t st) {
+  using namespace fi::gemm;
+  if (K <= kRowParts * 2048 && (K > 2048 || M < kWaveRows))
+    hipLaunchKernelGGL(rmsnorm_row_kernel, dim3((unsigned)M), dim3(256), 0, st, x, x_stride, (int)K, w,
+                       eps, out, out_stride);
+  else
+    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, st, x, x_stride,
+                       (int)M, (int)K, w, eps, out, out_stride);
 }
 
 // gemv_kernel; `norm`: with the RMSNorm fused into it.  Packed weights: eight waves (two per SIMD
@@ -1585,9 +1636,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   }
   if (norm) {  // separate norm pass into the workspace
     half_t* normed = (half_t*)ws;
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, st,
-                       (const half_t*)x, x_stride, (int)M, (int)K, (const half_t*)norm_w, eps,
-                       normed, K);
+    launch_rmsnorm((const half_t*)x, x_stride, M, K, (const half_t*)norm_w, eps, normed, K, st);
     p.x = normed;
     p.x_stride = K;
   }
@@ -1684,9 +1733,8 @@ extern "C" int fi_rmsnorm(const void* x, int64_t x_stride, int64_t M, int64_t hi
     set_error("fi_rmsnorm: rows must be 16-byte aligned and strides cover the rows");
     return FI_ERR_INVALID;
   }
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0,
-                     (hipStream_t)stream, (const half_t*)x, x_stride, (int)M, (int)hidden,
-                     (const half_t*)weight, eps, (half_t*)out, out_stride);
+  launch_rmsnorm((const half_t*)x, x_stride, M, hidden, (const half_t*)weight, eps, (half_t*)out,
+                 out_stride, (hipStream_t)stream);
   return check_launch("fi_rmsnorm");
 }
 

@@ -110,3 +110,19 @@ def test_rms_norm_int4_matmul_few_rows(hip, M, K, pad):
     bound = OI.matmul_bound(xn, w16) + mag * 2.0 ** -10  # an fp16 ulp in a normalized element
     got = out.float().cpu().numpy().astype(np.float64)
     assert np.all(np.abs(got - OI.matmul_exact(xn, w16)) <= bound)
+
+
+# Both norm kernels at the edges of their choice: rows of one chunk, of exactly and just over 2048
+# elements (few rows and many), the longest row of a workgroup and one past it; strided rows.
+@pytest.mark.parametrize("M,H,pad", [(5, 8, 0), (1023, 2048, 8), (1024, 2048, 0), (1025, 2056, 16),
+                                     (33, 6152, 0), (2, 8192, 8), (2, 8200, 0), (1500, 3072, 0)])
+def test_rms_norm_kernel_choice(hip, M, H, pad):
+    banner(f"rms_norm M={M} H={H} row pad {pad}")
+    from fast_infer_amd import rms_norm
+
+    x, w = _inputs(M + H, M, H, 1.0)
+    big = torch.full((M, H + pad), float("nan"), dtype=torch.float16, device=DEV)
+    big[:, :H] = torch.from_numpy(x).to(DEV)
+    got = rms_norm(big[:, :H], torch.from_numpy(w).to(DEV)).float().cpu().numpy().astype(np.float64)
+    exact = ON.rms_norm_exact(x, w)
+    assert np.all(np.abs(got - exact) <= ON.norm_bound(exact))
