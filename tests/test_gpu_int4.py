@@ -146,7 +146,7 @@ def test_int4_matmul_strided_x_and_batch_dims(hip):
     _check(out.reshape(14, N), x.reshape(14, K).numpy(), dequantize_int4(packed, scales).cpu().numpy())
 
 
-# 17..64 rows run the split-K kernel (gemm_sk_kernel): one K group, a two-way K split
+# 17..64 rows run split-K tiles (mid_gemm_kernel): one K group, a two-way K split
 # whose second part is shorter, an 8-way split of 64 groups, partial last column tiles,
 # strided X rows, the QKV shape at 33 and 48 rows, an N that is not a multiple of 4 with
 # and without a K split (scalar output stores), and a grid of 257 column tiles
@@ -189,7 +189,7 @@ def test_int4_matmul_prefill_size_sampled(hip):
 
 
 # 129 rows and up: the weight dequantized once, then the 256 x 256-tile fp16 GEMM
-# (wide_gemm_kernel).  Shapes: partial row and column tiles, two K steps (K 128) and
+# (tile_gemm_kernel).  Shapes: partial row and column tiles, two K steps (K 128) and
 # 128 (K 8192), row tiles in multiples of 8 (the XCD-banded tile order, also with a partial
 # last row tile) and not, N not a multiple of 8 (element stores), output rows with a stride
 # and an output that is only 2-byte aligned (element stores), X rows with a stride; packed
