@@ -148,7 +148,12 @@ FI_KV_OUT_OF_BLOCKS = 1
 FI_KV_TABLE_FULL = 2
 FI_KV_NEGATIVE_COUNT = 3
 
+# entry points the wrappers call once per launch
+FAST = ("fi_flash_attention_fwd", "fi_paged_attention_fwd", "fi_rope_store_kv", "fi_int4_matmul",
+        "fi_rmsnorm", "fi_rmsnorm_int4_matmul")
+
 _lib = None
+_calls = None
 _lock = threading.Lock()
 
 
@@ -158,7 +163,7 @@ class FastInferError(RuntimeError):
 
 def load() -> ctypes.CDLL:
     """Load the HIP library once and declare every entry point's signature."""
-    global _lib
+    global _lib, _calls
     if _lib is not None:
         return _lib
     with _lock:
@@ -173,8 +178,22 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+        from . import _fastcall
+
+        for name in FAST:
+            _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+        _calls = _fastcall
         _lib = lib
         return lib
+
+
+def calls():
+    """The entry points of ``FAST`` as native functions (csrc/fastcall.c): positional integers
+    (None for a null pointer) and floats, the return code back.  The wrappers' call path; every
+    other use goes through ``load()``."""
+    if _calls is None:
+        load()
+    return _calls
 
 
 def check(rc: int, what: str) -> None:

@@ -134,8 +134,7 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
     if batch == 0 or seq_len == 0:
         return o
-    lib = _lib.load()
-    rc = lib.fi_flash_attention_fwd(
+    rc = _lib.calls().fi_flash_attention_fwd(
         q_ptr, k_ptr, v_ptr, work.data_ptr(),
         batch, num_heads, num_kv_heads, seq_len, head_dim,
         qs[0], qs[1], qs[2], ks[0], ks[1], ks[2], vs[0], vs[1], vs[2],
@@ -225,14 +224,13 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if batch == 0:
         return o
 
-    lib = _lib.load()
     need = _lib.workspace_size("fi_paged_attention_workspace_size", batch, num_q_heads,
                                num_kv_heads, max(num_tokens, 1), head_dim)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     ws_ptr = workspace.data_ptr() if (need and workspace is not None) else None
     ws_bytes = workspace.numel() * workspace.element_size() if ws_ptr else 0
-    rc = lib.fi_paged_attention_fwd(
+    rc = _lib.calls().fi_paged_attention_fwd(
         q_ptr, qs[0], qs[1],
         k_cache.data_ptr(), v_cache.data_ptr(), num_blocks, block_size, num_kv_heads,
         block_table.data_ptr(), block_table.stride(0), bt_cols,

@@ -3,7 +3,8 @@
 Usage: ``python -m fast_infer_amd.build`` (or ``build_library()`` from Python).
 Each ``csrc/*.hip`` is compiled to an object in ``csrc/_build/`` in parallel, then
 linked into ``fast_infer_amd/libfastinfer_hip.so``.  The library exports only the
-``extern "C"`` entry points declared in ``include/fast_infer_amd.h``.
+``extern "C"`` entry points declared in ``include/fast_infer_amd.h``.  ``csrc/fastcall.c`` becomes
+the CPython module ``_fastcall.so``, through which the wrappers call the library.
 """
 
 from __future__ import annotations
@@ -13,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -20,6 +22,7 @@ CSRC = PKG_DIR / "csrc"
 BUILD_DIR = CSRC / "_build"
 LIB_NAME = "libfastinfer_hip.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+FASTCALL_PATH = PKG_DIR / "_fastcall.so"  # csrc/fastcall.c: the wrappers' native call path
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from emitting packed fp32 VALU instructions.
@@ -61,6 +64,18 @@ def _compile(hipcc: str, src: Path, extra: list[str]) -> Path:
     return obj
 
 
+def build_fastcall() -> Path:
+    """Compile the CPython module through which the wrappers call the library (host C only)."""
+    tmp = FASTCALL_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CC") or "gcc", "-O2", "-Wall", "-shared", "-fPIC",
+           "-I", sysconfig.get_paths()["include"], str(CSRC / "fastcall.c"), "-o", str(tmp)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"building {FASTCALL_PATH.name} failed:\n{' '.join(cmd)}\n{res.stderr}")
+    os.replace(tmp, FASTCALL_PATH)
+    return FASTCALL_PATH
+
+
 def build_library(verbose: bool = False, extra_flags: list[str] | None = None) -> Path:
     """Compile every csrc/*.hip for gfx950 and link the shared library; returns its path."""
     hipcc = _hipcc()
@@ -78,6 +93,7 @@ def build_library(verbose: bool = False, extra_flags: list[str] | None = None) -
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{res.stdout}{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    build_fastcall()
     if verbose:
         print(f"built {LIB_PATH}")
     return LIB_PATH

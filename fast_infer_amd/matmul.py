@@ -99,7 +99,7 @@ def int4_matmul(x: torch.Tensor, w, scales=None, groupsize: int = 128, *,
         workspace = _workspace(x.device, stream, need)
     ws_ptr = workspace.data_ptr() if need else None
     ws_bytes = workspace.numel() * workspace.element_size() if need else 0
-    rc = _lib.load().fi_int4_matmul(x_ptr, x_stride, M, K, w_ptr, w_stride, s_ptr, s_stride, N,
+    rc = _lib.calls().fi_int4_matmul(x_ptr, x_stride, M, K, w_ptr, w_stride, s_ptr, s_stride, N,
                                     groupsize, out.data_ptr(), N, ws_ptr, ws_bytes, stream)
     _lib.check(rc, "int4_matmul")
     return out if len(x_shape) == 2 else out.reshape(*x_shape[:-1], N)
@@ -171,7 +171,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5) -> torch.
     rows = x2.shape[0]
     out = torch.empty(rows, hidden, dtype=torch.float16, device=x.device)
     if rows:
-        rc = _lib.load().fi_rmsnorm(x_ptr, x_stride, rows, hidden, wt.data_ptr(), float(eps),
+        rc = _lib.calls().fi_rmsnorm(x_ptr, x_stride, rows, hidden, wt.data_ptr(), float(eps),
                                     out.data_ptr(), hidden, _lib.tensor_stream(x))
         _lib.check(rc, "rms_norm")
     return out.reshape(x.shape)
@@ -206,7 +206,7 @@ def rms_norm_int4_matmul(x: torch.Tensor, norm_weight: torch.Tensor, w, eps: flo
         workspace = _workspace(x.device, stream, need)
     ws_ptr = workspace.data_ptr() if need else None
     ws_bytes = workspace.numel() * workspace.element_size() if need else 0
-    rc = _lib.load().fi_rmsnorm_int4_matmul(x_ptr, x_stride, M, K, nw.data_ptr(), float(eps),
+    rc = _lib.calls().fi_rmsnorm_int4_matmul(x_ptr, x_stride, M, K, nw.data_ptr(), float(eps),
                                             w_ptr, w_stride, s_ptr, s_stride, N, groupsize,
                                             out.data_ptr(), N, ws_ptr, ws_bytes, stream)
     _lib.check(rc, "rms_norm_int4_matmul")

@@ -153,7 +153,7 @@ def rope_store_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None,
     else:
         kc_ptr = vc_ptr = bt_ptr = None
         n_blocks = bs = bt_stride = bt_cols = 0
-    rc = _lib.load().fi_rope_store_kv(
+    rc = _lib.calls().fi_rope_store_kv(
         q_ptr, qs[0], qs[1], qs[2], k_ptr, ks[0], ks[1], ks[2], v_ptr, vs[0], vs[1], vs[2],
         cos_t.data_ptr(), sin_t.data_ptr(), table_rows,
         q_out.data_ptr(), qo[0], qo[1], qo[2], ko_ptr, ko[0], ko[1], ko[2],

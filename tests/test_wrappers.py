@@ -88,3 +88,44 @@ def test_workspace_size_cache_matches_direct_queries():
                 == lib.fi_int4_matmul_workspace_size(*sizes))
         assert (_lib.workspace_size("fi_rmsnorm_int4_matmul_workspace_size", *sizes)
                 == lib.fi_rmsnorm_int4_matmul_workspace_size(*sizes))
+
+
+def test_native_calls_agree_with_the_library():
+    """The native call path hands every argument on as the ctypes binding does: the same return
+    codes and messages for calls that validation ends (no kernel runs), argument by argument."""
+    lib, calls = _lib.load(), _lib.calls()
+    a = 1 << 40  # an aligned address no call here dereferences
+    good = {
+        "fi_flash_attention_fwd": [a, a, a, a, 0, 24, 8, 64, 128, 1, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 8, 0.1,
+                                   None, None, 0, 64, None, 0, 0, None],
+        "fi_paged_attention_fwd": [a, 8, 8, a, a, 4, 64, 8, a, 4, 4, a, 100, a, 8, 8, 0, 24, 128, 0.1, None,
+                                   0, None],
+        "fi_rope_store_kv": [a, 8, 8, 8, a, 8, 8, 8, a, 8, 8, 8, a, a, 64, a, 8, 8, 8, None, 0, 0, 0, a, a,
+                             4, 64, a, 4, 4, 0, 1, 24, 8, 128, 0, None, None],
+        "fi_int4_matmul": [a, 256, 0, 256, a, 128, a, 2, 64, 128, a, 64, None, 0, None],
+        "fi_rmsnorm": [a, 256, 0, 256, a, 1e-5, a, 256, None],
+        "fi_rmsnorm_int4_matmul": [a, 256, 0, 256, a, 1e-5, a, 128, a, 2, 64, 128, a, 64, None, 0, None],
+    }
+    assert set(good) == set(_lib.FAST)
+    sizes = {"fi_flash_attention_fwd": range(4, 9), "fi_paged_attention_fwd": (5, 6, 7, 10, 12, 16, 17, 18),
+             "fi_rope_store_kv": (14, 30, 31, 32, 33, 34), "fi_int4_matmul": (2, 3, 8),
+             "fi_rmsnorm": (2, 3), "fi_rmsnorm_int4_matmul": (2, 3, 8)}
+    for name, args in good.items():
+        native, reference = getattr(calls, name), getattr(lib, name)
+        assert len(args) == len(_lib.SIGNATURES[name][1])
+        assert native(*args) == reference(*args) == _lib.FI_OK, name  # empty calls
+        for i in sizes[name]:  # every size, made negative: refused with the same message
+            bad = list(args)
+            bad[i] = -3 - i
+            assert native(*bad) == reference(*bad), (name, i)
+            native(*bad)
+            said = lib.fi_last_error()
+            reference(*bad)
+            assert said == lib.fi_last_error(), (name, i)
+        with pytest.raises(TypeError, match="arguments"):
+            native(*args[:-1])
+        for wrong in (1.5, "1", None):  # in place of a size
+            with pytest.raises(TypeError):
+                native(*[wrong if i == sizes[name][0] else x for i, x in enumerate(args)])
+        with pytest.raises(OverflowError):
+            native(*[1 << 70 if i == 4 else x for i, x in enumerate(args)])
