@@ -178,8 +178,12 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
-        from . import _fastcall
-
+        try:
+            from . import _fastcall
+        except ImportError as e:
+            raise FastInferError(
+                "_fastcall.so is not built; run `python -m fast_infer_amd.build` "
+                "(or __graft_entry__.build()) first") from e
         for name in FAST:
             _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
         _calls = _fastcall
