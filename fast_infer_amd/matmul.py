@@ -48,24 +48,53 @@ def _norm_weight(w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     return w if w.is_contiguous() else w.contiguous()
 
 
-# Split-K calls need a workspace for their fp32 partials; one per (device, stream), grown
-# on demand, so back-to-back calls on a stream reuse it.  A buffer that is outgrown is
-# kept alive, never returned to the allocator: a HIP graph captured earlier may hold its
-# address (graphs captured on one stream share the key), and replaying that graph must
-# not write into memory that was handed out again.
+# Calls that split K, unpack the weight or normalize rows first need a workspace; one per
+# (device, stream), grown on demand, so back-to-back calls on a stream reuse it.  A captured
+# call takes none of it: its graph may be replayed beside eager calls on that stream and beside
+# other graphs captured there (torch captures on one shared stream by default).
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
-_outgrown: list[torch.Tensor] = []
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        if ws is not None:
-            _outgrown.append(ws)
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws
+
+
+def _capturing(t: torch.Tensor, stream: int) -> bool:
+    """Whether `stream`, the current stream on the device of `t`, is being captured (the
+    default stream never is)."""
+    if not stream:
+        return False
+    index = t.get_device()
+    if index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(index):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def _out_and_workspace(x: torch.Tensor, M: int, N: int, need: int, stream: int,
+                       workspace: torch.Tensor | None):
+    """The fp16 output [M, N] and the pointer and size of `need` bytes of workspace: the
+    caller's when it is large enough, else the stream's, else, under capture, memory of the
+    call's own.  That is one allocation with the output, so it lives where and as long as the
+    output does: in the graph's pool, or for a capture torch does not know of, with the tensor
+    that its owner has to keep anyway."""
+    if not need:
+        return torch.empty(M, N, dtype=torch.float16, device=x.device), None, 0
+    if workspace is None or workspace.numel() * workspace.element_size() < need:
+        if _capturing(x, stream):
+            nbytes = M * N * 2
+            at = (nbytes + 255) // 256 * 256  # the workspace is 256-byte aligned
+            buf = torch.empty(at + need, dtype=torch.uint8, device=x.device)
+            out = buf[:nbytes].view(torch.float16).view(M, N)
+            return out, buf.data_ptr() + at, need
+        workspace = _workspace(x.device, stream, need)
+    out = torch.empty(M, N, dtype=torch.float16, device=x.device)
+    return out, workspace.data_ptr(), workspace.numel() * workspace.element_size()
 
 
 def int4_matmul(x: torch.Tensor, w, scales=None, groupsize: int = 128, *,
@@ -75,7 +104,7 @@ def int4_matmul(x: torch.Tensor, w, scales=None, groupsize: int = 128, *,
     K/groupsize])`` or an fp16 ``[N, K]`` tensor; ``scales`` is ignored as in the
     reference.  Accumulation is fp32, the output rounded to fp16 once.  ``workspace``
     (optional) must not be shared by calls that overlap in time; by default one cached
-    workspace per device and stream is used.  The packed kernels read 128-wide groups (the
+    workspace per device and stream is used, and under graph capture one of the call's own.  The packed kernels read 128-wide groups (the
     reference's); packed weights with another group size are dequantized first (the same
     fp16 values) and take the fp16 form."""
     _need_cuda("x", x)
@@ -90,15 +119,11 @@ def int4_matmul(x: torch.Tensor, w, scales=None, groupsize: int = 128, *,
         x = x.to(torch.float16)
     x2, x_stride, x_ptr = _rows16(x if len(x_shape) == 2 else x.reshape(-1, K), 2)
     M = x2.shape[0]
-    out = torch.empty(M, N, dtype=torch.float16, device=x.device)
     if M == 0 or N == 0:
-        return out if len(x_shape) == 2 else out.reshape(*x_shape[:-1], N)
+        return torch.empty(*x_shape[:-1], N, dtype=torch.float16, device=x.device)
     stream = _lib.tensor_stream(x)
     need = _lib.workspace_size("fi_int4_matmul_workspace_size", M, N, K)
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = _workspace(x.device, stream, need)
-    ws_ptr = workspace.data_ptr() if need else None
-    ws_bytes = workspace.numel() * workspace.element_size() if need else 0
+    out, ws_ptr, ws_bytes = _out_and_workspace(x, M, N, need, stream, workspace)
     rc = _lib.calls().fi_int4_matmul(x_ptr, x_stride, M, K, w_ptr, w_stride, s_ptr, s_stride, N,
                                     groupsize, out.data_ptr(), N, ws_ptr, ws_bytes, stream)
     _lib.check(rc, "int4_matmul")
@@ -197,15 +222,11 @@ def rms_norm_int4_matmul(x: torch.Tensor, norm_weight: torch.Tensor, w, eps: flo
     nw = _norm_weight(norm_weight, x)
     x2, x_stride, x_ptr = _rows16(x if len(x_shape) == 2 else x.reshape(-1, K), 2)
     M = x2.shape[0]
-    out = torch.empty(M, N, dtype=torch.float16, device=x.device)
     if M == 0 or N == 0:
-        return out if len(x_shape) == 2 else out.reshape(*x_shape[:-1], N)
+        return torch.empty(*x_shape[:-1], N, dtype=torch.float16, device=x.device)
     stream = _lib.tensor_stream(x)
     need = _lib.workspace_size("fi_rmsnorm_int4_matmul_workspace_size", M, N, K)
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = _workspace(x.device, stream, need)
-    ws_ptr = workspace.data_ptr() if need else None
-    ws_bytes = workspace.numel() * workspace.element_size() if need else 0
+    out, ws_ptr, ws_bytes = _out_and_workspace(x, M, N, need, stream, workspace)
     rc = _lib.calls().fi_rmsnorm_int4_matmul(x_ptr, x_stride, M, K, nw.data_ptr(), float(eps),
                                             w_ptr, w_stride, s_ptr, s_stride, N, groupsize,
                                             out.data_ptr(), N, ws_ptr, ws_bytes, stream)

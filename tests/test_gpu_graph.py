@@ -113,6 +113,50 @@ def test_decode_step_graph_replay(hip, B):
         assert torch.isfinite(noise)
 
 
+@pytest.mark.parametrize("M,N,K,norm", [(8, 5120, 3072, False), (4, 3072, 8192, False),
+                                        (12, 5120, 3072, True), (300, 3072, 8192, False)])
+def test_default_captures_replayed_at_once(hip, M, N, K, norm):
+    """Two graphs of split-K calls, captured the ordinary way (both on torch's shared capture
+    stream, no workspace given), replayed at the same time on two streams beside eager calls on
+    that capture stream: no call shares its workspace with another, so all keep their bits."""
+    banner(f"two default captures replayed at once, {M} x {N} x {K}, norm {norm}")
+    from fast_infer_amd import int4_matmul, quantize_int4_groupwise, rms_norm_int4_matmul
+
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    w = quantize_int4_groupwise((torch.randn(N, K, device=DEV, generator=g) * 0.02).half())
+    nw = (1.0 + 0.1 * torch.randn(K, device=DEV, generator=g)).half()
+    xs = [torch.randn(M, K, device=DEV, generator=g).half() for _ in range(3)]
+
+    def call(x):
+        return rms_norm_int4_matmul(x, nw, w) if norm else int4_matmul(x, w)
+
+    refs = [call(x) for x in xs]
+    capture = torch.cuda.graph.default_capture_stream or torch.cuda.Stream()
+    torch.cuda.graph.default_capture_stream = capture
+    with torch.cuda.stream(capture):
+        call(xs[2])
+    torch.cuda.synchronize()
+    graphs, outs = [], []
+    for x in xs[:2]:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            outs.append([call(x) for _ in range(20)])
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for rep in range(6):
+        for o in outs[0] + outs[1]:
+            o.zero_()
+        torch.cuda.synchronize()
+        for graph, st in zip(graphs, streams):
+            with torch.cuda.stream(st):
+                graph.replay()
+        with torch.cuda.stream(capture):
+            eager = [call(xs[2]) for _ in range(20)]
+        torch.cuda.synchronize()
+        for got, ref in ((outs[0], refs[0]), (outs[1], refs[1]), (eager, refs[2])):
+            assert all(torch.equal(o, ref) for o in got), rep
+
+
 def test_int4_workspace_two_captures_shared_pool(hip):
     """Two graphs captured back to back on a shared memory pool, the second needing a larger
     split-K workspace than the first: the first graph's workspace must stay allocated, so
