@@ -11,6 +11,7 @@ model.py:82 and the projection after it in one call.
 
 from __future__ import annotations
 
+import threading
 import warnings
 
 import torch
@@ -49,18 +50,25 @@ def _norm_weight(w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 
 # Calls that split K, unpack the weight or normalize rows first need a workspace; one per
-# (device, stream), grown on demand, so back-to-back calls on a stream reuse it.  A captured
-# call takes none of it: its graph may be replayed beside eager calls on that stream and beside
-# other graphs captured there (torch captures on one shared stream by default).
-_workspaces: dict[tuple[int, int], torch.Tensor] = {}
+# (device, stream), grown on demand, so back-to-back calls on a stream reuse it.  It is the
+# thread's own: such a call may be several launches, and those of two threads on one stream
+# (both on the default one) can alternate.  A captured call takes none of it: its graph may be
+# replayed beside eager calls on that stream and beside other graphs captured there (torch
+# captures on one shared stream by default).
+class _Workspaces(threading.local):
+    def __init__(self):
+        self.of: dict[tuple[int, int], torch.Tensor] = {}
+
+
+_workspaces = _Workspaces()
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    ws = _workspaces.get(key)
+    ws = _workspaces.of.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
+        _workspaces.of[key] = ws
     return ws
 
 
@@ -104,7 +112,8 @@ def int4_matmul(x: torch.Tensor, w, scales=None, groupsize: int = 128, *,
     K/groupsize])`` or an fp16 ``[N, K]`` tensor; ``scales`` is ignored as in the
     reference.  Accumulation is fp32, the output rounded to fp16 once.  ``workspace``
     (optional) must not be shared by calls that overlap in time; by default one cached
-    workspace per device and stream is used, and under graph capture one of the call's own.  The packed kernels read 128-wide groups (the
+    workspace per thread, device and stream is used, and under graph capture one of the call's
+    own.  The packed kernels read 128-wide groups (the
     reference's); packed weights with another group size are dequantized first (the same
     fp16 values) and take the fp16 form."""
     _need_cuda("x", x)

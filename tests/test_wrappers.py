@@ -129,3 +129,25 @@ def test_native_calls_agree_with_the_library():
                 native(*[wrong if i == sizes[name][0] else x for i, x in enumerate(args)])
         with pytest.raises(OverflowError):
             native(*[1 << 70 if i == 4 else x for i, x in enumerate(args)])
+
+
+def test_cached_workspace_is_the_threads_own():
+    """Two threads on one stream get different workspaces (their calls may be several launches
+    each), one thread the same one again until it is outgrown."""
+    import threading
+
+    cpu = torch.device("cpu", 0)
+    got = {}
+
+    def use(name):
+        first = matmul._workspace(cpu, 0, 4096)
+        got[name] = (first, matmul._workspace(cpu, 0, 1 << 20), matmul._workspace(cpu, 0, 1 << 21))
+
+    threads = [threading.Thread(target=use, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for first, again, grown in got.values():
+        assert first is again and grown.numel() == 1 << 21
+    assert got[0][0].data_ptr() != got[1][0].data_ptr()
