@@ -1288,13 +1288,15 @@ inline int64_t partial_bytes(int64_t M, int64_t N, const Plan& pl) {
   return pl.splits <= 1 ? 0 : pl.splits * ceil_div(M, pl.mt) * pl.mt * ceil_div(N, pl.nt) * pl.nt * 4;
 }
 
-// The cheapest plan; split_ok false: without a K split (no workspace for its partials).  Up to
-// kFusedNormM rows it is gemv_kernel where the norm is fused or its workgroups fill the CUs; a
-// narrow deep weight is better split (3072 columns, K 8192: 4 rows packed 10.6 -> 9.6 us, 1
+// The cheapest plan whose partials take at most `room` bytes.  Up to kFusedNormM rows it is
+// gemv_kernel where the norm is fused or its workgroups fill the CUs; a narrow deep weight is
+// better split (3072 columns, K 8192: 4 rows packed 10.6 -> 9.6 us, 1
 // row fp16 16.3 -> 14.3; 16384 columns fp16 20.0 us, 20.9 tiled).
 inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus,
-                        bool split_ok) {
+                        int64_t room) {
   const int64_t groups = K / kGroup;
+  // the partials of a call that large stay within the unpacked weight's bytes
+  if (M >= kDenseMinM) room = std::min(room, N * K * 2);
   Plan best{true, false, 16, 16, 1};
   if (M <= kFusedNormM && (norm || ceil_div(N, 16) > cus)) return best;
   float best_us = M <= kGemvMaxM ? gemv_cost(M, N, groups, int4, cus) : 1e30f;
@@ -1306,14 +1308,13 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
     if (int4 && t.dense && M < kDenseMinM) continue;
     const int64_t tiles = ceil_div(M, t.mt) * ceil_div(N, t.nt);
     if (tiles > 0x7ffffff) continue;
-    const bool may_split = split_ok && (t.split > 0) && tiles <= kMaxSplitTiles;
+    const bool may_split = t.split > 0 && tiles <= kMaxSplitTiles;
     for (int64_t s = 1; s <= kMaxSplits && s <= groups; ++s) {
       if (s > 1 && (!may_split || tiles * s > 5 * (int64_t)cus)) break;
       const int64_t per = ceil_div(groups, s), splits = ceil_div(groups, per);
       if (splits != s) continue;  // a smaller count with the same groups per split
       const Plan pl{false, t.dense, t.mt, t.nt, (int)splits};
-      // the partials of a call that large stay within the unpacked weight's bytes
-      if (M >= kDenseMinM && partial_bytes(M, N, pl) > N * K * 2) break;
+      if (partial_bytes(M, N, pl) > room) break;
       const int64_t on_cu = ceil_div(tiles * splits, cus);
       float us = t.fixed + per * ((on_cu / t.per_cu) * t.load[t.per_cu] + t.load[on_cu % t.per_cu]);
       if (splits > 1) us += t.split + t.per_split * splits;
@@ -1328,19 +1329,35 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
 }
 
 // choose_plan, remembered per thread for the last few sizes (it weighs some 50 plans).
-inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus,
-                 bool split_ok = true) {
+inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus) {
   struct Entry {
     int64_t M, N, K;
     int form;
     Plan pl;
   };
   static thread_local Entry memo[64] = {};
-  const int form = 8 * cus + 4 * norm + 2 * int4 + split_ok;
+  const int form = 4 * cus + 2 * norm + int4;
   Entry& e = memo[(M * 31 + N * 7 + K / kGroup * 3 + form) & 63];
   if (e.M != M || e.N != N || e.K != K || e.form != form)
-    e = Entry{M, N, K, form, choose_plan(M, N, K, int4, norm, cus, split_ok)};
+    e = Entry{M, N, K, form, choose_plan(M, N, K, int4, norm, cus, INT64_MAX)};
   return e.pl;
+}
+
+// Bytes of partials without which a call of 17 to 128 rows is refused; with this much, or what
+// its plan takes if that is less, it runs (on a plan that fits).  Most of these calls need none:
+// the bound is what a split into about two workgroups per CU, kept below the weight's bytes,
+// takes (packed weights up to 64 rows: one workgroup per CU, at most eight groups each).
+inline int64_t least_partials(int64_t M, int64_t N, int64_t K, bool int4, int cus) {
+  const int64_t groups = K / kGroup, tiles = ceil_div(N, kNTile);
+  const bool few = int4 && M <= 64;
+  int64_t s = 1;
+  if (few)
+    s = std::max(ceil_div(groups, 8), std::min(groups, cus / tiles));
+  else if (tiles < 256)
+    s = std::min({ceil_div(512, tiles), std::max<int64_t>(1, K / (16 * M)), groups});
+  s = ceil_div(groups, ceil_div(groups, s));
+  if (s == 1) return 0;
+  return 4 * s * (few ? tiles * kNTile * (M <= 32 ? 32 : 64) : M * N);
 }
 
 }  // namespace gemm
@@ -1593,14 +1610,22 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
   if (!workspace || ((uintptr_t)workspace & 255)) workspace_bytes = 0;
   Plan pl = plan(M, N, K, int4, norm, cus);
   Layout l = layout(M, N, K, pl, int4, norm);
-  // Up to kGemvMaxM rows, and fp16 weights from kDenseMinM rows, a call without room for the
-  // partials runs unsplit; packed weights from kDenseMinM rows always need the size queried.
+  // A call without room for its plan's partials runs on a plan that fits: up to kGemvMaxM rows
+  // gemv_kernel, from there the cheapest with what there is.  Packed weights from kDenseMinM
+  // rows always need the size queried, 17 to 128 rows least_partials.
   size_t need = l.total;
-  if (M >= kDenseMinM && int4) need = l.rows + round256(N * K * 2);
-  if (workspace_bytes < l.total && (M <= kGemvMaxM || (M >= kDenseMinM && !int4))) {
-    pl = M <= kGemvMaxM ? Plan{true, false, 16, 16, 1} : plan(M, N, K, int4, norm, cus, false);
-    l = layout(M, N, K, pl, int4, norm);
-    need = l.total;
+  if (M >= kDenseMinM && int4) {
+    need = l.rows + round256(N * K * 2);
+  } else if (workspace_bytes < l.total) {
+    if (M > kGemvMaxM && M < kDenseMinM)
+      need = std::min(l.total, l.rows + round256(least_partials(M, N, K, int4, cus)));
+    else
+      need = l.rows;
+    if (workspace_bytes >= need) {
+      pl = M <= kGemvMaxM ? Plan{true, false, 16, 16, 1}
+                          : choose_plan(M, N, K, int4, norm, cus, (int64_t)(workspace_bytes - l.rows));
+      l = layout(M, N, K, pl, int4, norm);
+    }
   }
   if (workspace_bytes < need) {
     set_error("%s: workspace of %zu bytes (256-byte aligned) needed, %zu given", fn, need,

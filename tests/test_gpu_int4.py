@@ -520,6 +520,48 @@ def test_calls_without_room_for_partials(hip):
             _check_device(out, x, w16)
 
 
+# What calls of 17 to 128 rows have to bring: nothing but the normalized rows for most (the
+# first four), else the partials of a split into about two workgroups per CU; with that much
+# and less than the plan's own they run, with less they are refused.  The last two plans take
+# less than that bound, and run with what they take.
+@pytest.mark.parametrize("M,N,K,form,least", [(97, 5120, 3072, "packed", 0), (128, 3072, 3072, "fp16", 0),
+                                              (128, 5120, 3072, "packed", 0), (65, 16384, 3072, "fp16", 0),
+                                              (17, 5120, 3072, "packed", 3 * 80 * 64 * 32 * 4),
+                                              (128, 3072, 8192, "fp16", 4 * 128 * 3072 * 4),
+                                              (64, 16384, 3072, "packed", 2 * 256 * 64 * 64 * 4),
+                                              (40, 5120, 3072, "packed", 3 * 80 * 64 * 64 * 4)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_least_workspace_of_17_to_128_rows(hip, M, N, K, form, least, norm):
+    banner(f"linear call with its least workspace M={M} N={N} K={K} {form} norm {norm}")
+    from fast_infer_amd import _lib, dequantize_int4, rms_norm
+
+    lib = _lib.load()
+    packed, scales = _packed(M + N, N, K)
+    w16 = dequantize_int4(packed, scales)
+    w = (packed.data_ptr(), K // 2, scales.data_ptr(), K // 128) if form == "packed" else \
+        (w16.data_ptr(), K, None, 0)
+    x, nw = torch.randn(M, K, device=DEV).half(), torch.randn(K, device=DEV).half()
+    rows = M * K * 2 if norm else 0
+    size = lib.fi_rmsnorm_int4_matmul_workspace_size if norm else lib.fi_int4_matmul_workspace_size
+    least = min(least, size(M, N, K) - rows)
+    ws = torch.full((rows + least + 4096,), 255, dtype=torch.uint8, device=DEV)
+    out = torch.empty(M, N, dtype=torch.float16, device=DEV)
+    st = _lib.stream_handle(torch.device(DEV))
+
+    def call(nbytes):
+        tail = (*w, N, 128, out.data_ptr(), N, ws.data_ptr() if nbytes else None, nbytes, st)
+        if norm:
+            return lib.fi_rmsnorm_int4_matmul(x.data_ptr(), K, M, K, nw.data_ptr(), 1e-5, *tail)
+        return lib.fi_int4_matmul(x.data_ptr(), K, M, K, *tail)
+
+    if rows + least:
+        assert call(rows + least - 256) == _lib.FI_ERR_WORKSPACE
+    _lib.check(call(rows + least), "linear call")
+    torch.cuda.synchronize()
+    assert (ws[rows + least:] == 255).all()
+    _check_device(out, rms_norm(x, nw) if norm else x, w16)
+
+
 @pytest.mark.parametrize("form", ["packed", "fp16"])
 def test_rows_too_far_apart_for_buffer_offsets(hip, form):
     """20 rows of X spread over more than 2 GiB (gemm_kernel), K split and not."""
