@@ -126,3 +126,30 @@ def test_rms_norm_kernel_choice(hip, M, H, pad):
     got = rms_norm(big[:, :H], torch.from_numpy(w).to(DEV)).float().cpu().numpy().astype(np.float64)
     exact = ON.rms_norm_exact(x, w)
     assert np.all(np.abs(got - exact) <= ON.norm_bound(exact))
+
+
+def test_rms_norm_more_rows_than_a_workgroup_each(hip):
+    """2^24 rows of 2056 elements, in place: a launch of 256 threads per row would pass the 2^32
+    threads that one dimension takes."""
+    banner("rms_norm of 2^24 rows x 2056")
+    from fast_infer_amd import _lib
+
+    M, H = 1 << 24, 2056
+    if torch.cuda.mem_get_info()[0] < M * H * 2 + (8 << 30):
+        pytest.skip("needs 77 GB of free device memory")
+    row, w = _inputs(H, 3, H, 1.0)
+    rows, wt = torch.from_numpy(row).to(DEV), torch.from_numpy(w).to(DEV)
+    x = torch.empty(M, H, dtype=torch.float16, device=DEV)
+    x[:] = rows[0]
+    x[M // 2 + 1], x[M - 1] = rows[1], rows[2]
+    rc = _lib.load().fi_rmsnorm(x.data_ptr(), H, M, H, wt.data_ptr(), 1e-5, x.data_ptr(), H,
+                                _lib.stream_handle(torch.device(DEV)))
+    _lib.check(rc, "fi_rmsnorm")
+    got = x[[0, M // 2 + 1, M - 1]].double().cpu().numpy()
+    exact = ON.rms_norm_exact(row, w)
+    assert np.all(np.abs(got - exact) <= ON.norm_bound(exact))
+    x[M // 2 + 1], x[M - 1] = x[0], x[0]
+    for part in x.split(1 << 21):
+        assert bool((part == x[0]).all())
+    del x
+    torch.cuda.empty_cache()
