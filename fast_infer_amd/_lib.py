@@ -180,13 +180,12 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         try:
             from . import _fastcall
-        except ImportError as e:
-            raise FastInferError(
-                "_fastcall.so is not built; run `python -m fast_infer_amd.build` "
-                "(or __graft_entry__.build()) first") from e
-        for name in FAST:
-            _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
-        _calls = _fastcall
+        except ImportError:  # not built (no compiler or headers for it): the same calls, slower
+            _calls = lib
+        else:
+            for name in FAST:
+                _fastcall.bind(name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+            _calls = _fastcall
         _lib = lib
         return lib
 
@@ -194,7 +193,7 @@ def load() -> ctypes.CDLL:
 def calls():
     """The entry points of ``FAST`` as native functions (csrc/fastcall.c): positional integers
     (None for a null pointer) and floats, the return code back.  The wrappers' call path; every
-    other use goes through ``load()``."""
+    other use goes through ``load()``, as the wrappers' calls do where that module is not built."""
     if _calls is None:
         load()
     return _calls

@@ -15,6 +15,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -64,14 +65,23 @@ def _compile(hipcc: str, src: Path, extra: list[str]) -> Path:
     return obj
 
 
-def build_fastcall() -> Path:
-    """Compile the CPython module through which the wrappers call the library (host C only)."""
+def build_fastcall() -> Path | None:
+    """Compile the CPython module through which the wrappers call the library (host C only).
+    Where that is not possible (no C compiler, no Python headers) it warns, leaves no module
+    behind and returns None: the wrappers then call through ctypes."""
     tmp = FASTCALL_PATH.with_suffix(".so.tmp")
     cmd = [os.environ.get("CC") or "gcc", "-O2", "-Wall", "-shared", "-fPIC",
            "-I", sysconfig.get_paths()["include"], str(CSRC / "fastcall.c"), "-o", str(tmp)]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"building {FASTCALL_PATH.name} failed:\n{' '.join(cmd)}\n{res.stderr}")
+    try:
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        error = f"exit code {res.returncode}\n{res.stderr}" if res.returncode else None
+    except OSError as e:
+        error = str(e)
+    if error is not None:
+        FASTCALL_PATH.unlink(missing_ok=True)  # an older one may not fit the library
+        warnings.warn(f"{FASTCALL_PATH.name} not built, calls go through ctypes:\n"
+                      f"{' '.join(cmd)}\n{error}", RuntimeWarning, stacklevel=2)
+        return None
     os.replace(tmp, FASTCALL_PATH)
     return FASTCALL_PATH
 

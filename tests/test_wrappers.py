@@ -151,3 +151,33 @@ def test_cached_workspace_is_the_threads_own():
     for first, again, grown in got.values():
         assert first is again and grown.numel() == 1 << 21
     assert got[0][0].data_ptr() != got[1][0].data_ptr()
+
+
+def test_without_the_native_call_module(tmp_path, monkeypatch):
+    """Where the call module is missing the library loads all the same and the wrappers' calls
+    go through ctypes; where it cannot be compiled the build warns and goes on without it."""
+    import subprocess
+    import sys
+
+    from fast_infer_amd import build
+
+    code = ("import sys; sys.modules['fast_infer_amd._fastcall'] = None\n"
+            "from fast_infer_amd import _lib\n"
+            "a = 1 << 40\n"
+            "assert _lib.load().fi_version() and _lib.calls() is _lib.load()\n"
+            "assert _lib.calls().fi_rmsnorm(a, 256, 0, 256, a, 1e-5, a, 256, None) == _lib.FI_OK\n"
+            "assert _lib.calls().fi_rmsnorm(a, 100, 1, 100, a, 1e-5, a, 100, None) != _lib.FI_OK\n")
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                         cwd=build.PKG_DIR.parent)
+    assert res.returncode == 0, res.stderr
+
+    stale = tmp_path / "_fastcall.so"
+    stale.write_bytes(b"")
+    monkeypatch.setattr(build, "FASTCALL_PATH", stale)
+    for compiler in ("false", str(tmp_path / "no-such-compiler")):
+        monkeypatch.setenv("CC", compiler)
+        with pytest.warns(RuntimeWarning, match="ctypes"):
+            assert build.build_fastcall() is None
+        assert not stale.exists()
+    monkeypatch.delenv("CC")
+    assert build.build_fastcall() == stale and stale.exists()
