@@ -73,20 +73,31 @@ __global__ __launch_bounds__(64) void xcd_probe_kernel(unsigned* out) {
 
 // Arrival counters, zero at load and left zero by every launch.  Launches on one stream follow
 // one another, so they share the stream's set (one per stream, in order of first use, up to
-// kXcdStreams streams).  A captured launch may be replayed beside any stream: each gets
-// counters of its own, from a part of the array that is only ever handed out once (16 MiB,
-// some 8000 launches; captures past it use the second launch).
+// kXcdStreams streams).  A graph may be replayed beside any stream and any other graph: each
+// capture gets sets of its own, one for every stream taking part (what is captured on one
+// stream forms a chain in the graph), from a part of the array that is only ever handed out
+// once: 16 MiB, 2 to 8 KiB a set; captures past it use the second launch.  A set for each
+// launch lasted 146 captures of a 28-layer step with two such calls a layer; this lasts 8192.
 constexpr int kXcdStreams = 16;
 constexpr int kXcdSet = 8 * kXcdCounters;
 constexpr int kXcdCaptured = 4 << 20;
 __device__ __attribute__((aligned(256))) unsigned g_xcd_counters[kXcdStreams * kXcdSet + kXcdCaptured];
+
+struct XcdCapture {  // the set of one stream in one capture
+  hipStream_t st = nullptr;
+  unsigned long long id = 0;
+  unsigned* counters = nullptr;
+  int stride = 0;
+};
 
 struct XcdDevice {
   int state = 0;  // 0: not probed, 1: groups share an XCD, -1: they do not (or no answer)
   unsigned* counters = nullptr;
   hipStream_t streams[kXcdStreams] = {};
   int used = 0;      // streams with a set
-  int captured = 0;  // counters handed to captured launches
+  int captured = 0;  // counters handed to captures
+  XcdCapture captures[kXcdStreams];  // the latest, a place per stream (any one may be taken over)
+  int next = 0;
 };
 
 static std::mutex& xcd_mutex() {
@@ -156,16 +167,28 @@ unsigned* xcd_counters(hipStream_t st, int per_group, int* stride) {
   XcdDevice& xd = xcd_device(dev);
   if (!xcd_ready(xd, dev, st)) return nullptr;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (st != nullptr && hipStreamIsCapturing(st, &cs) != hipSuccess) {
+  unsigned long long id = 0;
+  if (st != nullptr && hipStreamGetCaptureInfo(st, &cs, &id) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
-  if (cs != hipStreamCaptureStatusNone) {
-    *stride = (per_group + 63) / 64 * 64;
-    if (xd.captured + 8 * *stride > kXcdCaptured) return nullptr;
-    unsigned* c = xd.counters + kXcdStreams * kXcdSet + xd.captured;
-    xd.captured += 8 * *stride;
-    return c;
+  if (cs == hipStreamCaptureStatusInvalidated) return nullptr;
+  if (cs == hipStreamCaptureStatusActive) {
+    int i = 0;
+    while (i < kXcdStreams && xd.captures[i].st != st) ++i;
+    if (i == kXcdStreams) {
+      i = xd.next;
+      xd.next = (i + 1) % kXcdStreams;
+    }
+    XcdCapture& c = xd.captures[i];
+    if (c.st != st || c.id != id || c.stride < per_group) {
+      const int need = (per_group + 63) / 64 * 64;
+      if (xd.captured + 8 * need > kXcdCaptured) return nullptr;
+      c = XcdCapture{st, id, xd.counters + kXcdStreams * kXcdSet + xd.captured, need};
+      xd.captured += 8 * need;
+    }
+    *stride = c.stride;
+    return c.counters;
   }
   *stride = kXcdCounters;
   int i = 0;

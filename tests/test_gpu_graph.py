@@ -157,6 +157,81 @@ def test_default_captures_replayed_at_once(hip, M, N, K, norm):
             assert all(torch.equal(o, ref) for o in got), rep
 
 
+def test_captured_branches_of_split_calls(hip):
+    """One capture on two streams, 20 split-K calls on each side of a fork: the branches may run
+    at once, so each keeps counters of its own; calls of one branch and calls that need more
+    counters than the first (a wide weight after a narrow one) share or replace theirs."""
+    banner("two branches of split-K calls in one graph")
+    from fast_infer_amd import int4_matmul, quantize_int4_groupwise
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    ws = [quantize_int4_groupwise((torch.randn(n, 3072, device=DEV, generator=g) * 0.02).half())
+          for n in (640, 36864)]
+    xs = [torch.randn(8, 3072, device=DEV, generator=g).half() for _ in range(2)]
+    refs = [[int4_matmul(x, w) for w in ws] for x in xs]
+    main, side = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    outs = [[], []]
+    with torch.cuda.graph(graph, stream=main):
+        side.wait_stream(main)
+        with torch.cuda.stream(side):
+            outs[1] = [int4_matmul(xs[1], ws[i % 3 // 2]) for i in range(20)]
+        outs[0] = [int4_matmul(xs[0], ws[i % 3 // 2]) for i in range(20)]
+        main.wait_stream(side)
+    for rep in range(4):
+        for o in outs[0] + outs[1]:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, ref in zip(outs, refs):
+            assert all(torch.equal(o, ref[i % 3 // 2]) for i, o in enumerate(got)), rep
+
+
+def test_many_captures_keep_the_in_launch_sum(hip):
+    """A server that captures its step again and again: after 9000 captured split-K calls in 150
+    graphs, a call is still one node (its K splits are added inside the launch).  The counters
+    are told apart by the runtime's capture ids: no two captures may share one."""
+    banner("150 captures of 60 split-K calls")
+    import ctypes
+
+    from fast_infer_amd import _lib, quantize_int4_groupwise
+
+    maps = open("/proc/self/maps").read().split("\n")
+    hiprt = ctypes.CDLL(next(m.split()[-1] for m in maps if "libamdhip64" in m))
+    lib = _lib.load()
+    M, N, K = 8, 5120, 3072
+    w, sc = quantize_int4_groupwise((torch.randn(N, K, device=DEV) * 0.02).half())
+    x, out = torch.randn(M, K, device=DEV).half(), torch.empty(M, N, dtype=torch.float16, device=DEV)
+    need = lib.fi_int4_matmul_workspace_size(M, N, K)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    side = torch.cuda.Stream()
+
+    def call():
+        _lib.check(lib.fi_int4_matmul(x.data_ptr(), K, M, K, w.data_ptr(), K // 2, sc.data_ptr(), K // 128,
+                                      N, 128, out.data_ptr(), N, ws.data_ptr(), need, side.cuda_stream),
+                   "fi_int4_matmul")
+
+    call()  # the placement check runs at a device's first eager call
+    torch.cuda.synchronize()
+    st = ctypes.c_void_p(side.cuda_stream)
+    ids = set()
+    for i in range(150):
+        graph, nodes = ctypes.c_void_p(), ctypes.c_size_t()
+        status, capture = ctypes.c_int(), ctypes.c_ulonglong()
+        assert hiprt.hipStreamBeginCapture(st, 1) == 0  # thread-local mode
+        assert hiprt.hipStreamGetCaptureInfo(st, ctypes.byref(status), ctypes.byref(capture)) == 0
+        ids.add(capture.value)
+        for _ in range(60):
+            call()
+        assert hiprt.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+        assert hiprt.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0
+        assert hiprt.hipGraphDestroy(graph) == 0
+        assert nodes.value == 60, i
+    assert len(ids) == 150
+
+
 def test_int4_workspace_two_captures_shared_pool(hip):
     """Two graphs captured back to back on a shared memory pool, the second needing a larger
     split-K workspace than the first: the first graph's workspace must stay allocated, so
