@@ -479,47 +479,70 @@ __global__ __launch_bounds__(kHeadDim) void merge_kernel(Params p) {
 }
 
 // Partition size (tokens, a multiple of kWgTokens) for a call of `units` = rows x head groups.
-// 256 CUs hold two workgroups each, and a second round of them, however small, costs a whole
-// workgroup's time (about 4 us of latency before it streams): the smallest partitions whose
-// workgroups fit one round, else the cap.  Workgroups are counted with every row at the maximum
-// length; with per-row lengths about a third of them is taken to be empty.  64-token partitions
-// pay only while half the slots stay free, and the merge reads 0.5 KiB per partition and head.
-// Measured against the smallest partition of at least 128 tokens that gave 2048 workgroups:
-// 1 row of 1024 tokens 9.5 -> 9.0 us (64 tokens, was 128), 4 of 4096 23.0 -> 17.4 (256, was
-// 128), 7 of 100..3001 18.1 -> 15.2 (256, was 128), 16 of 1024 21.7 -> 18.1 (256, was 128), 64 of
-// 4096 184 -> 171 (512, was 384); 32 of 512..4096 stays at 384 (50.6 us; 51.6 with 320, 52.4
-// with 512).
-// Up to kDirectTokens a call is one partition with no merge, except that the longer ones of few
-// units are cut into 64-token partitions (1 row of 500: 8.6 us against 10.4, 8 of 512 10.4
-// against 11.5, but 32 of 500 24.0 against 13.6).
-constexpr int64_t kDirectTokens = 512;
+//
+// With per-row lengths (`lens`) the host sees only their bound, and the rows may all be far
+// below it or one far above the others: about kSmallWgs workgroups if every row had the bound,
+// 128 to 384 tokens each, so that short rows still spread over several workgroups and a long
+// one over many.  Sizes that fill one round of the CUs at the bound are 15% faster where lengths
+// are uniform (7 rows of 100..3001: 14.2 against 16.9 us), but slower wherever they are not: 8
+// rows of 256..680 under a bound of 4096 15.0 against 12.5 us, 8 rows of 16 heads, lognormal
+// under 2048, 16.1 against 12.5, one row of 64 under a bound of 512 8.1 against 5.3.
+//
+// One shared length is known to the host.  256 CUs hold two workgroups each, and a second round
+// of them, however small, costs a whole workgroup's time (about 4 us of latency before it
+// streams): the smallest partitions whose workgroups fit one round, else the cap (against the
+// sizes above: 4 rows of 4096 22.8 -> 17.6 us, 12 of 1024 19.0 -> 16.4, 8 of 8192 52.6 -> 48.8;
+// past one round 32 of 2048 52.8 -> 50.7, but 48 of 700 with 16 heads 51.8 -> 54.5 at 512
+// tokens, a full and a small partition a row, so below 1024 tokens the cap is 384).  Partitions
+// of 64 tokens pay while half the slots stay free and a merge adds up no more than 16 (1 row of
+// 500 11.5 -> 8.7 us, of 1024 9.7 -> 9.1, but of 2048 10.2 -> 10.9; 48 units of 400 11.4 -> 12.0).
+constexpr int64_t kDirectTokens = 512;   // up to this: one partition with no merge, or 64 tokens
 constexpr int64_t kUnsplitTokens = 320;  // at most this: always one partition
+constexpr int64_t kMaxTokens64 = 1024;   // most tokens cut into partitions of 64
 constexpr int64_t kRoundWgs = 512;       // workgroups of one round
-constexpr int64_t kRoundWgsLens = 704;   // the same with per-row lengths
+constexpr int64_t kSmallWgs = 2048;
 static int tokens_per_split(int64_t units, int64_t num_tokens, bool lens) {
   auto wgs = [&](int64_t tps) { return units * ((num_tokens + tps - 1) / tps); };
-  const int64_t most = lens ? kRoundWgsLens : kRoundWgs;
-  int64_t tps;
-  if (num_tokens <= kDirectTokens) {
-    tps = num_tokens > kUnsplitTokens && wgs(64) <= kRoundWgs ? 64 : num_tokens;
-  } else if (wgs(64) <= kRoundWgs / 2) {
-    tps = 64;
+  int64_t tps, least = 128;
+  if (!lens && num_tokens > kUnsplitTokens && num_tokens <= kMaxTokens64 && wgs(64) <= kRoundWgs / 2) {
+    tps = least = 64;
+  } else if (num_tokens <= kDirectTokens) {
+    tps = num_tokens;
+  } else if (lens) {
+    const int64_t want = (kSmallWgs + units - 1) / units;
+    tps = std::min<int64_t>((num_tokens + want - 1) / want, 384);
   } else {
     tps = 128;
-    while (tps < 512 && wgs(tps) > most) tps += tps < 384 ? 64 : 128;
-    if (wgs(tps) > most) tps = lens ? 384 : 512;
+    while (tps < 512 && wgs(tps) > kRoundWgs) tps += tps < 384 ? 64 : 128;
+    if (num_tokens < 1024) tps = std::min<int64_t>(tps, 384);
   }
   const int64_t min_tps = (num_tokens + kMaxSplits - 1) / kMaxSplits;
-  if (tps < min_tps) tps = min_tps;
+  tps = std::max({tps, min_tps, least});
   tps = (tps + kWgTokens - 1) / kWgTokens * kWgTokens;
-  if (tps > kMaxSplitTokens) tps = kMaxSplitTokens;
-  return (int)tps;
+  return (int)std::min<int64_t>(tps, kMaxSplitTokens);
+}
+
+// Bytes of partial results of `splits` partitions a row.
+static size_t partial_bytes(int64_t batch, int64_t num_q_heads, int64_t splits) {
+  return splits <= 1 ? 0 : (size_t)(batch * num_q_heads * splits * (kHeadDim + 2)) * sizeof(float);
 }
 
 static int heads_per_wg(int64_t group) {
   for (int h = kMaxHeadsPerWg; h >= 1; --h)
     if (group % h == 0) return h;
   return 1;
+}
+
+// Partition size and partitions per row of a call of at least one row.
+struct Cut {
+  int tps;
+  int64_t splits;
+};
+static Cut cut(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t num_tokens, bool lens) {
+  const int64_t group = num_q_heads / num_kv_heads;
+  const int64_t units = batch * num_kv_heads * (group / heads_per_wg(group));
+  const int tps = tokens_per_split(units, std::max<int64_t>(num_tokens, 1), lens);
+  return {tps, std::max<int64_t>((num_tokens + tps - 1) / tps, 1)};
 }
 
 }  // namespace decode
@@ -535,14 +558,18 @@ extern "C" size_t fi_paged_attention_workspace_size(int64_t batch, int64_t num_q
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t wg_per_row = num_kv_heads * (group / heads_per_wg(group));
   if (max_num_tokens <= kUnsplitTokens) return 0;
-  // enough for any num_tokens up to this one: fewer tokens may be cut into more partitions
+  // enough for any num_tokens up to this one, with per-row lengths or without: at most
+  // kRoundWgs / 2 workgroups of 64 tokens ...
   const int64_t units = batch * wg_per_row;
-  const int64_t tps = std::min(tokens_per_split(units, max_num_tokens, false),
-                               tokens_per_split(units, max_num_tokens, true));
-  const int64_t splits = std::max((max_num_tokens + tps - 1) / tps,
-                                  std::min((max_num_tokens + 63) / 64, kRoundWgsLens / units));
-  if (splits <= 1) return 0;
-  return (size_t)(batch * num_q_heads * splits * (fi::kHeadDim + 2) * sizeof(float));
+  int64_t splits = std::min((std::min(max_num_tokens, kMaxTokens64) + 63) / 64, kRoundWgs / 2 / units);
+  if (splits <= kUnsplitTokens / 64) splits = 0;  // the shortest such call has more partitions
+  if (max_num_tokens > kDirectTokens) {
+    // ... of at least 128 tokens up to kSmallWgs, or partitions of the smaller cap
+    const int64_t small = std::min((max_num_tokens + 127) / 128, (kSmallWgs + units - 1) / units);
+    const int64_t capped = std::min<int64_t>((max_num_tokens + 383) / 384, kMaxSplits);
+    splits = std::max({splits, small, capped});
+  }
+  return partial_bytes(batch, num_q_heads, splits);
 }
 
 namespace {
@@ -614,15 +641,13 @@ int paged_fwd(const char* fn, const void* q, int64_t q_sb, int64_t q_sh, const v
   p.heads_per_wg = heads_per_wg(group);
   p.scale_log2 = sm_scale * kLog2e;
   const int64_t wg_per_row = num_kv_heads * (group / p.heads_per_wg);
-  const size_t need =
-      fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads, num_tokens, head_dim);
-  p.tokens_per_split = tokens_per_split(batch * wg_per_row, num_tokens > 0 ? num_tokens : 1,
-                                        context_lens != nullptr);
+  Cut c = cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr);
+  const size_t need = partial_bytes(batch, num_q_heads, c.splits);
   // calls of up to kDirectTokens tokens run without a workspace too, as one partition
   if (num_tokens <= kDirectTokens && (!workspace || workspace_bytes < need))
-    p.tokens_per_split = (int)kDirectTokens;
-  int64_t splits = (num_tokens + p.tokens_per_split - 1) / p.tokens_per_split;
-  if (splits < 1) splits = 1;
+    c = {(int)kDirectTokens, 1};
+  const int64_t splits = c.splits;
+  p.tokens_per_split = c.tps;
   p.max_splits = (int)splits;
   p.direct = splits == 1;
   p.head_dim = (int)head_dim;
@@ -733,11 +758,14 @@ extern "C" int fi_paged_attention_fwd_noalloc(const void* q, int64_t q_sb, int64
   using namespace fi;
   static const char* fn = "fi_paged_attention_fwd_noalloc";
   clear_error();
-  // up to kDirectTokens tokens: one partition, which leaves the shared scratch alone
-  const size_t need = batch > 0 && num_tokens > decode::kDirectTokens
-                          ? fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads,
-                                                              num_tokens, head_dim)
-                          : 0;
+  // up to kDirectTokens tokens: one partition, which leaves the shared scratch alone (sizes
+  // that are no call's are left to paged_fwd)
+  size_t need = 0;
+  if (batch > 0 && num_tokens > decode::kDirectTokens && num_q_heads > 0 && num_kv_heads > 0 &&
+      num_q_heads % num_kv_heads == 0 && head_dim_ok(head_dim))
+    need = decode::partial_bytes(
+        batch, num_q_heads,
+        decode::cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr).splits);
   if (need > kScratchBytes) {
     set_error("%s: these sizes need %zu bytes of split-K scratch, more than the %zu bytes "
               "this entry point holds per device; use fi_paged_attention_fwd with a workspace",

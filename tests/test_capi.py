@@ -257,3 +257,37 @@ def test_paged_workspace_size_covers_smaller_calls(lib):
                 tps = max(128, -(-max(min(384, -(-n // want)), -(-n // 1024)) // 64) * 64)
                 before = batch * kv * group * -(-n // tps) * 130 * 4
                 assert n <= 512 or before > scratch or need <= scratch, (batch, kv, group, n)
+
+
+def test_paged_partitions(lib):
+    """Partitions a call is cut into, as the workspace it asks for tells: with per-row lengths
+    (all rows may be far below the bound, or one far above the rest) 128 to 384 tokens in about
+    2048 workgroups at the bound, never one round of workgroups; with one shared length at most
+    that many, one round where that is enough.  The size query covers every one of them."""
+    import re
+
+    from fast_infer_amd import _lib
+
+    def splits(batch, hq, hkv, n, lens):
+        rc = lib.fi_paged_attention_fwd(16, hq * 128, 128, 16, 16, 1, 64, hkv, 16, 64, 64, 16 if lens else None,
+                                        n, 16, hq * 128, 128, batch, hq, 128, 1.0, None, 0, None)
+        assert rc == _lib.FI_ERR_WORKSPACE
+        need = int(re.search(rb"workspace of (\d+) bytes", lib.fi_last_error()).group(1))
+        assert need % (batch * hq * 130 * 4) == 0
+        return need // (batch * hq * 130 * 4)
+
+    for kv, group in ((8, 3), (1, 8), (16, 1), (4, 32)):
+        per_row = kv * (group // (16 if group == 32 else group))
+        for batch in (1, 2, 3, 7, 12, 33, 64, 200, 1000):
+            units, most = batch * per_row, {True: 0, False: 0}
+            for n in list(range(513, 1300, 41)) + [2048, 3001, 4096, 8192, 40000, 400000]:
+                want = -(-2048 // units)
+                tps = max(128, -(-max(min(384, -(-n // want)), -(-n // 1024)) // 64) * 64)
+                with_lens, shared = splits(batch, kv * group, kv, n, True), splits(batch, kv * group, kv, n, False)
+                assert with_lens == -(-n // tps), (kv, group, batch, n)
+                assert shared <= max(with_lens, 16 if n <= 1024 and units * -(-n // 64) <= 256 else 0)
+                assert units * shared <= 512 or shared <= -(-n // 384)
+                size = lib.fi_paged_attention_workspace_size(batch, kv * group, kv, n, 128)
+                for lens, count in ((True, with_lens), (False, shared)):
+                    most[lens] = max(most[lens], count)
+                    assert size >= most[lens] * batch * kv * group * 130 * 4, (kv, group, batch, n)
