@@ -579,6 +579,24 @@ static int heads_per_wg(int64_t group) {
   return 1;
 }
 
+// Several query heads per workgroup share each staged K/V tile, but make the grid that many
+// times smaller, and a small grid leaves workgroup slots (two per CU) idle for the whole call.
+// Workgroups, in sixteenths of a CU, from which they are faster than one head per workgroup:
+// from 1 to 2 per CU, the later the less a workgroup shares (two heads, narrow heads) and the
+// longer its chain of key tiles, whose sum a CU with one workgroup waits for.  Measured on 1036
+// grids of 1 to 2 per CU (256 CUs; time with several heads / with one): 3 x 128 wide 0.94 to
+// 0.63 all over (3 x 1111 49.7 -> 42.5 us), from 0.79 at one per CU for up to four query tiles;
+// 3 x 64 wide, 32 tiles 1.14 at 384 workgroups, 1.01 at 448 and 0.95 at 480; 2 x 128 wide, 4
+// tiles 1.16 at 256, 1.07 at 288 and 0.84 at 300, 24 tiles 1.16 at 384 and 0.97 at 432; 2 x 64
+// wide, 12 tiles 1.11 at 384 and 0.96 at 456, 64 tiles 1.16 at 448.
+static int several_heads_from(int hpw, int64_t head_dim, int64_t q_tiles) {
+  static constexpr int8_t kFrom[2][2][5] = {// query tiles: up to 4, 11, 15, 23, more
+                                            {{19, 24, 29, 31, 32}, {19, 24, 25, 27, 29}},
+                                            {{16, 24, 24, 26, 29}, {16, 24, 24, 24, 24}}};
+  return kFrom[hpw == 3][head_dim > 64]
+              [q_tiles <= 4 ? 0 : q_tiles <= 11 ? 1 : q_tiles <= 15 ? 2 : q_tiles <= 23 ? 3 : 4];
+}
+
 }  // namespace prefill
 }  // namespace fi
 
@@ -639,17 +657,11 @@ extern "C" int fi_flash_attention_fwd(const void* q, const void* k, const void* 
 
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t q_tiles = (seq_len + kQTile - 1) / kQTile;
-  // Several query heads per workgroup share each staged K/V tile, but make the grid that
-  // many times smaller, and a small grid leaves workgroup slots (two per CU) idle for the whole
-  // call: below one and a half workgroups per CU one head per workgroup is faster (3 heads and 1
-  // head: batch 1 x 512 20.6 and 13.0 us, 3 x 700 29.1 and 26.5, 4 x 512 (one per CU) 23.5 and
-  // 22.6, 1 x 3000 (376 workgroups) 92.8 and 90.5; but 6 x 512 (384) 25.0 and 30.3, 3 x 1111
-  // (432) 42.5 and 49.7), except that prompts of a few tiles gain from one per CU (8 x 200 14.8
-  // and 16.7).
   const int64_t cus = device_cu_count((hipStream_t)stream);
   int hpw = heads_per_wg(group);
-  const int64_t hpw_wgs = batch * num_kv_heads * (group / hpw) * q_tiles;
-  if (hpw > 1 && hpw_wgs < (q_tiles <= 4 ? cus : cus + cus / 2)) hpw = 1;
+  if (hpw > 1 && batch * num_kv_heads * (group / hpw) * q_tiles * 16 <
+                     cus * several_heads_from(hpw, head_dim, q_tiles))
+    hpw = 1;
   Params p;
   p.q = (const half_t*)q;
   p.k = (const half_t*)k;

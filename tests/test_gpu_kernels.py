@@ -566,3 +566,33 @@ def test_prefill_grid_switches(hip, B, S):
             assert float((out[b, h].float() - ref).abs().max()) <= ATOL, (b, h)
         for pool, x in ((kc, k), (vc, v)):
             assert torch.equal(pool[table[b].long()].flatten(0, 1)[:S], x[b].transpose(0, 1))
+
+
+# The same for groups and widths with other switches (two heads per workgroup, and heads of 64),
+# on both sides of each and around the folded grids, with pools of 64-token blocks and of others
+# (the kernels that write a row at a time).
+@pytest.mark.parametrize("hq,hkv,d,B,S,bs", [(16, 8, 128, 4, 800, 64), (16, 8, 128, 8, 800, 64),
+                                             (16, 8, 128, 8, 200, 16), (32, 8, 128, 5, 256, 64),
+                                             (32, 8, 128, 1, 1500, 64), (32, 8, 128, 1, 2048, 48),
+                                             (12, 4, 64, 3, 2048, 64), (12, 4, 64, 5, 1500, 16),
+                                             (8, 4, 64, 9, 700, 64), (24, 8, 128, 6, 513, 32)])
+def test_prefill_grid_switches_of_other_groups(hip, hq, hkv, d, B, S, bs):
+    banner(f"prefill grid switches {hq}/{hkv} heads of {d}, B={B} S={S}, block {bs}")
+    from fast_infer_amd import flash_attention
+
+    g = torch.Generator(device="cuda:0").manual_seed(B * S + hq)
+    q, k, v = (torch.randn(B, S, h, d, device="cuda:0", generator=g).half().transpose(1, 2)
+               for h in (hq, hkv, hkv))
+    blocks = -(-S // bs)
+    table = torch.randperm(B * blocks, device="cuda:0", generator=g).int().view(B, blocks)
+    kc, vc = (torch.zeros(B * blocks, bs, hkv, d, dtype=torch.float16, device="cuda:0") for _ in range(2))
+    out = flash_attention(q, k, v, k_cache=kc, v_cache=vc, block_table=table, block_size=bs)
+    mask = torch.ones(S, S, dtype=torch.bool, device="cuda:0").triu_(1)
+    for b in range(B):
+        for h in sorted({0, 1, hq // 2, hq - 1}):
+            kv = h * hkv // hq
+            s = q[b, h].float() @ k[b, kv].float().t().contiguous() * d ** -0.5
+            ref = s.masked_fill_(mask, -math.inf).softmax(-1) @ v[b, kv].float()
+            assert float((out[b, h].float() - ref).abs().max()) <= ATOL, (b, h)
+        for pool, x in ((kc, k), (vc, v)):
+            assert torch.equal(pool[table[b].long()].flatten(0, 1)[:S], x[b].transpose(0, 1))
