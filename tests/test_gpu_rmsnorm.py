@@ -128,6 +128,18 @@ def test_rms_norm_kernel_choice(hip, M, H, pad):
     assert np.all(np.abs(got - exact) <= ON.norm_bound(exact))
 
 
+@pytest.mark.parametrize("M,H", [(8191, 2056), (8192, 2056), (12031, 2176), (12032, 2176)])
+def test_rms_norm_many_rows_kernel_choice(hip, M, H):
+    banner(f"rms_norm M={M} H={H}")
+    from fast_infer_amd import rms_norm
+
+    x, w = (torch.from_numpy(a).to(DEV) for a in _inputs(M + H, M, H, 1.0))
+    exact = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-5) * w.double()
+    got = rms_norm(x, w).double()
+    # ON.norm_bound on the device
+    assert bool(((got - exact).abs() <= torch.from_numpy(ON.norm_bound(exact.cpu().numpy())).to(DEV)).all())
+
+
 def test_rms_norm_more_rows_than_a_workgroup_each(hip):
     """2^24 rows of 2056 elements, in place: a launch of 256 threads per row would pass the 2^32
     threads that one dimension takes."""
