@@ -139,6 +139,8 @@ SIGNATURES = {
          _ptr, _sz,                              # workspace
          _ptr],                                  # stream
     ),
+    "fi_selftest_linear_plan": (
+        ctypes.c_int, [_i64, _i64, _i64, ctypes.c_int, ctypes.c_int, _ptr]),
     "fi_selftest_mfma_f16": (ctypes.c_int, [_ptr, _ptr, _ptr, _ptr]),
 }
 

@@ -1250,48 +1250,76 @@ struct Plan {
 // apart, from here 256 rows of X (and of an fp16 W) have to span less than 2 GiB.
 constexpr int kDenseMinM = 129;
 constexpr int kGemvMaxM = 16;    // rows of one gemv_kernel workgroup
-constexpr int kMaxSplits = 10;
+constexpr int kMaxSplits = 16;
 constexpr int kMaxSplitTiles = 8 * kXcdCounters;  // tiles of a split call
 
-// Time of a call with one tile shape, in us, as measured on MI355X (3072, 5120 and 16384
-// columns, K 3072 and 8192, 5 to 5000 rows, cold weights, fitted by least squares; the tile
-// chosen by it is within 1.3% of the fastest measured on average):
-//   fixed + groups per split x (full rounds x load[per_cu] + load[workgroups of the last round
-//   on a CU]) + (K split: split + per_split x splits)
+// Time of a call with one tile shape, in us, as measured on MI355X and fitted by least squares:
+// 8232 sizes of 1 to 30000 rows, 88 to 28672 columns and K 128 to 14336, cold weights, each with
+// every tile and several K splits.  The plan chosen by it is within 1% of the fastest on average,
+// on sizes left out of the fit too, and within 6% for 19 of 20 (timings and fit:
+// profiles/linear_plans.py).  Tables fitted to K 3072 and 8192 alone lost elsewhere (fp16 weights,
+// K 384, 17 rows x 7168 columns 6.1 -> 10.5 us on 128 x 128 tiles; 5.2 with these):
+//   fixed + per_wg x (workgroups on a CU - 1) + per_mb x weight MB + per_x_mb x MB of X read by
+//   all column tiles + groups per split x (full rounds x load[per_cu] + load[workgroups of the
+//   last round on a CU]) + (K split: split + per_split x splits)
 // where a round is per_cu workgroups on every CU, and load[n] the time of one 128-wide K group
-// with n workgroups on the CU.
+// with n workgroups on the CU.  A CU's workgroups are those of its XCD, which takes an eighth of
+// the tiles.
 struct TileCost {
   bool dense;
   int mt, nt, per_cu;
-  float fixed, load[5], split, per_split;
+  float fixed, load[5], split, per_split, per_wg, per_mb, per_x_mb;
 };
 constexpr TileCost kPackedTiles[] = {
-    {false, 16, 64, 4, 3.4f, {0, 0.46f, 0.52f, 0.74f, 1.01f}, 0.94f, 0.15f},
-    {false, 32, 64, 4, 3.4f, {0, 0.49f, 0.57f, 0.86f, 1.28f}, 1.11f, 0.24f},
-    {false, 64, 64, 4, 4.6f, {0, 0.53f, 0.73f, 1.28f, 1.67f}, 1.12f, 0.28f},
-    {false, 64, 128, 4, 6.8f, {0, 0.77f, 1.36f, 2.12f, 2.83f}, 0.54f, 0.51f},
-    {false, 128, 64, 2, 3.5f, {0, 0.82f, 1.43f}, 2.0f, 0.73f},
-    {false, 128, 128, 2, 4.8f, {0, 1.28f, 2.22f}, 3.15f, 1.22f},
-    {true, 128, 128, 2, 2.4f, {0, 1.53f, 1.82f}, 0, 0},
-    {true, 256, 256, 1, 7.1f, {0, 2.45f}, 0, 0},
+    {false, 16, 64, 4, 3.127f, {0, 0.303f, 0.363f, 0.452f, 0.574f}, 0.753f, 0.112f, 0.244f, 0.1381f, 0.0689f},
+    {false, 32, 64, 4, 3.261f, {0, 0.354f, 0.418f, 0.577f, 0.764f}, 0.898f, 0.154f, 0.321f, 0.126f, 0.0444f},
+    {false, 64, 64, 4, 3.567f, {0, 0.443f, 0.527f, 0.843f, 1.013f}, 1.34f, 0.256f, 0.521f, 0.0904f, 0.0384f},
+    {false, 64, 128, 4, 4.225f, {0, 0.718f, 1.038f, 1.469f, 1.754f}, 1.788f, 0.539f, 1.078f, 0.0836f, 0.0528f},
+    {false, 128, 64, 2, 4.099f, {0, 0.645f, 0.854f}, 2.06f, 0.547f, 1.366f, 0.0661f, 0.0344f},
+    {false, 128, 128, 2, 5.345f, {0, 1.033f, 1.365f}, 3.251f, 0.971f, 2.677f, 0.0711f, 0.0484f},
+    {true, 128, 128, 2, 5.226f, {0, 1.208f, 1.071f}, 0, 0, 1.92f, 0.0f, 0.0436f},
+    {true, 256, 256, 1, 12.287f, {0, 1.788f}, 0, 0, 9.089f, 0.0164f, 0.0677f},
 };
 constexpr TileCost kHalfTiles[] = {
-    {true, 32, 64, 2, 6.1f, {0, 0.28f, 0.55f}, 0.22f, 0.36f},
-    {true, 64, 64, 2, 6.3f, {0, 0.37f, 0.76f}, 0.61f, 0.46f},
-    {true, 64, 128, 2, 5.9f, {0, 0.63f, 1.28f}, 2.43f, 0.61f},
-    {true, 128, 64, 2, 4.8f, {0, 0.66f, 1.29f}, 2.52f, 0.73f},
-    {true, 128, 128, 2, 0.7f, {0, 1.59f, 2.09f}, 8.33f, 1.21f},
-    {true, 256, 256, 1, 0.2f, {0, 2.85f}, 0, 0},
+    {true, 32, 64, 2, 3.518f, {0, 0.24f, 0.428f}, 0.886f, 0.145f, 0.516f, 0.1152f, 0.0414f},
+    {true, 64, 64, 2, 3.662f, {0, 0.288f, 0.459f}, 1.122f, 0.251f, 0.77f, 0.1064f, 0.0509f},
+    {true, 64, 128, 2, 3.795f, {0, 0.482f, 0.763f}, 1.778f, 0.56f, 0.988f, 0.1196f, 0.0739f},
+    {true, 128, 64, 2, 3.85f, {0, 0.486f, 0.706f}, 1.952f, 0.571f, 1.141f, 0.104f, 0.0406f},
+    {true, 128, 128, 2, 4.227f, {0, 1.206f, 1.044f}, 3.66f, 1.0f, 2.255f, 0.0987f, 0.0698f},
+    {true, 256, 256, 1, 11.089f, {0, 1.926f}, 0, 0, 9.416f, 0.1499f, 0.0699f},
 };
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// The same for gemv_kernel (fits 5 to 16 rows of the shapes above): its workgroups on a CU add
-// up, and every one reads the M rows of X.
-inline float gemv_cost(int64_t M, int64_t N, int64_t groups, bool int4, int cus) {
+inline float weight_mb(int64_t N, int64_t K, bool packed) { return (packed ? 0.5e-6f : 2e-6f) * N * K; }
+
+inline float tile_cost(const TileCost& t, int64_t M, int64_t N, int64_t K, int64_t splits, bool int4,
+                       int cus) {
+  const int64_t tiles_n = ceil_div(N, t.nt), tiles = ceil_div(M, t.mt) * tiles_n;
+  const int64_t on_cu = ceil_div(splits * ceil_div(tiles, 8), std::max(cus / 8, 1));
+  const int64_t per = ceil_div(K / kGroup, splits);
+  const float x_mb = 2e-6f * M * K;
+  float us = t.fixed + t.per_wg * (on_cu - 1) + t.per_mb * weight_mb(N, K, int4 && !t.dense) +
+             t.per_x_mb * tiles_n * x_mb +
+             per * ((on_cu / t.per_cu) * t.load[t.per_cu] + t.load[on_cu % t.per_cu]);
+  if (splits > 1) us += t.split + t.per_split * splits;
+  if (x_mb > 32) us = std::max(us, 0.13f * tiles_n * x_mb);  // X read past the L2s, at 7.7 TB/s
+  if (t.mt == 256) us *= 0.98f;                              // ties go to the largest tile
+  if (int4 && t.dense) us += 2.5f + 0.62e-6f * N * K;        // unpacking the weight first
+  return us;
+}
+
+// The same for gemv_kernel (1 to 16 rows): its workgroups on a CU add up, every one reads the M
+// rows of X, and each pass over its waves' chunks (24 groups packed, 12 fp16) costs a latency.
+inline float gemv_cost(int64_t M, int64_t N, int64_t K, bool int4, int cus) {
+  const int64_t groups = K / kGroup;
   const float load = (float)ceil_div(ceil_div(N, 16), cus);
-  return int4 ? 2.2f + groups * (0.1f + 0.064f * (load - 1) + 0.0055f * load * M)
-              : 1.65f + groups * (0.2f + 0.155f * (load - 1) + 0.0053f * load * M);
+  const float passes = (float)ceil_div(groups, int4 ? 24 : 12) - 1, mb = weight_mb(N, K, int4);
+  // 3% off: within the model's error the simpler kernel, with no workspace
+  return 0.97f * (int4 ? 3.8448f + 1.2024f * (load - 1) + groups * (0.0204f + 0.0026f * load * M) + 0.1016f * mb +
+                         passes * (1.3374f + 1.1724f * (load - 1)) + 0.0725f * load * M
+                       : 4.0113f + 1.2468f * (load - 1) + groups * (0.0168f + 0.0037f * load * M) + 0.0595f * mb +
+                         passes * (1.4026f + 1.3258f * (load - 1)) + 0.0341f * load * M);
 }
 
 // fp32 partial sums of a tiled plan, bytes
@@ -1299,18 +1327,17 @@ inline int64_t partial_bytes(int64_t M, int64_t N, const Plan& pl) {
   return pl.splits <= 1 ? 0 : pl.splits * ceil_div(M, pl.mt) * pl.mt * ceil_div(N, pl.nt) * pl.nt * 4;
 }
 
-// The cheapest plan whose partials take at most `room` bytes.  Up to kFusedNormM rows it is
-// gemv_kernel where the norm is fused or its workgroups fill the CUs; a narrow deep weight is
-// better split (3072 columns, K 8192: 4 rows packed 10.6 -> 9.6 us, 1
-// row fp16 16.3 -> 14.3; 16384 columns fp16 20.0 us, 20.9 tiled).
+// The cheapest plan whose partials take at most `room` bytes.  Up to kFusedNormM rows gemv_kernel
+// where it takes the norm in, and for fp16 weights so wide that it fills every CU four times (the
+// model misses whole rounds of it: 2 rows x 16384 columns, K 11008 72.5 us, 81.9 tiled).
 inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus,
                         int64_t room) {
   const int64_t groups = K / kGroup;
   // the partials of a call that large stay within the unpacked weight's bytes
   if (M >= kDenseMinM) room = std::min(room, N * K * 2);
   Plan best{true, false, 16, 16, 1};
-  if (M <= kFusedNormM && (norm || ceil_div(N, 16) > cus)) return best;
-  float best_us = M <= kGemvMaxM ? gemv_cost(M, N, groups, int4, cus) : 1e30f;
+  if (M <= kFusedNormM && (norm || (!int4 && ceil_div(N, 16) >= 4 * (int64_t)cus))) return best;
+  float best_us = M <= kGemvMaxM ? gemv_cost(M, N, K, int4, cus) : 1e30f;
   const TileCost* costs = int4 ? kPackedTiles : kHalfTiles;
   const int n = int4 ? (int)(sizeof(kPackedTiles) / sizeof(TileCost))
                      : (int)(sizeof(kHalfTiles) / sizeof(TileCost));
@@ -1318,6 +1345,9 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
     const TileCost& t = costs[c];
     if (int4 && t.dense && M < kDenseMinM) continue;
     const int64_t tiles = ceil_div(M, t.mt) * ceil_div(N, t.nt);
+    // only tiles that the rows fill at least half, and small ones while they are few (others
+    // were not timed)
+    if ((t.mt > 32 && t.mt >= 2 * M) || (t.mt < 128 && M > 8 * t.mt && tiles > 1024)) continue;
     if (tiles > 0x7ffffff) continue;
     const bool may_split = t.split > 0 && tiles <= kMaxSplitTiles;
     for (int64_t s = 1; s <= kMaxSplits && s <= groups; ++s) {
@@ -1326,10 +1356,7 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
       if (splits != s) continue;  // a smaller count with the same groups per split
       const Plan pl{false, t.dense, t.mt, t.nt, (int)splits};
       if (partial_bytes(M, N, pl) > room) break;
-      const int64_t on_cu = ceil_div(tiles * splits, cus);
-      float us = t.fixed + per * ((on_cu / t.per_cu) * t.load[t.per_cu] + t.load[on_cu % t.per_cu]);
-      if (splits > 1) us += t.split + t.per_split * splits;
-      if (int4 && t.dense) us += 2.5f + 0.62e-6f * N * K;  // unpacking the weight first
+      const float us = tile_cost(t, M, N, K, splits, int4, cus);
       if (us < best_us) {
         best_us = us;
         best = pl;
@@ -1339,7 +1366,7 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
   return best;
 }
 
-// choose_plan, remembered per thread for the last few sizes (it weighs some 50 plans).
+// choose_plan, remembered per thread for the last few sizes (it weighs some 60 plans).
 inline Plan plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, int cus) {
   struct Entry {
     int64_t M, N, K;
@@ -1701,6 +1728,23 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
 }
 
 }  // namespace
+
+extern "C" int fi_selftest_linear_plan(int64_t M, int64_t N, int64_t K, int packed, int norm,
+                                       int32_t* plan) {
+  using namespace fi;
+  clear_error();
+  if (M <= 0 || N <= 0 || K <= 0 || K % gemm::kGroup || M >= (1ll << 30) || N >= (1ll << 30) ||
+      K >= (1ll << 30) || !plan) {
+    set_error("fi_selftest_linear_plan: sizes must be positive and K a multiple of %d", gemm::kGroup);
+    return FI_ERR_INVALID;
+  }
+  const gemm::Plan pl = gemm::plan(M, N, K, packed != 0, norm != 0, device_cu_count(nullptr));
+  plan[0] = pl.gemv ? 0 : pl.dense ? 2 : 1;
+  plan[1] = pl.mt;
+  plan[2] = pl.nt;
+  plan[3] = pl.splits;
+  return FI_OK;
+}
 
 extern "C" size_t fi_int4_matmul_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % fi::gemm::kGroup) return 0;

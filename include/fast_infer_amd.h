@@ -365,6 +365,14 @@ FI_API int fi_int4_dequantize(const void* packed, int64_t p_stride, const void* 
                        int64_t w_stride, void* stream);
 
 /*
+ * The plan a linear call of these sizes takes on the current device (host only, no launch):
+ * plan[0] 0 = one pass over the columns, 1 = packed weights unpacked inside the GEMM, 2 = fp16
+ * weights, or packed ones unpacked first; plan[1], plan[2] rows and columns of its tiles; plan[3] K
+ * splits.  For the tests, which choose their sizes by it.
+ */
+FI_API int fi_selftest_linear_plan(int64_t M, int64_t N, int64_t K, int packed, int norm, int32_t* plan);
+
+/*
  * Self-test of the gfx950 MFMA fragment layout the attention kernels assume
  * (no counterpart in the reference; used by the test suite).  One wave computes
  * C[16x16] = A[16x32] * B[32x16] with v_mfma_f32_16x16x32_f16, where lane l holds

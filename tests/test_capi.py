@@ -291,3 +291,47 @@ def test_paged_partitions(lib):
                 for lens, count in ((True, with_lens), (False, shared)):
                     most[lens] = max(most[lens], count)
                     assert size >= most[lens] * batch * kv * group * 130 * 4, (kv, group, batch, n)
+
+
+def test_linear_plans(lib):
+    """What choose_plan makes of sizes over its whole range: only splits whose parts cover K, no
+    more partials than the size queries report, and the plans that measured fastest by far where
+    the tables could mislead: no large tiles for few rows of short K, one pass over the columns
+    for a row of a wide or deep packed weight."""
+    import random
+
+    from fast_infer_amd import _lib
+
+    plan = (ctypes.c_int32 * 4)()
+
+    def ask(M, N, K, packed, norm=0):
+        assert lib.fi_selftest_linear_plan(M, N, K, packed, norm, plan) == _lib.FI_OK
+        return tuple(plan)
+
+    r = random.Random(7)
+    for _ in range(4000):
+        M = r.choice([r.randint(1, 16), r.randint(1, 128), r.randint(1, 3000), r.randint(1, 100000)])
+        N, K = r.choice([r.randint(1, 400), r.randint(1, 30000)]), 128 * r.randint(1, 120)
+        for packed in (0, 1):
+            kind, mt, nt, splits = ask(M, N, K, packed)
+            groups = K // 128
+            assert kind in ((0, 2) if not packed else (0, 1, 2))
+            if kind == 0:
+                assert M <= 16 and splits == 1
+                continue
+            assert not packed or kind == 1 or M >= 129
+            assert 1 <= splits <= groups and -(-groups // -(-groups // splits)) == splits
+            if splits > 1:
+                partials = splits * -(-M // mt) * mt * -(-N // nt) * nt * 4
+                assert partials <= lib.fi_int4_matmul_workspace_size(M, N, K)
+                assert mt < 256 and (M < 129 or partials <= N * K * 2)
+            if M <= 4:
+                assert ask(M, N, K, packed, norm=1)[0] == 0
+    for M in (17, 32, 40, 64):
+        for N in (1536, 3072, 7168):
+            for K in (128, 256, 384, 512):
+                assert ask(M, N, K, 0)[1] <= 64 and ask(M, N, K, 0)[3] == 1, (M, N, K)
+    for N, K in ((4096, 11008), (5120, 3072), (3072, 3072), (16384, 3072)):
+        assert ask(1, N, K, 1)[0] == 0, (N, K)
+    assert lib.fi_selftest_linear_plan(0, 64, 128, 1, 0, plan) == _lib.FI_ERR_INVALID
+    assert lib.fi_selftest_linear_plan(1, 64, 100, 1, 0, plan) == _lib.FI_ERR_INVALID

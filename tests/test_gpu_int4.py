@@ -188,11 +188,9 @@ def test_int4_matmul_prefill_size_sampled(hip):
     _check(out16[rows.to(DEV)], x[rows.to(DEV)].cpu().numpy(), w16.cpu().numpy())
 
 
-# 129 rows and up: the weight dequantized once, then the 256 x 256-tile fp16 GEMM
-# (tile_gemm_kernel).  Shapes: partial row and column tiles, two K steps (K 128) and
-# 128 (K 8192), row tiles in multiples of 8 (the XCD-banded tile order, also with a partial
-# last row tile) and not, N not a multiple of 8 (element stores), output rows with a stride
-# and an output that is only 2-byte aligned (element stores), X rows with a stride; packed
+# 129 rows and up on tiles smaller than 256 x 256 (test_largest_tiles has those): partial row and
+# column tiles, one K group and 64, N not a multiple of 8 (element stores), output rows with a
+# stride and an output that is only 2-byte aligned (element stores), X rows with a stride; packed
 # and fp16 weights, every row against float64.
 @pytest.mark.parametrize("M,N,K,xpad,opad,ooff", [(129, 264, 128, 0, 0, 0),
                                                   (257, 130, 1024, 8, 6, 1),
@@ -231,6 +229,56 @@ def test_int4_matmul_dense_path_shapes(hip, M, N, K, xpad, opad, ooff):
         rows = buf[ooff:ooff + M * ld].view(M, ld)
         _check(rows[:, :N], x.cpu().numpy(), w16.cpu().numpy())
         # nothing written between rows or past the last one
+        assert torch.isnan(rows[:, N:]).all() and torch.isnan(buf[:ooff]).all()
+        assert torch.isnan(buf[ooff + M * ld:]).all()
+
+
+def _plan(M, N, K, form):
+    import ctypes
+
+    from fast_infer_amd import _lib
+
+    plan = (ctypes.c_int32 * 4)()
+    _lib.check(_lib.load().fi_selftest_linear_plan(M, N, K, form == "packed", 0, plan), "plan")
+    return tuple(plan)
+
+
+# The largest tiles, and packed weights unpacked for 128 x 128 ones, on sizes that the plan (asked
+# first) sends there: row tiles banded by XCD (a multiple of eight of them) and not, full and
+# with a partial last one; column counts that are no multiple of the tile and of 8 (element
+# stores), output rows with a stride, an output that is only 2-byte aligned, X rows with a
+# stride; every row against float64.
+@pytest.mark.parametrize("M,N,K,tile,xpad,opad,ooff", [(2048, 5120, 3072, 256, 0, 0, 0),
+                                                       (2000, 5120, 3072, 256, 8, 0, 0),
+                                                       (1700, 5120, 3072, 256, 0, 8, 0),
+                                                       (6000, 2052, 1024, 256, 0, 4, 0),
+                                                       (2040, 5128, 2048, 256, 16, 0, 1),
+                                                       (1400, 3072, 3072, 128, 0, 0, 0),
+                                                       (2100, 3072, 8192, 128, 24, 0, 0)])
+def test_largest_tiles(hip, M, N, K, tile, xpad, opad, ooff):
+    banner(f"int4_matmul {tile} x {tile} tiles M={M} N={N} K={K} x pad {xpad} out pad {opad} offset {ooff}")
+    from fast_infer_amd import _lib, dequantize_int4
+
+    lib = _lib.load()
+    packed, scales = _packed(M + N, N, K)
+    w16 = dequantize_int4(packed, scales)
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    xbig = torch.full((M + 300, K + xpad), float("nan"), device=DEV).half()
+    xbig[:M, :K] = torch.randn(M, K, device=DEV, generator=g).half()
+    ld = N + opad
+    ws = torch.empty(lib.fi_int4_matmul_workspace_size(M, N, K), dtype=torch.uint8, device=DEV)
+    st = _lib.stream_handle(torch.device(DEV))
+    forms = [f for f in ("packed", "fp16") if _plan(M, N, K, f) == (2, tile, tile, 1)]
+    assert "packed" in forms and (tile == 128 or "fp16" in forms)
+    for form in forms:
+        buf = torch.full((M * ld + 8,), float("nan"), dtype=torch.float16, device=DEV)
+        w = (packed.data_ptr(), K // 2, scales.data_ptr(), K // 128) if form == "packed" else \
+            (w16.data_ptr(), K, None, 0)
+        rc = lib.fi_int4_matmul(xbig.data_ptr(), K + xpad, M, K, *w, N, 128, buf.data_ptr() + 2 * ooff, ld,
+                                ws.data_ptr(), ws.numel(), st)
+        _lib.check(rc, "fi_int4_matmul")
+        rows = buf[ooff:ooff + M * ld].view(M, ld)
+        _check_device(rows[:, :N], xbig[:M, :K], w16)
         assert torch.isnan(rows[:, N:]).all() and torch.isnan(buf[:ooff]).all()
         assert torch.isnan(buf[ooff + M * ld:]).all()
 
