@@ -1252,6 +1252,7 @@ constexpr int kDenseMinM = 129;
 constexpr int kGemvMaxM = 16;    // rows of one gemv_kernel workgroup
 constexpr int kMaxSplits = 16;
 constexpr int kMaxSplitTiles = 8 * kXcdCounters;  // tiles of a split call
+constexpr int64_t kMaxTiles = (1 << 24) - 8;      // of any: 2^32 threads a launch dimension
 
 // Time of a call with one tile shape, in us, as measured on MI355X and fitted by least squares:
 // 8232 sizes of 1 to 30000 rows, 88 to 28672 columns and K 128 to 14336, cold weights, each with
@@ -1348,7 +1349,7 @@ inline Plan choose_plan(int64_t M, int64_t N, int64_t K, bool int4, bool norm, i
     // only tiles that the rows fill at least half, and small ones while they are few (others
     // were not timed)
     if ((t.mt > 32 && t.mt >= 2 * M) || (t.mt < 128 && M > 8 * t.mt && tiles > 1024)) continue;
-    if (tiles > 0x7ffffff) continue;
+    if (tiles > kMaxTiles) continue;
     const bool may_split = t.split > 0 && tiles <= kMaxSplitTiles;
     for (int64_t s = 1; s <= kMaxSplits && s <= groups; ++s) {
       if (s > 1 && (!may_split || tiles * s > 5 * (int64_t)cus)) break;
@@ -1677,7 +1678,7 @@ int run_linear(const char* fn, const void* x, int64_t x_stride, int64_t M, int64
     set_error("fi_int4_matmul: 256 rows of X or W span 2^31 bytes or more");
     return FI_ERR_UNSUPPORTED;
   }
-  if (!pl.gemv && ceil_div(M, pl.mt) * ceil_div(N, pl.nt) > 0x7ffffff) {
+  if (pl.gemv && M > kGemvMaxM) {  // no tiled plan: more than kMaxTiles tiles of any shape
     set_error("fi_int4_matmul: too many output tiles");
     return FI_ERR_UNSUPPORTED;
   }

@@ -187,6 +187,10 @@ def test_int4_validation(lib):
     assert need > 0
     assert lib.fi_int4_matmul(16, 3072, 40, 3072, 16, 1536, 16, 24, 5120, 128, 16, 5120, None,
                               0, None) == _lib.FI_ERR_WORKSPACE
+    # more output tiles than one launch takes
+    assert lib.fi_int4_matmul(16, 128, 1 << 29, 128, 16, 128, None, 0, 1 << 29, 128, 16, 1 << 29, None,
+                              0, None) == _lib.FI_ERR_UNSUPPORTED
+    assert b"tiles" in lib.fi_last_error()
     # quantize / dequantize take power-of-two group sizes from 8 to 512
     assert lib.fi_int4_quantize(16, 256, 4, 256, 96, 16, 128, 16, 2, None) == \
         _lib.FI_ERR_UNSUPPORTED
