@@ -948,9 +948,12 @@ __device__ __forceinline__ void lds_barrier() {
 // a fixed order.
 //
 // kNormRows > 0: the RMSNorm of up to that many rows fused, shared out over the workgroup (packed
-// weights, 1 or 2 rows) or a row per wave.  5120 columns, K 3072, packed, cold weights: 1 row
-// 8.0 us, 8.8 a row per wave; 16384 columns 12.2 against 15.2 and, 2 rows, 13.6 against 15.1.  4
-// rows shared out take 10.9 against 9.1, and fp16 weights, bound by their stream, lose too.
+// weights, 1 row, or 2 of more than kShortRow elements) or a row per wave.  5120 columns, K 3072,
+// packed, cold weights: 1 row 8.0 us, 8.8 a row per wave; 16384 columns 12.2 against 15.2 and, 2
+// rows, 13.6 against 15.1.  4 rows shared out take 10.9 against 9.1, 2 short rows leave most
+// threads idle (7168 columns, K 256 6.2 against 5.6), and fp16 weights, bound by their stream,
+// lose too.
+constexpr int kShortRow = 1024;
 template <bool kInt4, int kChunk, int kNormRows, int kW>
 __global__ __launch_bounds__(64 * kW, kNormRows == kFusedNormM ? 1 : 2) void gemv_kernel(Params p) {
   constexpr bool kNorm = kNormRows > 0;
@@ -1543,7 +1546,7 @@ void launch_gemv(const fi::gemm::Params& p, bool int4, bool norm, hipStream_t st
     hipLaunchKernelGGL((gemv_kernel<false, 3, 4, 4>), grid, four, lds, st, p);
   else if (p.M == 1)
     hipLaunchKernelGGL((gemv_kernel<true, 3, 1, 8>), grid, eight, lds, st, p);
-  else if (p.M == 2)
+  else if (p.M == 2 && p.K > kShortRow)
     hipLaunchKernelGGL((gemv_kernel<true, 3, 2, 8>), grid, eight, lds, st, p);
   else
     hipLaunchKernelGGL((gemv_kernel<true, 6, 4, 4>), grid, four, lds, st, p);

@@ -93,7 +93,8 @@ def test_rms_norm_int4_matmul_vs_oracle(hip, M, packed_weights):
 # several per thread, a length that leaves threads idle, the longest shared-out row, one past it,
 # strided rows, and a last column tile with one column.
 @pytest.mark.parametrize("M", [1, 2])
-@pytest.mark.parametrize("K,pad", [(128, 0), (3072, 8), (4096, 0), (4224, 64), (8192, 0), (8320, 0)])
+@pytest.mark.parametrize("K,pad", [(128, 0), (1024, 0), (1152, 8), (3072, 8), (4096, 0), (4224, 64),
+                                   (8192, 0), (8320, 0)])
 def test_rms_norm_int4_matmul_few_rows(hip, M, K, pad):
     banner(f"rms_norm_int4_matmul M={M} K={K} row pad {pad}")
     from fast_infer_amd import dequantize_int4, quantize_int4_groupwise, rms_norm_int4_matmul
