@@ -493,18 +493,23 @@ __global__ __launch_bounds__(kHeadDim) void merge_kernel(Params p) {
 // streams): the smallest partitions whose workgroups fit one round, else the cap (against the
 // sizes above: 4 rows of 4096 22.8 -> 17.6 us, 12 of 1024 19.0 -> 16.4, 8 of 8192 52.6 -> 48.8;
 // past one round 32 of 2048 52.8 -> 50.7, but 48 of 700 with 16 heads 51.8 -> 54.5 at 512
-// tokens, a full and a small partition a row, so below 1024 tokens the cap is 384).  Partitions
-// of 64 tokens pay while half the slots stay free and a merge adds up no more than 16 (1 row of
-// 500 11.5 -> 8.7 us, of 1024 9.7 -> 9.1, but of 2048 10.2 -> 10.9; 48 units of 400 11.4 -> 12.0).
-constexpr int64_t kDirectTokens = 512;   // up to this: one partition with no merge, or 64 tokens
-constexpr int64_t kUnsplitTokens = 320;  // at most this: always one partition
+// tokens, a full and a small partition a row, so below 1024 tokens the cap is 384).
+//
+// Partitions of 64 tokens pay, with either, while half the slots stay free and a merge adds up no
+// more than 16 (1 row of 1024 9.7 -> 9.1 us, of 2048 10.2 -> 10.9; 513 to 1024 tokens 6% over seven
+// kinds of per-row lengths).  Calls of up to 512 tokens, one partition and no merge, gain where
+// the length is shared (1 row of 500 11.5 -> 8.7; 48 units of 400 11.4 -> 12.0) and lose where rows
+// may be short (above).
+constexpr int64_t kDirectTokens = 512;   // up to this, with lengths: one partition, no merge
+constexpr int64_t kUnsplitTokens = 320;  // the same without
 constexpr int64_t kMaxTokens64 = 1024;   // most tokens cut into partitions of 64
 constexpr int64_t kRoundWgs = 512;       // workgroups of one round
 constexpr int64_t kSmallWgs = 2048;
 static int tokens_per_split(int64_t units, int64_t num_tokens, bool lens) {
   auto wgs = [&](int64_t tps) { return units * ((num_tokens + tps - 1) / tps); };
   int64_t tps, least = 128;
-  if (!lens && num_tokens > kUnsplitTokens && num_tokens <= kMaxTokens64 && wgs(64) <= kRoundWgs / 2) {
+  if (num_tokens > (lens ? kDirectTokens : kUnsplitTokens) && num_tokens <= kMaxTokens64 &&
+      wgs(64) <= kRoundWgs / 2) {
     tps = least = 64;
   } else if (num_tokens <= kDirectTokens) {
     tps = num_tokens;
