@@ -2,16 +2,16 @@
 
 Two layers of a decode step are captured once with ``torch.cuda.graph`` and replayed
 several times, with other GPU work and host synchronisation between the replays:
-  - RMSNorm fused with the INT4 QKV projection (one-pass kernel at 8 rows; a norm pass,
-    then split-K GEMM plus reduction at 64 rows);
+  - RMSNorm and the INT4 QKV projection (a norm pass, then a GEMM whose K splits are added
+    inside its launch, six of them at 8 rows and three at 64);
   - the fused RoPE + pool write at per-row positions;
   - paged attention over per-row lengths;
   - the INT4 O projection.
 
 Each replay must equal the eager step bit for bit: the same kernels on the same inputs,
 rewriting the same pool slots. None of these entry points records a memset or allocates
-inside the library. The caller's caches (INT4 workspace, decode workspace) are set up by
-an eager call before capture.
+inside the library. The decode workspace is the caller's; the INT4 workspaces are part of the
+graph (one per captured call).
 
 A captured ``PagedKVCache.append`` advances the device allocator once per replay, exactly
 as the same number of eager appends on a twin cache does.
@@ -78,7 +78,7 @@ def test_decode_step_graph_replay(hip, B):
 
     st = _setup(B, 50 + B)
     ws = paged_attention_workspace(B, HQ, HKV, 1024, D, DEV)
-    # eager reference (also sets up the INT4 workspace cache); the step rewrites the same
+    # eager reference; the step rewrites the same
     # pool slots each time, so running it again leaves the pools unchanged
     ref = _step(st, st["x"], ws).clone()
     ref_pools = [(k.clone(), v.clone()) for k, v in st["pools"]]
@@ -233,30 +233,34 @@ def test_many_captures_keep_the_in_launch_sum(hip):
 
 
 def test_int4_workspace_two_captures_shared_pool(hip):
-    """Two graphs captured back to back on a shared memory pool, the second needing a larger
-    split-K workspace than the first: the first graph's workspace must stay allocated, so
-    replaying both (in either order, repeatedly) equals the eager results bit for bit."""
-    banner("int4 split-K workspace across two captures (17 then 64 rows)")
-    from fast_infer_amd import int4_matmul, quantize_int4_groupwise
+    """Graphs captured back to back on a shared memory pool, the last needing a larger split-K
+    workspace than the first: the first graph's workspace must stay allocated, so replaying
+    all (in either order, repeatedly) equals the eager results bit for bit."""
+    banner("int4 split-K workspace across captures (8, 17, then 64 rows)")
+    from fast_infer_amd import _lib, int4_matmul, quantize_int4_groupwise
+
+    rows = (8, 17, 64)
+    sizes = [_lib.load().fi_int4_matmul_workspace_size(m, 5120, 3072) for m in rows]
+    assert 0 < sizes[0] < sizes[-1]
 
     g = torch.Generator(device=DEV).manual_seed(77)
     w = quantize_int4_groupwise((torch.randn(5120, 3072, device=DEV, generator=g) * 0.02).half())
-    xs = {m: torch.randn(m, 3072, device=DEV, generator=g).half() for m in (17, 64)}
+    xs = {m: torch.randn(m, 3072, device=DEV, generator=g).half() for m in rows}
     refs = {m: int4_matmul(x, w).clone() for m, x in xs.items()}
     torch.cuda.synchronize()
     pool = torch.cuda.graph_pool_handle()
     graphs, outs = {}, {}
-    for m in (17, 64):
+    for m in rows:
         graphs[m] = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graphs[m], pool=pool):
             outs[m] = int4_matmul(xs[m], w)
         torch.cuda.synchronize()
     for rep in range(3):
-        for m in ((17, 64) if rep % 2 == 0 else (64, 17)):
+        for m in (rows if rep % 2 == 0 else rows[::-1]):
             outs[m].zero_()
             graphs[m].replay()
         torch.cuda.synchronize()
-        for m in (17, 64):
+        for m in rows:
             assert torch.equal(outs[m], refs[m]), (rep, m)
 
 
