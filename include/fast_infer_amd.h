@@ -39,8 +39,8 @@
  *   - Calls are reentrant.  The library's host-side state is the per-thread error
  *     message and, per device, cached on first use: the CU count (an atomic), and,
  *     under a mutex, the result of the workgroup-placement probe and the split-K counters
- *     handed out (fi_int4_matmul: a set for each of the first 16 streams, counters of its own
- *     for each captured call while they last; other calls use a second launch), and per
+ *     handed out (fi_int4_matmul: a set for each of the first 16 streams, and one for each stream
+ *     of each graph capture while they last; other calls use a second launch), and per
  *     thread the tile plans of the last few linear-layer sizes.  No other library is called.
  *   - Return value: FI_OK or an FI_ERR_* code; fi_last_error() then gives a
  *     message for the calling thread.
@@ -307,9 +307,10 @@ FI_API int fi_kv_reset(int32_t* block_table, int64_t bt_stride, int64_t max_bloc
  *   reference's) and K a multiple of 128; for another group size, dequantize with
  *   fi_int4_dequantize and pass the fp16 weight.  Some shapes split K or unpack the weight
  *   into memory first: then a workspace of fi_int4_matmul_workspace_size(M, N, K) bytes (enough
- *   for either weight form) is required (FI_ERR_WORKSPACE otherwise; calls of up to 16 rows,
- *   and fp16 weights from 129 rows, run without one, slower); calls that overlap in time must
- *   not share one.  From 129 rows 256 rows of X (and of an fp16 W) have to span less than
+ *   for either weight form) is required (FI_ERR_WORKSPACE otherwise).  With less some calls run
+ *   all the same, slower: up to 16 rows, and fp16 weights from 129 rows, without one; 17 to 128
+ *   rows with the partials of a K split into about two workgroups per CU, which for most sizes
+ *   is none.  Calls that overlap in time must not share a workspace.  From 129 rows 256 rows of X (and of an fp16 W) have to span less than
  *   2 GiB (FI_ERR_UNSUPPORTED otherwise).
  */
 FI_API size_t fi_int4_matmul_workspace_size(int64_t M, int64_t N, int64_t K);
