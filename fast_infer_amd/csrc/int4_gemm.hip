@@ -219,12 +219,13 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const half_t* x, int64_t x
 // 5.0 -> 3.4 us for 64 rows, 5.8 -> 5.1 for 1000, 37.5 -> 35.6 (5.7 TB/s) for 16384; of 8192 7.6 ->
 // 3.8 for 64.  Rows of up to 2048 elements leave threads idle, which many of them notice: 768
 // elements 4.5 -> 4.2 us for 1000 rows, but 17.3 against 21.2 for 16384, so they stay with
-// rmsnorm_kernel from kWaveRows rows; those a little longer, whose second part leaves three of
-// four waves idle, from 8192 (2056 elements; 16384 rows 30.9 against 36.5) to 24320 rows (2560
-// elements; 32768 rows 65.4 against 68.7); and all from kManyRows, whose 256 threads a row are
-// more than a launch takes (2^32 along x).
+// rmsnorm_kernel from kWaveRows rows; those of less than 2816, whose second part leaves three of
+// four waves idle, from kMoreRows (2056 elements, 12288 rows 19.9 against 18.4, 16384 28.4 against
+// 32.6; 2560 elements, 16384 rows 32.0 against 33.0); and all from kManyRows, whose 256 threads a
+// row are more than a launch takes (2^32 along x).
 constexpr int kRowParts = 4;
 constexpr int kWaveRows = 1024;
+constexpr int kMoreRows = 13000;
 constexpr int64_t kManyRows = 1 << 24;
 __global__ __launch_bounds__(256) void rmsnorm_row_kernel(const half_t* x, int64_t x_stride, int K,
                                                           const half_t* w, float eps, half_t* out,
@@ -1521,7 +1522,7 @@ void launch_plan(fi::gemm::Params p, const fi::gemm::Plan& pl, void* workspace, 
 void launch_rmsnorm(const half_t* x, int64_t x_stride, int64_t M, int64_t K, const half_t* w,
                     float eps, half_t* out, int64_t out_stride, hipStream_t st) {
   using namespace fi::gemm;
-  const int64_t wave_rows = K <= 2048 ? kWaveRows : K < 2816 ? 7936 + 32 * (K - 2048) : kManyRows;
+  const int64_t wave_rows = K <= 2048 ? kWaveRows : K < 2816 ? kMoreRows : kManyRows;
   if (K <= kRowParts * 2048 && M < wave_rows)
     hipLaunchKernelGGL(rmsnorm_row_kernel, dim3((unsigned)M), dim3(256), 0, st, x, x_stride, (int)K, w,
                        eps, out, out_stride);

@@ -75,9 +75,10 @@ __global__ __launch_bounds__(64) void xcd_probe_kernel(unsigned* out) {
 // one another, so they share the stream's set (one per stream, in order of first use, up to
 // kXcdStreams streams).  A graph may be replayed beside any stream and any other graph: each
 // capture gets sets of its own, one for every stream taking part (what is captured on one
-// stream forms a chain in the graph), from a part of the array that is only ever handed out
-// once: 16 MiB, 2 to 8 KiB a set; captures past it use the second launch.  A set for each
-// launch lasted 146 captures of a 28-layer step with two such calls a layer; this lasts 8192.
+// stream forms a chain in the graph; a program that rewires a capture's dependencies by hand has
+// to keep that order), from a part of the array that is only ever handed out once: 16 MiB, 2 to 8
+// KiB a set; captures past it use the second launch.  A set for each launch lasted 146 captures
+// of a 28-layer step with two such calls a layer; this lasts 8192.
 constexpr int kXcdStreams = 16;
 constexpr int kXcdSet = 8 * kXcdCounters;
 constexpr int kXcdCaptured = 4 << 20;

@@ -40,7 +40,8 @@
  *     message and, per device, cached on first use: the CU count (an atomic), and,
  *     under a mutex, the result of the workgroup-placement probe and the split-K counters
  *     handed out (fi_int4_matmul: a set for each of the first 16 streams, and one for each stream
- *     of each graph capture while they last; other calls use a second launch), and per
+ *     of each graph capture while they last, whose calls have to stay in the order in which they
+ *     were captured; other calls use a second launch), and per
  *     thread the tile plans of the last few linear-layer sizes.  No other library is called.
  *   - Return value: FI_OK or an FI_ERR_* code; fi_last_error() then gives a
  *     message for the calling thread.

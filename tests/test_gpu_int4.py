@@ -491,6 +491,23 @@ def test_tiled_kernels(hip, M, N, K):
         _check_device(outs[0], x, w16)
 
 
+@pytest.mark.parametrize("M,N,K,form", [(17, 128, 14336, "packed"), (64, 200, 12032, "packed"),
+                                        (5, 130, 14336, "fp16"), (33, 256, 14336, "fp16")])
+def test_many_splits(hip, M, N, K, form):
+    """Deep narrow weights: more than ten K splits, added by the last workgroup of a tile four at
+    a time; the last split may be shorter."""
+    banner(f"linear call of many K splits M={M} N={N} K={K} {form}")
+    from fast_infer_amd import dequantize_int4, int4_matmul
+
+    assert _plan(M, N, K, form)[3] > 10
+    w = _packed(M + N, N, K)
+    w16 = dequantize_int4(*w)
+    x = torch.randn(M, K, device=DEV).half()
+    outs = [int4_matmul(x, w if form == "packed" else w16) for _ in range(3)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    _check_device(outs[0], x, w16)
+
+
 def test_tiled_kernels_two_launch_path(hip):
     """A stream without counters (hipStreamPerThread is never given any) adds the K splits in a
     second launch: the same bits as the in-launch sum, both weight forms."""

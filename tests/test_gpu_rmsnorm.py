@@ -129,7 +129,7 @@ def test_rms_norm_kernel_choice(hip, M, H, pad):
     assert np.all(np.abs(got - exact) <= ON.norm_bound(exact))
 
 
-@pytest.mark.parametrize("M,H", [(8191, 2056), (8192, 2056), (12031, 2176), (12032, 2176)])
+@pytest.mark.parametrize("M,H", [(12999, 2056), (13000, 2056), (13000, 2808), (13000, 2816)])
 def test_rms_norm_many_rows_kernel_choice(hip, M, H):
     banner(f"rms_norm M={M} H={H}")
     from fast_infer_amd import rms_norm
