@@ -763,14 +763,12 @@ extern "C" int fi_paged_attention_fwd_noalloc(const void* q, int64_t q_sb, int64
   using namespace fi;
   static const char* fn = "fi_paged_attention_fwd_noalloc";
   clear_error();
-  // up to kDirectTokens tokens: one partition, which leaves the shared scratch alone (sizes
-  // that are no call's are left to paged_fwd)
-  size_t need = 0;
-  if (batch > 0 && num_tokens > decode::kDirectTokens && num_q_heads > 0 && num_kv_heads > 0 &&
-      num_q_heads % num_kv_heads == 0 && head_dim_ok(head_dim))
-    need = decode::partial_bytes(
-        batch, num_q_heads,
-        decode::cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr).splits);
+  // up to kDirectTokens tokens: one partition, which leaves the shared scratch alone.  The size
+  // query decides beyond, not the fewer bytes that a call of one shared length may take
+  const size_t need = num_tokens > decode::kDirectTokens
+                          ? fi_paged_attention_workspace_size(batch, num_q_heads, num_kv_heads,
+                                                              num_tokens, head_dim)
+                          : 0;
   if (need > kScratchBytes) {
     set_error("%s: these sizes need %zu bytes of split-K scratch, more than the %zu bytes "
               "this entry point holds per device; use fi_paged_attention_fwd with a workspace",

@@ -299,6 +299,21 @@ def test_paged_partitions(lib):
                     assert size >= most[lens] * batch * kv * group * 130 * 4, (kv, group, batch, n)
 
 
+@pytest.mark.parametrize("sizes", [(6, 32, 4, 168207), (52, 64, 8, 8439), (1479, 1, 1, 19455), (5, 21, 3, 298296)])
+@pytest.mark.parametrize("lens", [True, False])
+def test_noalloc_refuses_by_the_size_query(lib, sizes, lens):
+    """The allocation-free decode call refuses every size whose query exceeds its scratch, also
+    where one shared length would take fewer bytes."""
+    from fast_infer_amd import _lib
+
+    batch, hq, hkv, n = sizes
+    assert lib.fi_paged_attention_workspace_size(batch, hq, hkv, n, 128) > 32 << 20
+    blocks = -(-n // 64)
+    rc = lib.fi_paged_attention_fwd_noalloc(16, hq * 128, 128, 16, 16, batch * blocks, 64, hkv, 16, blocks, blocks,
+                                            16 if lens else None, n, 16, hq * 128, 128, batch, hq, 128, 1.0, None)
+    assert rc == _lib.FI_ERR_UNSUPPORTED and b"scratch" in lib.fi_last_error()
+
+
 def test_linear_plans(lib):
     """What choose_plan makes of sizes over its whole range: only splits whose parts cover K, no
     more partials than the size queries report, and the plans that measured fastest by far where
