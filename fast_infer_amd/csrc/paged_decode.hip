@@ -505,11 +505,11 @@ constexpr int64_t kUnsplitTokens = 320;  // the same without
 constexpr int64_t kMaxTokens64 = 1024;   // most tokens cut into partitions of 64
 constexpr int64_t kRoundWgs = 512;       // workgroups of one round
 constexpr int64_t kSmallWgs = 2048;
-static int tokens_per_split(int64_t units, int64_t num_tokens, bool lens) {
+static int tokens_per_split(int64_t units, int64_t num_tokens, bool lens, bool may64) {
   auto wgs = [&](int64_t tps) { return units * ((num_tokens + tps - 1) / tps); };
   int64_t tps, least = 128;
-  if (num_tokens > (lens ? kDirectTokens : kUnsplitTokens) && num_tokens <= kMaxTokens64 &&
-      wgs(64) <= kRoundWgs / 2) {
+  if (may64 && num_tokens > (lens ? kDirectTokens : kUnsplitTokens) &&
+      num_tokens <= kMaxTokens64 && wgs(64) <= kRoundWgs / 2) {
     tps = least = 64;
   } else if (num_tokens <= kDirectTokens) {
     tps = num_tokens;
@@ -538,15 +538,17 @@ static int heads_per_wg(int64_t group) {
   return 1;
 }
 
-// Partition size and partitions per row of a call of at least one row.
+// Partition size and partitions per row of a call of at least one row, with partitions of 64
+// tokens or without (up to kDirectTokens tokens that is one partition).
 struct Cut {
   int tps;
   int64_t splits;
 };
-static Cut cut(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t num_tokens, bool lens) {
+static Cut cut(int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t num_tokens, bool lens,
+               bool may64) {
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t units = batch * num_kv_heads * (group / heads_per_wg(group));
-  const int tps = tokens_per_split(units, std::max<int64_t>(num_tokens, 1), lens);
+  const int tps = tokens_per_split(units, std::max<int64_t>(num_tokens, 1), lens, may64);
   return {tps, std::max<int64_t>((num_tokens + tps - 1) / tps, 1)};
 }
 
@@ -646,11 +648,11 @@ int paged_fwd(const char* fn, const void* q, int64_t q_sb, int64_t q_sh, const v
   p.heads_per_wg = heads_per_wg(group);
   p.scale_log2 = sm_scale * kLog2e;
   const int64_t wg_per_row = num_kv_heads * (group / p.heads_per_wg);
-  Cut c = cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr);
+  Cut c = cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr, true);
+  // what partitions of 64 tokens take that the larger ones did not is never needed
+  if (!workspace || workspace_bytes < partial_bytes(batch, num_q_heads, c.splits))
+    c = cut(batch, num_q_heads, num_kv_heads, num_tokens, context_lens != nullptr, false);
   const size_t need = partial_bytes(batch, num_q_heads, c.splits);
-  // calls of up to kDirectTokens tokens run without a workspace too, as one partition
-  if (num_tokens <= kDirectTokens && (!workspace || workspace_bytes < need))
-    c = {(int)kDirectTokens, 1};
   const int64_t splits = c.splits;
   p.tokens_per_split = c.tps;
   p.max_splits = (int)splits;

@@ -114,7 +114,8 @@ FI_API int fi_flash_attention_fwd(const void* q, const void* k, const void* v, v
  * Bytes of device workspace fi_paged_attention_fwd needs for these sizes
  * (0 when the call is served by a single pass).  `max_num_tokens` is the bound
  * later passed as `num_tokens`; the size also serves every smaller one.  Calls of up to
- * 512 tokens run without the workspace too, in a single pass that is slower for few rows.
+ * 512 tokens run without the workspace too, in a single pass, and calls of up to 1024 on what
+ * partitions of 128 tokens take; both are slower for few rows.
  */
 FI_API size_t fi_paged_attention_workspace_size(int64_t batch, int64_t num_q_heads,
                                          int64_t num_kv_heads, int64_t max_num_tokens,

@@ -264,11 +264,11 @@ def test_paged_workspace_size_covers_smaller_calls(lib):
 
 
 def test_paged_partitions(lib):
-    """Partitions a call is cut into, as the workspace it asks for tells: with per-row lengths
-    (all rows may be far below the bound, or one far above the rest) 128 to 384 tokens in about
-    2048 workgroups at the bound, never one round of workgroups; with one shared length at most
-    that many, one round where that is enough; with either 64 tokens for few rows of up to 1024.
-    The size query covers every one of them."""
+    """Partitions a call is cut into, as the workspace it asks for at least tells: with per-row
+    lengths (all rows may be far below the bound, or one far above the rest) 128 to 384 tokens in
+    about 2048 workgroups at the bound, never one round of workgroups; with one shared length at
+    most that many, one round where that is enough.  The size query covers every one of them, and
+    the 64-token partitions that few rows of up to 1024 tokens run in where there is room."""
     import re
 
     from fast_infer_amd import _lib
@@ -290,11 +290,11 @@ def test_paged_partitions(lib):
                 tps = max(128, -(-max(min(384, -(-n // want)), -(-n // 1024)) // 64) * 64)
                 with_lens, shared = splits(batch, kv * group, kv, n, True), splits(batch, kv * group, kv, n, False)
                 few = n <= 1024 and units * -(-n // 64) <= 256
-                assert with_lens == -(-n // (64 if few else tps)), (kv, group, batch, n)
+                assert with_lens == -(-n // tps), (kv, group, batch, n)
                 assert shared <= with_lens
                 assert units * shared <= 512 or shared <= -(-n // 384)
                 size = lib.fi_paged_attention_workspace_size(batch, kv * group, kv, n, 128)
-                for lens, count in ((True, with_lens), (False, shared)):
+                for lens, count in ((True, with_lens), (False, shared), (True, few * -(-n // 64))):
                     most[lens] = max(most[lens], count)
                     assert size >= most[lens] * batch * kv * group * 130 * 4, (kv, group, batch, n)
 

@@ -542,6 +542,49 @@ def test_paged_decode_short_calls_without_workspace(hip):
     assert float((outs[0] - outs[1]).abs().max()) <= ATOL and torch.equal(outs[1], outs[2])
 
 
+@pytest.mark.parametrize("batch,tokens", [(1, 513), (1, 1024), (2, 1000), (3, 640)])
+@pytest.mark.parametrize("with_lens", [False, True])
+def test_paged_decode_on_the_workspace_of_larger_partitions(hip, batch, tokens, with_lens):
+    """513 to 1024 tokens, few rows: partitions of 64 tokens with the size queried; with less, down
+    to what partitions of 128 take, those; refused below."""
+    banner(f"paged decode batch {batch} tokens {tokens} lens {with_lens} on less workspace")
+    from fast_infer_amd import _lib
+
+    lib = _lib.load()
+    hq, hkv, d, bs = 24, 8, 128, 64
+    mb = -(-tokens // bs)
+    kc, vc = (torch.randn(batch * mb, bs, hkv, d, device="cuda:0").half() for _ in range(2))
+    q = torch.randn(batch, hq, d, device="cuda:0").half()
+    table = torch.randperm(batch * mb, device="cuda:0").int().view(batch, mb)
+    cl = torch.full((batch,), tokens, dtype=torch.int32, device="cuda:0") if with_lens else None
+    per_split = batch * hq * 130 * 4
+    least = -(-tokens // 128) * per_split
+    need = lib.fi_paged_attention_workspace_size(batch, hq, hkv, tokens, d)
+    assert need >= -(-tokens // 64) * per_split > least
+    ws = torch.empty(need + 256, dtype=torch.uint8, device="cuda:0")
+    outs = []
+    for nbytes in (need, -(-tokens // 64) * per_split - 4, least, least - 4):
+        ws.fill_(255)
+        out = torch.empty_like(q)
+        rc = lib.fi_paged_attention_fwd(
+            q.data_ptr(), hq * d, d, kc.data_ptr(), vc.data_ptr(), batch * mb, bs, hkv, table.data_ptr(), mb, mb,
+            None if cl is None else cl.data_ptr(), tokens, out.data_ptr(), hq * d, d, batch, hq, d, d ** -0.5,
+            ws.data_ptr(), nbytes, _lib.stream_handle(q.device))
+        if nbytes < least:
+            assert rc == _lib.FI_ERR_WORKSPACE
+            continue
+        _lib.check(rc, "fi_paged_attention_fwd")
+        assert bool((ws[nbytes:] == 255).all())
+        assert bool((ws[least:] == 255).all()) == (nbytes < -(-tokens // 64) * per_split)
+        outs.append(out.float())
+    for b in range(batch):
+        k, v = (c[table[b].long()].flatten(0, 1)[:tokens].float() for c in (kc, vc))
+        s = torch.einsum("kgd,nkd->kgn", q[b].float().view(hkv, 3, d), k) * d ** -0.5
+        ref = torch.einsum("kgn,nkd->kgd", s.softmax(-1), v).reshape(hq, d)
+        assert all(float((o[b] - ref).abs().max()) <= ATOL for o in outs)
+    assert torch.equal(outs[1], outs[2])
+
+
 # Prefill grids around the switches of the launch: one head per workgroup below one and a half
 # workgroups per CU (one, up to four query tiles), the lightest-first second half up to two per
 # CU (its first row inside, at the end of and past the grid), and grids past both.
